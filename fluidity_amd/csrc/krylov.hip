@@ -70,13 +70,15 @@ struct KrylovWork {
     std::vector<int32_t> mc_ptr;  // colour c owns mc_rows[mc_ptr[c] .. mc_ptr[c+1])
     int64_t mc_key = -1;          // sparsity generation of the colouring
     // GMRES
-    DevBuf<double> V, H, gv, cs, sn, hcol;
+    DevBuf<double> V, gm_work;  // basis; block sums, Hessenberg column, rotations
     DevBuf<float> V32;
-    int gm = 0;
+    DevBuf<unsigned char> gm_state;
+    void* gm_host = nullptr;    // the solve's progress, in pinned memory that the device writes
     bool have_x = false;
     bool prepared = false, prepared_mixed = false;
     ~KrylovWork() {
         if (h_scal && h_scal_owned) (void)hipHostFree(h_scal);
+        if (gm_host) (void)hipHostFree(gm_host);
     }
 };
 
@@ -1450,118 +1452,583 @@ static int run_cg1(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_info
 }
 
 // ------------------------- GMRES ------------------------------------------
+//
+// Restarted GMRES with left preconditioning and classical Gram-Schmidt done
+// twice, driven from the device: the Hessenberg column, its Givens rotations
+// and the convergence test are taken by one wave beside the next iteration's
+// dot products, so an iteration is four kernels and no host round trip:
+//   k_gm_sell / k_gm_csr  normalises the last w into basis vector v_k and
+//                         forms w = D^-1 A v_k (SSOR: A v_k, then the sweeps)
+//   k_gm_dots             h1_j = w . v_j; one more workgroup closes the
+//                         column before this one
+//   k_gm_orth<.., DOTS>   w -= sum h1_j v_j and, from the same registers,
+//                         h2_j = w . v_j (the second pass's coefficients)
+//   k_gm_orth<.., NORM>   w -= sum h2_j v_j and |w|^2
+// The basis is read three times an iteration instead of five, and the sums
+// over blocks are taken by every consumer block in the same fixed order.
+// The iteration counter and the done flag reach the host through a word in
+// pinned memory, which it polls a few iterations behind what it has queued.
+// What bounds it: small systems, the chain of four launches (each two or
+// three dependent memory round trips, 4-6 us); large ones, reading the basis
+// (6 TB/s with 32 vectors of 373k rows: 15-17 us a pass).  Whole time steps
+// on one MI355X, against ten launches and three waits for the host an
+// iteration: 64 x 64 P1 triangles, 18 iterations, 2.04 -> 0.65 ms; 71^3 x 6
+// P1 tetrahedra, 30 iterations, 5.80 -> 2.87 ms; 40^3 x 6 P2, 14.4 -> 9.7 ms.
 
-template <typename T>
-__device__ __forceinline__ T lane_sum(T v, int L) {
-    for (int off = L >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+constexpr int kGmGrid = 256;    // blocks of the basis kernels: one per CU, so that a consumer block can sum the
+                                // partial sums of every basis vector itself (256 x 31 doubles)
+constexpr int kGmReg = 32;      // basis vectors held in registers; longer bases are read more often
+constexpr int kGmAhead = 3;     // iterations queued beyond the last one known to be finished
+
+// Threads of the basis kernels for NB vectors in registers: as many as the
+// registers allow, since a block per CU has to cover the memory latency.
+constexpr int gm_block(int NB) { return NB <= 16 ? 1024 : 512; }
+
+// Device state of a solve.
+struct GmState {
+    double rnorm0, last;
+    double rtol, atol;
+    int32_t its, max_its, kk, reason, done, first;
+};
+
+// What the host sees of it, in pinned memory: word = 2 its + done while the
+// solve runs (one store, nothing ordered after it), the state after it.
+struct GmHost {
+    int64_t word;
+    GmState st;
+};
+
+// Where the kernels find the solve's small arrays (m: restart length).
+struct GmDev {
+    GmState* st;
+    GmHost* host;
+    double *p1, *p2, *pn;   // block sums: h1 and h2 per basis vector, |w|^2
+    double *h1, *h2;        // the column's coefficients
+    double *R, *g, *cs, *sn, *y;
+    int m, nb;              // nb: blocks of the basis kernels
+};
+
+__device__ __forceinline__ int gm_done(const GmDev& d) {
+    return __hip_atomic_load(&d.st->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// w = D^-1 (A v)  [left Jacobi]
+// Lane `lane`'s value (the same lane in the whole wave), without the
+// latency of a shuffle through LDS.
+__device__ __forceinline__ double gm_lane(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+__device__ __forceinline__ double gm_wave_sum(double t) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    return t;
+}
+
+// A lane's share of nb <= kGmGrid block sums; gm_wave_sum of it is their
+// total, in the same order in every wave.
+__device__ __forceinline__ double gm_share(const double* __restrict__ p, int nb) {
+    const int lane = threadIdx.x & 63;
+    double v[kGmGrid / 64];
+#pragma unroll
+    for (int q = 0; q < kGmGrid / 64; q++) v[q] = q * 64 < nb ? p[min(lane + 64 * q, nb - 1)] : 0.0;
+    double t = 0.0;
+#pragma unroll
+    for (int q = 0; q < kGmGrid / 64; q++) t += lane + 64 * q < nb ? v[q] : 0.0;
+    return t;
+}
+
+__device__ __forceinline__ void gm_publish(const GmDev& d, const GmState& s) {
+    __hip_atomic_store(&d.host->word, (int64_t)2 * s.its + s.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// One wave: the norm of the last w closes column kk - 1 (rotations,
+// residual estimate, convergence test), or opens a cycle when kk = 0.  Lane
+// j holds entry j of the column and rotation j, 64 entries at a time.
+__device__ __forceinline__ void gm_close_column(const GmDev& d, int kk) {
+    const int lane = threadIdx.x & 63, c = kk - 1;
+    const double nn = gm_share(d.pn, d.nb);
+    GmState s = *d.st;
+    const double gc = c >= 0 ? d.g[c] : 0.0;
+    if (s.done) return;
+    if (kk == 0) {
+        const double hn = sqrt(gm_wave_sum(nn));
+        if (lane == 0) {
+            s.kk = 0;
+            d.g[0] = hn;
+            if (s.first) {
+                s.first = 0;
+                s.rnorm0 = s.last = hn;
+                if (hn == 0.0 || hn <= s.atol) {
+                    s.reason = KSP_CONVERGED_ATOL;
+                    s.done = 1;
+                }
+            }
+            *d.st = s;
+            gm_publish(d, s);
+        }
+        return;
+    }
+    double* Rc = d.R + (size_t)c * (d.m + 1);
+    double a = 0.0;  // the entry that the next rotation takes, the same in every lane
+    for (int j0 = 0; j0 <= c; j0 += 64) {
+        const int j = j0 + lane;
+        const double h = j <= c ? d.h1[j] + d.h2[j] : 0.0;
+        const double cj = j < c ? d.cs[j] : 0.0, sj = j < c ? d.sn[j] : 0.0;
+        double r = 0.0;
+        for (int q = 0; q < min(64, c + 1 - j0); q++) {
+            const double b = gm_lane(h, q);  // entry j0 + q, rotated against a by rotation j0 + q - 1
+            if (j0 + q == 0) {
+                a = b;
+                continue;
+            }
+            const double cq = q > 0 ? gm_lane(cj, q - 1) : d.cs[j0 - 1], sq = q > 0 ? gm_lane(sj, q - 1) : d.sn[j0 - 1];
+            const double up = cq * a + sq * b;
+            if (q > 0) {
+                if (lane == q - 1) r = up;
+            } else if (lane == 0) {
+                Rc[j0 - 1] = up;
+            }
+            a = -sq * a + cq * b;
+        }
+        if (j < c && lane < 63) Rc[j] = r;
+    }
+    const double hn = sqrt(gm_wave_sum(nn));
+    if (lane == 0) {
+        const double den = sqrt(a * a + hn * hn);
+        const double cc = den == 0.0 ? 1.0 : a / den, sc = den == 0.0 ? 0.0 : hn / den;
+        d.cs[c] = cc;
+        d.sn[c] = sc;
+        Rc[c] = cc * a + sc * hn;
+        d.g[c + 1] = -sc * gc;
+        d.g[c] = cc * gc;
+        s.its += 1;
+        s.kk = c + 1;
+        s.last = fabs(-sc * gc);
+        if (s.last != s.last) s.reason = KSP_DIVERGED_NANORINF;
+        else if (s.last <= s.atol) s.reason = KSP_CONVERGED_ATOL;
+        else if (s.last <= s.rtol * s.rnorm0) s.reason = KSP_CONVERGED_RTOL;
+        else if (s.its >= s.max_its) s.reason = KSP_DIVERGED_ITS;
+        s.done = s.reason != 0;
+        *d.st = s;
+        gm_publish(d, s);
+    }
+}
+
+__global__ void k_gm_begin(GmDev d, double rtol, double atol, int max_its, int resume) {
+    GmState s = *d.st;
+    if (!resume) {
+        s.rnorm0 = s.last = 0.0;
+        s.rtol = rtol;
+        s.atol = atol;
+        s.its = 0;
+        s.max_its = max_its;
+        s.first = 1;
+    }
+    s.kk = 0;
+    s.reason = s.done = 0;
+    *d.st = s;
+    gm_publish(d, s);
+}
+
+// The scale that normalises w, from |w|^2 (0 for w = 0).
+__device__ __forceinline__ double gm_scale(double share) {
+    const double nrm = sqrt(gm_wave_sum(share));
+    return nrm > 0.0 ? 1.0 / nrm : 0.0;
+}
+
+// v = w / |w| and y = D^-1 A v (D^-1 absent: y = A v) over the slices of the
+// solver matrix.  The row
+// sums are formed from w and scaled at the end, so the norm's block sums are
+// in flight with the first slice.  The kernel holds nothing else: closing the
+// column here took it from 8 to 5 waves a SIMD (15 -> 22 us on 373k rows).
+template <typename V, typename CT>
+__global__ void __launch_bounds__(kRowBlock)
+k_gm_sell(SellOp<V, CT> m, const V* __restrict__ w, V* __restrict__ v, V* __restrict__ y,
+          const V* __restrict__ dinv, GmDev d) {
+    const double share = gm_share(d.pn, d.nb);
+    if (gm_done(d)) return;
+    constexpr int WPB = kRowBlock / kSlice;
+    constexpr int U = 8;
+    const int wave = threadIdx.x / kSlice, lane = threadIdx.x % kSlice;
+    const RowBlocks it((m.nsl + WPB - 1) / WPB);
+    for (int g = it.b; g < it.hi; g += it.step) {
+        const int sl = g * WPB + wave;
+        if (sl >= m.nsl) continue;
+        const int r0 = sl * kSlice, row = r0 + lane;
+        const int base = m.sptr[sl], wd = (m.sptr[sl + 1] - base) / kSlice;
+        const int rc = min(row, m.n - 1), len = row < m.n ? m.rowptr[rc + 1] - m.rowptr[rc] : 0;
+        const V wi = w[rc], di = dinv ? dinv[rc] : (V)1;
+        V acc = (V)0;
+        for (int j0 = 0; j0 < wd; j0 += U) {  // loads batched as in k_sell
+            int cj[U];
+            V av[U], xv[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int slot = base + min(j0 + u, wd - 1) * kSlice + lane;
+                cj[u] = csr_col(m.col, slot, r0);
+                av[u] = m.val[slot];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) xv[u] = w[cj[u]];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (j0 + u < len) acc += av[u] * xv[u];
+        }
+        const double s = gm_scale(share);
+        if (row < m.n) {
+            v[row] = (V)((double)wi * s);
+            y[row] = di * (V)((double)acc * s);
+        }
+    }
+}
+
+// The same over the CSR matrix, L lanes a row.
 template <int L, typename V>
 __global__ void __launch_bounds__(kRowBlock)
-k_gm_matvec(int n, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-            const V* __restrict__ val, const V* __restrict__ dinv, const V* __restrict__ x,
-            V* __restrict__ y) {
+k_gm_csr(int n, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col, const V* __restrict__ val,
+         const V* __restrict__ w, V* __restrict__ v, V* __restrict__ y, const V* __restrict__ dinv, GmDev d) {
+    const double share = gm_share(d.pn, d.nb);
+    if (gm_done(d)) return;
+    const double s = gm_scale(share);
     constexpr int ROWS = kRowBlock / L;
     const int lane = threadIdx.x % L, rloc = threadIdx.x / L;
     for (int grp = blockIdx.x; grp * ROWS < n; grp += gridDim.x) {
         const int row = grp * ROWS + rloc;
         V acc = (V)0;
         if (row < n)
-            for (int k = rowptr[row] + lane; k < rowptr[row + 1]; k += L) acc += val[k] * x[col[k]];
-        acc = lane_sum<V>(acc, L);
-        if (row < n && lane == 0) y[row] = dinv ? dinv[row] * acc : acc;
+            for (int k = rowptr[row] + lane; k < rowptr[row + 1]; k += L) acc += val[k] * w[col[k]];
+        for (int off = L >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+        if (row < n && lane == 0) {
+            v[row] = (V)((double)w[row] * s);
+            y[row] = (dinv ? dinv[row] : (V)1) * (V)((double)acc * s);
+        }
     }
 }
 
-// h[j] = w . V_j for j <= kk (one pass over w), partials per block
-template <typename V>
-__global__ void __launch_bounds__(kVecBlock)
-k_gm_dots(int n, int kk, const V* __restrict__ Vb, const V* __restrict__ w,
-          double* __restrict__ partials) {
-    __shared__ double sh[kVecBlock / 64][1];
-    for (int j = 0; j <= kk; j++) {
-        const V* vj = Vb + (size_t)n * j;
-        double s = 0.0;
-        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-            s += (double)w[i] * (double)vj[i];
-        double a[1] = {s};
-        block_sum<1>(a, sh);
-        if (threadIdx.x == 0) partials[(size_t)j * gridDim.x + blockIdx.x] = a[0];
+// One step of gm_block_sums on the first 2 HALF values: lane pairs at
+// distance MASK exchange, each keeps HALF sums; then the steps below it.
+template <int HALF, int MASK, int NB>
+__device__ __forceinline__ void gm_halve(double (&a)[NB], int lane, int& j) {
+    if constexpr (HALF > 0) {
+        const bool hi = lane & MASK;
+#pragma unroll
+        for (int q = 0; q < HALF; q++) {
+            const double keep = hi ? a[q + HALF] : a[q], send = hi ? a[q] : a[q + HALF];
+            a[q] = keep + __shfl_xor(send, MASK, 64);
+        }
+        j += hi ? HALF : 0;
+        gm_halve<HALF / 2, MASK / 2, NB>(a, lane, j);
+    } else if constexpr (MASK > 0) {
+        a[0] += __shfl_xor(a[0], MASK, 64);
+        gm_halve<0, MASK / 2, NB>(a, lane, j);
     }
 }
 
-// hcol[j] (+)= sum over blocks (fixed order); one block per j
-__global__ void k_gm_reduce(int kk, int nblk, const double* __restrict__ partials,
-                            double* __restrict__ hcol, int accumulate) {
-    __shared__ double sh[kVecBlock / 64][1];
-    const int j = blockIdx.x;
-    if (j > kk) return;
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += partials[(size_t)j * nblk + b];
-    double a[1] = {s};
-    block_sum<1>(a, sh);
-    if (threadIdx.x == 0) hcol[j] = accumulate ? hcol[j] + a[0] : a[0];
+// Sums NB (8, 16 or 32) per-thread values over the block: each step of a
+// wave halves the values a lane still carries (it sends the half its partner
+// keeps), so NB sums take about 2 NB shuffles and not 12 NB.  out[j] for j < nv.
+template <int NB, int B>
+__device__ __forceinline__ void gm_block_sums(double (&a)[NB], int nv, double* __restrict__ out, int stride) {
+    __shared__ double sh[B / 64][NB];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int j = 0;
+    gm_halve<NB / 2, 32, NB>(a, lane, j);
+    __syncthreads();  // the last use of sh
+    if ((lane & (64 / NB - 1)) == 0) sh[wave][j] = a[0];
+    __syncthreads();
+    if ((int)threadIdx.x < NB && (int)threadIdx.x < nv) {
+        double t = sh[0][threadIdx.x];
+#pragma unroll
+        for (int q = 1; q < B / 64; q++) t += sh[q][threadIdx.x];
+        out[(size_t)threadIdx.x * stride] = t;
+    }
 }
 
-// w -= sum_j h[j] V_j  (h from hcol, or its second-pass increment)
+// Totals of the block sums of nv <= NB basis vectors, into LDS (zero past
+// nv): 16 lanes a vector when there are at most 16 blocks, a wave a vector
+// otherwise, every load issued before the first sum.
+template <int NB, int B>
+__device__ __forceinline__ void gm_totals(const double* __restrict__ p, int nv, int nb, double (&sh)[NB],
+                                          double* __restrict__ h) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (nb <= 16) {
+        const int j = threadIdx.x >> 4, b = threadIdx.x & 15;
+        double t = j < nv && b < nb ? p[(size_t)j * nb + b] : 0.0;
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        if (b == 0 && j < NB) sh[j] = t;
+    } else {
+        constexpr int W = B / 64, R = (NB + W - 1) / W;
+        double t[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int j = wave + r * W;
+            t[r] = j < nv ? gm_share(p + (size_t)j * nb, nb) : 0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            t[r] = gm_wave_sum(t[r]);
+            const int j = wave + r * W;
+            if (lane == 0 && j < NB) sh[j] = t[r];
+        }
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && (int)threadIdx.x < nv) h[threadIdx.x] = sh[threadIdx.x];
+}
+
+// Row i of basis vectors 0 .. nv-1 (1 <= nv <= 8 for NB = 8, NB / 2 < nv <= NB
+// beyond; past nv the last one again): unconditional loads, all in flight
+// together.
+template <typename V, int NB>
+__device__ __forceinline__ void gm_load(const V* __restrict__ Vb, size_t ldv, int nv, int i, V (&t)[NB]) {
+    const V* q = Vb + i;
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        t[j] = *q;
+        if ((NB > 8 && j < NB / 2) || j + 1 < nv) q += ldv;
+    }
+}
+
+// p1_j = block sums of w . v_j for j < nv; the last workgroup closes the
+// previous column.
+template <typename V, int NB>
+__global__ void __launch_bounds__(gm_block(NB))
+k_gm_dots(int n, size_t ldv, int nv, const V* __restrict__ Vb, const V* __restrict__ w, GmDev d) {
+    constexpr int B = gm_block(NB);
+    if ((int)blockIdx.x == d.nb) {
+        if (threadIdx.x < 64) gm_close_column(d, nv - 1);
+        return;
+    }
+    const int done = gm_done(d), step = d.nb * B;
+    const int i0 = blockIdx.x * B + threadIdx.x;
+    V t[NB], wi = (V)0;
+    if (i0 < n) {
+        gm_load<V, NB>(Vb, ldv, nv, i0, t);
+        wi = w[i0];
+    }
+    if (done) return;
+    double acc[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) acc[j] = 0.0;
+    for (int i = i0; i < n; i += step) {
+        if (i != i0) {
+            gm_load<V, NB>(Vb, ldv, nv, i, t);
+            wi = w[i];
+        }
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[j] = fma((double)wi, (double)t[j], acc[j]);
+    }
+    gm_block_sums<NB, B>(acc, nv, d.p1 + blockIdx.x, d.nb);
+}
+
+// w -= sum_j h_j v_j (j < nv), h the totals of the block sums p; then, from
+// the vectors still in registers, the block sums of w . v_j (DOTS) or of
+// |w|^2 (otherwise).  The first rows' loads are issued before the totals.
+template <typename V, int NB, bool DOTS>
+__global__ void __launch_bounds__(gm_block(NB))
+k_gm_orth(int n, size_t ldv, int nv, const V* __restrict__ Vb, V* __restrict__ w, const double* __restrict__ p,
+          double* __restrict__ h, double* __restrict__ out, GmDev d) {
+    constexpr int B = gm_block(NB);
+    __shared__ double sh[NB];
+    const int done = gm_done(d);
+    const int i0 = blockIdx.x * B + threadIdx.x;
+    V t[NB], wi = (V)0;
+    if (i0 < n) {
+        gm_load<V, NB>(Vb, ldv, nv, i0, t);
+        wi = w[i0];
+    }
+    if (done) return;
+    gm_totals<NB, B>(p, nv, d.nb, sh, h);
+    double acc[DOTS ? NB : 1];
+#pragma unroll
+    for (int j = 0; j < (DOTS ? NB : 1); j++) acc[j] = 0.0;
+    for (int i = i0; i < n; i += gridDim.x * B) {
+        if (i != i0) {
+            gm_load<V, NB>(Vb, ldv, nv, i, t);
+            wi = w[i];
+        }
+        double a = (double)wi;
+#pragma unroll
+        for (int j = 0; j < NB; j++) a = fma(-sh[j], (double)t[j], a);
+        const V o = (V)a;
+        w[i] = o;
+        if (DOTS) {
+#pragma unroll
+            for (int j = 0; j < NB; j++) acc[j] = fma((double)o, (double)t[j], acc[j]);
+        } else {
+            acc[0] = fma((double)o, (double)o, acc[0]);
+        }
+    }
+    if constexpr (DOTS) {
+        gm_block_sums<NB, B>(acc, nv, out + blockIdx.x, d.nb);
+    } else {
+        __shared__ double sn[B / 64][1];
+        block_sum<1>(acc, sn);
+        if (threadIdx.x == 0) out[blockIdx.x] = acc[0];
+    }
+}
+
+// The same for a basis longer than the registers hold, kGmReg vectors at a
+// time (h given), and the totals by a launch of their own.
 template <typename V>
-__global__ void __launch_bounds__(kVecBlock)
-k_gm_orth(int n, int kk, const V* __restrict__ Vb, const double* __restrict__ h, V* __restrict__ w) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        double acc = (double)w[i];
-        for (int j = 0; j <= kk; j++) acc -= h[j] * (double)Vb[(size_t)n * j + i];
-        w[i] = (V)acc;
+__global__ void __launch_bounds__(gm_block(kGmReg))
+k_gm_dots_long(int n, size_t ldv, int nv, const V* __restrict__ Vb, const V* __restrict__ w, double* __restrict__ out,
+               GmDev d) {
+    constexpr int B = gm_block(kGmReg);
+    if ((int)blockIdx.x == d.nb) {
+        if (threadIdx.x < 64) gm_close_column(d, nv - 1);
+        return;
+    }
+    if (gm_done(d)) return;
+    for (int c0 = 0; c0 < nv; c0 += kGmReg) {
+        double acc[kGmReg];
+#pragma unroll
+        for (int j = 0; j < kGmReg; j++) acc[j] = 0.0;
+        for (int i = blockIdx.x * B + threadIdx.x; i < n; i += d.nb * B) {
+            const double wi = (double)w[i];
+#pragma unroll
+            for (int j = 0; j < kGmReg; j++) acc[j] = fma(wi, (double)Vb[ldv * min(c0 + j, nv - 1) + i], acc[j]);
+        }
+        gm_block_sums<kGmReg, B>(acc, nv - c0, out + (size_t)c0 * d.nb + blockIdx.x, d.nb);
     }
 }
 
 template <typename V>
-__global__ void __launch_bounds__(kVecBlock)
-k_gm_scale(int n, const V* __restrict__ w, V* __restrict__ out, const double* __restrict__ nrm) {
-    const double s = nrm[0] > 0 ? 1.0 / nrm[0] : 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        out[i] = (V)((double)w[i] * s);
+__global__ void __launch_bounds__(gm_block(kGmReg))
+k_gm_orth_long(int n, size_t ldv, int nv, const V* __restrict__ Vb, V* __restrict__ w, const double* __restrict__ h,
+               double* __restrict__ pn, GmDev d) {
+    constexpr int B = gm_block(kGmReg);
+    if (gm_done(d)) return;
+    double acc[1] = {0.0};
+    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
+        double a = (double)w[i];
+#pragma unroll 8
+        for (int j = 0; j < nv; j++) a = fma(-h[j], (double)Vb[ldv * j + i], a);
+        const V o = (V)a;
+        w[i] = o;
+        acc[0] = fma((double)o, (double)o, acc[0]);
+    }
+    __shared__ double sn[B / 64][1];
+    block_sum<1>(acc, sn);
+    if (threadIdx.x == 0) pn[blockIdx.x] = acc[0];
+}
+
+__global__ void __launch_bounds__(64)
+k_gm_reduce(GmDev d, const double* __restrict__ p, double* __restrict__ h) {
+    const double t = gm_wave_sum(gm_share(p + (size_t)blockIdx.x * d.nb, d.nb));
+    if (!gm_done(d) && threadIdx.x == 0) h[blockIdx.x] = t;
+}
+
+constexpr int kGmNormBlock = 1024;
+
+// w = D^-1 r64 (D^-1 absent: r64) in the working precision, and |w|^2.
+template <typename V>
+__global__ void __launch_bounds__(kGmNormBlock)
+k_gm_precres_norm(int n, const double* __restrict__ r64, const double* __restrict__ dinv, V* __restrict__ out,
+                  GmDev d) {
+    double nn = 0.0;
+    for (int i = blockIdx.x * kGmNormBlock + threadIdx.x; i < n; i += gridDim.x * kGmNormBlock) {
+        const V o = dinv ? (V)(dinv[i] * r64[i]) : (V)r64[i];
+        out[i] = o;
+        nn += (double)o * (double)o;
+    }
+    double a[1] = {nn};
+    __shared__ double sn[kGmNormBlock / 64][1];
+    block_sum<1>(a, sn);
+    if (threadIdx.x == 0) d.pn[blockIdx.x] = a[0];
 }
 
 template <typename V>
-__global__ void __launch_bounds__(kVecBlock)
-k_gm_norm(int n, const V* __restrict__ w, double* __restrict__ partials) {
-    __shared__ double sh[kVecBlock / 64][1];
-    double s = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        s += (double)w[i] * (double)w[i];
-    double a[1] = {s};
-    block_sum<1>(a, sh);
-    if (threadIdx.x == 0) partials[blockIdx.x] = a[0];
+__global__ void __launch_bounds__(kGmNormBlock)
+k_gm_norm(int n, const V* __restrict__ w, GmDev d) {
+    double nn = 0.0;
+    for (int i = blockIdx.x * kGmNormBlock + threadIdx.x; i < n; i += gridDim.x * kGmNormBlock)
+        nn += (double)w[i] * (double)w[i];
+    double a[1] = {nn};
+    __shared__ double sn[kGmNormBlock / 64][1];
+    block_sum<1>(a, sn);
+    if (threadIdx.x == 0) d.pn[blockIdx.x] = a[0];
 }
 
-__global__ void k_gm_sqrt_reduce(int nblk, const double* __restrict__ partials, double* __restrict__ out) {
-    __shared__ double sh[kVecBlock / 64][1];
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += partials[b];
-    double a[1] = {s};
-    block_sum<1>(a, sh);
-    if (threadIdx.x == 0) out[0] = sqrt(a[0]);
+// One wave: closes column kk - 1 if the solve has not finished before it,
+// then y = R^-1 g over the cycle's columns.  Up to 64 columns, lane j keeps
+// g_j and the triangle is staged in LDS; y_i = g_i / R_ii by the reciprocals,
+// formed together, and one correction.
+__global__ void __launch_bounds__(64)
+k_gm_cycle_end(GmDev d, int kk) {
+    constexpr int N = 64;
+    __shared__ double sR[N * (N + 1) / 2];
+    if (kk > 0) gm_close_column(d, kk);
+    __syncthreads();
+    const int nc = __hip_atomic_load(&d.st->kk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), lane = threadIdx.x;
+    const int ld = d.m + 1;
+    if (nc <= N) {
+        for (int i = 0; i < nc; i++)
+            if (lane <= i) sR[i * (i + 1) / 2 + lane] = d.R[(size_t)i * ld + lane];
+        double g = lane < nc ? d.g[lane] : 0.0;
+        __syncthreads();
+        const double rd = lane < nc ? sR[lane * (lane + 1) / 2 + lane] : 1.0, inv = 1.0 / rd;
+        double y = 0.0;
+        for (int i = nc - 1; i >= 0; i--) {
+            const double gi = gm_lane(g, i), ri = gm_lane(rd, i), vi = gm_lane(inv, i);
+            double yi = gi * vi;
+            const double e = fma(-yi, ri, gi) * vi;
+            if (e == e) yi += e;
+            if (lane == i) y = yi;
+            if (lane < i) g = fma(-sR[i * (i + 1) / 2 + lane], yi, g);
+        }
+        if (lane < nc) d.y[lane] = y;
+        return;
+    }
+    for (int j = lane; j < nc; j += 64) d.y[j] = d.g[j];
+    __syncthreads();
+    for (int i = nc - 1; i >= 0; i--) {
+        const double yi = d.y[i] / d.R[(size_t)i * ld + i];
+        __syncthreads();
+        for (int j = lane; j < i; j += 64) d.y[j] -= d.R[(size_t)i * ld + j] * yi;
+        if (lane == 0) d.y[i] = yi;
+        __syncthreads();
+    }
 }
 
-// x += sum_j y_j V_j
+// x += sum_j y_j v_j over the cycle's columns
 template <typename V>
 __global__ void __launch_bounds__(kVecBlock)
-k_gm_update_x(int n, int kk, const V* __restrict__ Vb, const double* __restrict__ y, double* __restrict__ x) {
+k_gm_update_x(int n, size_t ldv, const V* __restrict__ Vb, GmDev d, double* __restrict__ x) {
+    const int kk = d.st->kk;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         double acc = x[i];
-        for (int j = 0; j < kk; j++) acc += y[j] * (double)Vb[(size_t)n * j + i];
+#pragma unroll 8
+        for (int j = 0; j < kk; j++) acc += d.y[j] * (double)Vb[ldv * j + i];
         x[i] = acc;
     }
 }
 
-// r_V = D^-1 r64  (left-preconditioned residual of the FP64 residual)
+// z = D^-1 r64 or r64 (pc_apply_host)
 template <typename V>
 __global__ void __launch_bounds__(kVecBlock)
 k_gm_precres(int n, const double* __restrict__ r64, const double* __restrict__ dinv, V* __restrict__ out) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
         out[i] = dinv ? (V)(dinv[i] * r64[i]) : (V)r64[i];
+}
+
+// Waits until the device has closed `its` columns or the solve is done; a
+// stream that ran dry or failed before that ends the wait.
+static int gm_wait(flgpu_ctx* c, const GmHost* host, int64_t its) {
+    for (unsigned spin = 1;; spin++) {
+        const int64_t w = __atomic_load_n(&host->word, __ATOMIC_ACQUIRE);
+        if ((w & 1) || w / 2 >= its) return FLGPU_OK;
+        if (spin % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(c->stream);
+            if (e == hipErrorNotReady) continue;
+            FLGPU_HIP(e);
+            const int64_t w2 = __atomic_load_n(&host->word, __ATOMIC_ACQUIRE);
+            if ((w2 & 1) || w2 / 2 >= its) return FLGPU_OK;
+            return set_error(FLGPU_EHIP, "flgpu_solve: gmres stopped at iteration %lld of %lld",
+                             (long long)(w2 / 2), (long long)its);
+        }
+    }
 }
 
 template <typename V>
@@ -1572,13 +2039,19 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
     const bool mixed = std::is_same<V, float>::value;
     const V* val = mixed ? (const V*)k->val32.p : (const V*)k->val64.p;
     const V* dinv = mixed ? (const V*)k->dinv32.p : (const V*)k->dinv.p;
+    const size_t ldv = ((size_t)n + 31) & ~(size_t)31;  // basis vectors start on whole lines
     V* Vb;
+    V* wb[2];  // the product reads one and writes the other
     if (mixed) {
-        FLGPU_TRY(k->V32.alloc((size_t)n * (m + 1)));
+        FLGPU_TRY(k->V32.alloc(ldv * m));
         Vb = (V*)k->V32.p;
+        wb[0] = (V*)k->w32.p;
+        wb[1] = (V*)k->z32.p;
     } else {
-        FLGPU_TRY(k->V.alloc((size_t)n * (m + 1)));
+        FLGPU_TRY(k->V.alloc(ldv * m));
         Vb = (V*)k->V.p;
+        wb[0] = (V*)k->w.p;
+        wb[1] = (V*)k->z.p;
     }
     if (sp->pc == FLGPU_PC_NONE) {
         hipLaunchKernelGGL((k_fill<double>), dim3(k->nblk), dim3(kVecBlock), 0, c->stream, n, 1.0, k->dinv.p);
@@ -1590,135 +2063,142 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
     const bool ssor = sp->pc == FLGPU_PC_SOR;
     if (ssor) FLGPU_TRY(ssor_prepare(c, k));
     V* tmp = mixed ? (V*)k->rt32.p : (V*)k->rt.p;
-    FLGPU_TRY(k->hcol.alloc(m + 2));
-    FLGPU_TRY(k->partials.reserve((size_t)kMaxVecGrid * (m + 2)));
-    const int nb = k->nblk;
+    const int nb = std::max(1, (int)std::min<int64_t>(kGmGrid, ((int64_t)n + 511) / 512));
+    const size_t mm = (size_t)m + 1;
+    FLGPU_TRY(k->gm_work.reserve((2 * mm + 1) * kGmGrid + 7 * mm + mm * m));
+    FLGPU_TRY(k->gm_state.reserve(sizeof(GmState)));
+    if (!k->gm_host) {
+        FLGPU_HIP(hipHostMalloc((void**)&k->gm_host, sizeof(GmHost), hipHostMallocMapped | hipHostMallocCoherent));
+        std::memset(k->gm_host, 0, sizeof(GmHost));
+    }
+    GmHost* host = static_cast<GmHost*>(k->gm_host);
+    GmDev d{};
+    d.st = reinterpret_cast<GmState*>(k->gm_state.p);
+    FLGPU_HIP(hipHostGetDevicePointer((void**)&d.host, host, 0));
+    d.m = m;
+    d.nb = nb;
+    d.p1 = k->gm_work.p;
+    d.p2 = d.p1 + mm * kGmGrid;
+    d.pn = d.p2 + mm * kGmGrid;
+    d.h1 = d.pn + kGmGrid;
+    d.h2 = d.h1 + mm;
+    d.g = d.h2 + mm;
+    d.cs = d.g + mm;
+    d.sn = d.cs + mm;
+    d.y = d.sn + mm;
+    d.R = d.y + mm;
     const int L = lanes_for(c);
     const int rows_per_blk = kRowBlock / L;
-    int mgrid = (int)std::min<int64_t>(kMaxRowGrid, (n + rows_per_blk - 1) / rows_per_blk);
-    mgrid = std::max(mgrid, 1);
-    auto matvec = [&](const V* xin, V* yout) -> int {
-#define FL_GMV(LL)                                                                                         \
-    case LL:                                                                                               \
-        hipLaunchKernelGGL((k_gm_matvec<LL, V>), dim3(mgrid), dim3(kRowBlock), 0, c->stream, n, c->rowptr.p, \
-                           c->col.p, val, ssor ? nullptr : dinv, xin, ssor ? tmp : yout);                  \
-        break;
-        switch (L) {
-            FL_GMV(4)
-            FL_GMV(8)
-            FL_GMV(16)
-            FL_GMV(32)
-            FL_GMV(64)
+    const int mgrid = std::max(1, (int)std::min<int64_t>(kMaxRowGrid, (n + rows_per_blk - 1) / rows_per_blk));
+    const V* sval = sell_values(k, val);
+    auto product = [&](const V* w, V* v, V* out) -> int {
+        const V* dv = ssor ? nullptr : dinv;
+        V* y = ssor ? tmp : out;
+        if (sval) {
+            const int grid = sell_grid(k->nsl);
+            if (k->sell16) {
+                const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol16.p, sval, nullptr};
+                hipLaunchKernelGGL((k_gm_sell<V, int16_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
+                                   d);
+            } else {
+                const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol32.p, sval, nullptr};
+                hipLaunchKernelGGL((k_gm_sell<V, int32_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
+                                   d);
+            }
+        } else {
+            auto launch = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(mgrid), dim3(kRowBlock), 0, c->stream, n, c->rowptr.p, c->col.p, val,
+                                   w, v, y, dv, d);
+            };
+            switch (L) {
+                case 4: launch(&k_gm_csr<4, V>); break;
+                case 8: launch(&k_gm_csr<8, V>); break;
+                case 16: launch(&k_gm_csr<16, V>); break;
+                case 32: launch(&k_gm_csr<32, V>); break;
+                default: launch(&k_gm_csr<64, V>); break;
+            }
         }
-#undef FL_GMV
-        if (ssor) FLGPU_TRY(ssor_sweeps<V>(c, k, val, tmp, yout, nullptr));
+        if (ssor) FLGPU_TRY(ssor_sweeps<V>(c, k, val, tmp, out, &d.st->done));
         return FLGPU_OK;
     };
-    std::vector<double> H((size_t)(m + 1) * m), g(m + 1), cs(m), sn(m), y(m), hc(m + 2);
-    double hn = 0.0;
-    int total = 0, reason = 0;
-    double rnorm0 = -1.0, last = 0.0;
+    // Gram-Schmidt of w against nv basis vectors, twice, and |w|^2
+    auto orthogonalise = [&](V* w, int nv) {
+        auto pass = [&](auto nbc) {
+            constexpr int NB = decltype(nbc)::value;
+            const dim3 grid(nb), block(gm_block(NB));
+            hipLaunchKernelGGL((k_gm_dots<V, NB>), dim3(nb + 1), block, 0, c->stream, n, ldv, nv, Vb, w, d);
+            hipLaunchKernelGGL((k_gm_orth<V, NB, true>), grid, block, 0, c->stream, n, ldv, nv, Vb, w, d.p1, d.h1,
+                               d.p2, d);
+            hipLaunchKernelGGL((k_gm_orth<V, NB, false>), grid, block, 0, c->stream, n, ldv, nv, Vb, w, d.p2, d.h2,
+                               d.pn, d);
+        };
+        if (nv <= 8) return pass(std::integral_constant<int, 8>());
+        if (nv <= 16) return pass(std::integral_constant<int, 16>());
+        if (nv <= kGmReg) return pass(std::integral_constant<int, kGmReg>());
+        const dim3 grid(nb), block(gm_block(kGmReg));
+        for (int q = 0; q < 2; q++) {
+            double *pq = q ? d.p2 : d.p1, *hq = q ? d.h2 : d.h1;
+            hipLaunchKernelGGL((k_gm_dots_long<V>), dim3(q ? nb : nb + 1), block, 0, c->stream, n, ldv, nv, Vb, w, pq, d);
+            hipLaunchKernelGGL(k_gm_reduce, dim3(nv), dim3(64), 0, c->stream, d, pq, hq);
+            hipLaunchKernelGGL((k_gm_orth_long<V>), grid, block, 0, c->stream, n, ldv, nv, Vb, w, hq, d.pn, d);
+        }
+    };
+    const int max_its = sp->max_its > 0 ? sp->max_its : 10000;
     Scal& h = *k->h_scal;
     std::memset(&h, 0, sizeof h);
     FLGPU_TRY(write_scal(c, k));
     FLGPU_TRY(norm_b(c, k));
-    FLGPU_TRY(read_scal(c, k));
-    const double bnorm = std::sqrt(h.bb);
+    host->word = 0;
+    hipLaunchKernelGGL(k_gm_begin, dim3(1), dim3(1), 0, c->stream, d, sp->rtol, sp->atol, max_its, 0);
     auto t0 = std::chrono::steady_clock::now();
     int refinements = 0;
-    while (!reason) {
+    bool have_residual = false;
+    for (;;) {
         // residual in FP64, preconditioned, in the working precision
-        FLGPU_TRY(true_residual(c, k));
-        hipLaunchKernelGGL((k_gm_precres<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, k->r.p,
-                           ssor ? nullptr : k->dinv.p, ssor ? tmp : Vb);
-        if (ssor) FLGPU_TRY(ssor_sweeps<V>(c, k, val, tmp, Vb, nullptr));
-        hipLaunchKernelGGL((k_gm_norm<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, Vb, k->partials.p);
-        hipLaunchKernelGGL(k_gm_sqrt_reduce, dim3(1), dim3(kVecBlock), 0, c->stream, nb, k->partials.p, k->hcol.p);
-        FLGPU_HIP(hipMemcpyAsync(&hn, k->hcol.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        FLGPU_HIP(hipStreamSynchronize(c->stream));
-        refinements++;
-        const double beta = hn;
-        if (rnorm0 < 0) {
-            rnorm0 = beta;
-            last = beta;
-            if (beta == 0.0 || beta <= sp->atol) {
-                reason = KSP_CONVERGED_ATOL;
-                break;
-            }
+        if (!have_residual) FLGPU_TRY(true_residual(c, k));
+        have_residual = false;
+        int cur = 0;
+        hipLaunchKernelGGL((k_gm_precres_norm<V>), dim3(nb), dim3(kGmNormBlock), 0, c->stream, n, k->r.p,
+                           ssor ? nullptr : k->dinv.p, ssor ? tmp : wb[0], d);
+        if (ssor) {
+            FLGPU_TRY(ssor_sweeps<V>(c, k, val, tmp, wb[0], nullptr));
+            hipLaunchKernelGGL((k_gm_norm<V>), dim3(nb), dim3(kGmNormBlock), 0, c->stream, n, wb[0], d);
         }
-        hipLaunchKernelGGL((k_gm_scale<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, Vb, Vb, k->hcol.p);
-        std::fill(g.begin(), g.end(), 0.0);
-        g[0] = beta;
-        int kk;
-        for (kk = 0; kk < m && !reason; kk++) {
-            V* vk = Vb + (size_t)n * kk;
-            V* vn = Vb + (size_t)n * (kk + 1);
-            FLGPU_TRY(matvec(vk, vn));
-            // classical Gram-Schmidt, twice
-            for (int pass = 0; pass < 2; pass++) {
-                hipLaunchKernelGGL((k_gm_dots<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, kk, Vb, vn,
-                                   k->partials.p);
-                hipLaunchKernelGGL(k_gm_reduce, dim3(kk + 1), dim3(kVecBlock), 0, c->stream, kk, nb, k->partials.p,
-                                   k->hcol.p + 1, 0);
-                hipLaunchKernelGGL((k_gm_orth<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, kk, Vb,
-                                   k->hcol.p + 1, vn);
-                FLGPU_HIP(hipMemcpyAsync(hc.data(), k->hcol.p + 1, sizeof(double) * (kk + 1),
-                                         hipMemcpyDeviceToHost, c->stream));
-                FLGPU_HIP(hipStreamSynchronize(c->stream));
-                for (int j = 0; j <= kk; j++) H[j + (m + 1) * kk] = (pass == 0 ? 0.0 : H[j + (m + 1) * kk]) + hc[j];
-            }
-            hipLaunchKernelGGL((k_gm_norm<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, vn, k->partials.p);
-            hipLaunchKernelGGL(k_gm_sqrt_reduce, dim3(1), dim3(kVecBlock), 0, c->stream, nb, k->partials.p, k->hcol.p);
-            hipLaunchKernelGGL((k_gm_scale<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, vn, vn, k->hcol.p);
-            FLGPU_HIP(hipMemcpyAsync(&hn, k->hcol.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            FLGPU_HIP(hipStreamSynchronize(c->stream));
-            H[kk + 1 + (m + 1) * kk] = hn;
-            for (int j = 0; j < kk; j++) {
-                const double a = H[j + (m + 1) * kk], b2 = H[j + 1 + (m + 1) * kk];
-                H[j + (m + 1) * kk] = cs[j] * a + sn[j] * b2;
-                H[j + 1 + (m + 1) * kk] = -sn[j] * a + cs[j] * b2;
-            }
-            const double a = H[kk + (m + 1) * kk], b2 = H[kk + 1 + (m + 1) * kk];
-            const double den = std::sqrt(a * a + b2 * b2);
-            cs[kk] = den == 0.0 ? 1.0 : a / den;
-            sn[kk] = den == 0.0 ? 0.0 : b2 / den;
-            H[kk + (m + 1) * kk] = cs[kk] * a + sn[kk] * b2;
-            H[kk + 1 + (m + 1) * kk] = 0.0;
-            g[kk + 1] = -sn[kk] * g[kk];
-            g[kk] = cs[kk] * g[kk];
-            total++;
-            last = std::fabs(g[kk + 1]);
-            if (last != last) reason = KSP_DIVERGED_NANORINF;
-            else if (last <= sp->atol) reason = KSP_CONVERGED_ATOL;
-            else if (last <= sp->rtol * rnorm0) reason = KSP_CONVERGED_RTOL;
-            else if (total >= (sp->max_its > 0 ? sp->max_its : 10000)) reason = KSP_DIVERGED_ITS;
-        }
-        for (int i = kk - 1; i >= 0; i--) {
-            double acc = g[i];
-            for (int j = i + 1; j < kk; j++) acc -= H[i + (m + 1) * j] * y[j];
-            y[i] = acc / H[i + (m + 1) * i];
-        }
-        FLGPU_HIP(hipMemcpyAsync(k->hcol.p, y.data(), sizeof(double) * kk, hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL((k_gm_update_x<V>), dim3(nb), dim3(kVecBlock), 0, c->stream, n, kk, Vb, k->hcol.p,
-                           k->x.p);
         FLGPU_HIP(hipGetLastError());
-        if (mixed && reason > 0) {
-            // the FP32 estimate converged: test the FP64 residual
-            FLGPU_TRY(true_residual(c, k));
-            FLGPU_TRY(read_scal(c, k));
-            if (std::sqrt(h.true_rr) > std::max(sp->rtol * bnorm, sp->atol) &&
-                total < (sp->max_its > 0 ? sp->max_its : 10000))
-                reason = 0;
+        refinements++;
+        const int64_t before = host->word / 2;  // closed columns of the earlier cycles: none is in flight
+        int kk = 0;
+        for (; kk < m; kk++) {
+            FLGPU_TRY(gm_wait(c, host, before + kk - kGmAhead));
+            if (__atomic_load_n(&host->word, __ATOMIC_ACQUIRE) & 1) break;
+            FLGPU_TRY(product(wb[cur], Vb + ldv * kk, wb[cur ^ 1]));
+            cur ^= 1;
+            orthogonalise(wb[cur], kk + 1);
+            FLGPU_HIP(hipGetLastError());
         }
+        hipLaunchKernelGGL(k_gm_cycle_end, dim3(1), dim3(64), 0, c->stream, d, kk);
+        hipLaunchKernelGGL((k_gm_update_x<V>), dim3(k->nblk), dim3(kVecBlock), 0, c->stream, n, ldv, Vb, d, k->x.p);
+        FLGPU_HIP(hipGetLastError());
+        FLGPU_TRY(gm_wait(c, host, before + kk));
+        if (!(__atomic_load_n(&host->word, __ATOMIC_ACQUIRE) & 1)) continue;
+        FLGPU_TRY(true_residual(c, k));
+        FLGPU_HIP(hipMemcpyAsync(&host->st, d.st, sizeof(GmState), hipMemcpyDeviceToHost, c->stream));
+        FLGPU_TRY(read_scal(c, k));
+        // mixed: the FP32 estimate converged, the FP64 residual decides
+        if (!mixed || host->st.reason <= 0 || std::sqrt(h.true_rr) <= std::max(sp->rtol * std::sqrt(h.bb), sp->atol) ||
+            host->st.its >= max_its)
+            break;
+        host->word = (int64_t)2 * host->st.its;
+        hipLaunchKernelGGL(k_gm_begin, dim3(1), dim3(1), 0, c->stream, d, sp->rtol, sp->atol, max_its, 1);
+        have_residual = true;
     }
-    FLGPU_TRY(true_residual(c, k));
-    FLGPU_TRY(read_scal(c, k));
     auto t1 = std::chrono::steady_clock::now();
+    const double bnorm = std::sqrt(h.bb);
     info->seconds = std::chrono::duration<double>(t1 - t0).count();
-    info->its = total;
-    info->reason = reason;
+    info->its = host->st.its;
+    info->reason = host->st.reason;
     info->true_relres = bnorm > 0 ? std::sqrt(h.true_rr) / bnorm : std::sqrt(h.true_rr);
-    info->precond_relres = rnorm0 > 0 ? last / rnorm0 : last;
+    info->precond_relres = host->st.rnorm0 > 0 ? host->st.last / host->st.rnorm0 : host->st.last;
     info->refinements = mixed ? refinements : 0;
     info->fallback = 0;
     return FLGPU_OK;

@@ -134,15 +134,17 @@ enum { DOT_NONE = 0, DOT_XY = 1, DOT_PC = 2 };
 // and nodes that neighbouring rows gather stay in one L2.
 struct RowBlocks {
     int b, hi, step;
-    __device__ __forceinline__ explicit RowBlocks(int nrb) {
-        b = blockIdx.x;
+    __device__ __forceinline__ explicit RowBlocks(int nrb) : RowBlocks(nrb, blockIdx.x, gridDim.x) {}
+    // as workgroup `wg` of the first `n` of the grid
+    __device__ __forceinline__ RowBlocks(int nrb, int wg, int n) {
+        b = wg;
         hi = nrb;
-        step = gridDim.x;
-        if ((gridDim.x & 7) == 0) {
-            const int xcd = blockIdx.x & 7;
-            b = (int)((int64_t)nrb * xcd / 8) + (int)(blockIdx.x >> 3);
+        step = n;
+        if ((n & 7) == 0) {
+            const int xcd = wg & 7;
+            b = (int)((int64_t)nrb * xcd / 8) + (wg >> 3);
             hi = (int)((int64_t)nrb * (xcd + 1) / 8);
-            step = gridDim.x >> 3;
+            step = n >> 3;
         }
     }
 };
