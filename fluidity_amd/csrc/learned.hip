@@ -275,9 +275,20 @@ k_node_gemm(int n, int d1, int d2, const float* __restrict__ X1, const float* __
     }
 }
 
+// Sums over the nodes (weight, bias and feature gradients) go through
+// per-block partial sums: about kSumBlocks blocks of consecutive nodes, then
+// k_part_sum.  Each block's share is short (96 nodes at 97k), because such a
+// sum is a serial chain: with 4096 nodes a block and one thread adding a
+// column's blocks, these sums were 16 of the 17 ms of a gradient (97k nodes,
+// 1.4M entries); now 0.3 ms, and a gradient 17.4 -> 0.89 ms.
+constexpr int kSumBlocks = 1024;
+
+static int sum_chunk(int n) { return std::max(64, ((n + kSumBlocks - 1) / kSumBlocks + 15) & ~15); }
+
 // MFMA weight gradient: part[blk][o][k] = sum_{n in chunk} dY[n][o] X[n][k]
-// with X = [X1 | X2] (K cols), O = dout.  One block per node chunk; every
-// wave of the block owns a (o,k) tile and walks the chunk.
+// with X = [X1 | X2] (K cols), O = dout.  One block per node chunk; each of
+// its waves owns a (o,k) tile and walks the chunk, the loads of a step
+// unconditional (nodes past the chunk re-read its last one and count 0).
 __global__ void __launch_bounds__(256)
 k_wgrad(int n, int chunk, int d1, int d2, const float* __restrict__ X1, const float* __restrict__ X2,
         int dout, const float* __restrict__ dY, float* __restrict__ part) {
@@ -288,21 +299,25 @@ k_wgrad(int n, int chunk, int d1, int d2, const float* __restrict__ X1, const fl
     const int nb0 = blockIdx.x * chunk, nb1 = min(nb0 + chunk, n);
     const int row = lane & 31, kg = lane >> 5;
     for (int tile = wave; tile < ntile; tile += nw) {
-        const int o0 = (tile / ktiles) * 32, k0 = (tile % ktiles) * 32;
+        const int o0 = (tile / ktiles) * 32, k0 = (tile % ktiles) * 32, k = k0 + row;
+        const float* xb = k < d1 ? X1 + k : X2 + (k - d1);
+        const int xs = k < d1 ? d1 : d2;
         f32x16 acc = {};
+#pragma unroll 2
         for (int s = nb0; s < nb1; s += 16) {
+            float av[8], bv[8];
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                const int nn = min(s + 8 * kg + t, nb1 - 1);
+                av[t] = dY[(size_t)nn * dout + o0 + row];
+                bv[t] = xb[(size_t)nn * xs];
+            }
             bf16x8 a, b;
 #pragma unroll
             for (int t = 0; t < 8; t++) {
-                const int nn = s + 8 * kg + t;
-                float av = 0.f, bv = 0.f;
-                if (nn < nb1) {
-                    av = dY[(size_t)nn * dout + o0 + row];
-                    const int k = k0 + row;
-                    bv = k < d1 ? X1[(size_t)nn * d1 + k] : X2[(size_t)nn * d2 + (k - d1)];
-                }
-                a[t] = (__bf16)av;
-                b[t] = (__bf16)bv;
+                const bool in = s + 8 * kg + t < nb1;
+                a[t] = (__bf16)(in ? av[t] : 0.f);
+                b[t] = (__bf16)(in ? bv[t] : 0.f);
             }
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
         }
@@ -315,23 +330,25 @@ k_wgrad(int n, int chunk, int d1, int d2, const float* __restrict__ X1, const fl
     }
 }
 
-// g[e] += sum_blk part[blk][e]  (fixed order)
-__global__ void k_wgrad_reduce(int nblk, int nel, const float* __restrict__ part, float* __restrict__ g) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nel) return;
+// g[e] += sum_blk part[blk][e] for e < nel: a block takes 64 columns, its
+// wave r the partial sums r, r + 16, ..., and the waves' sums are added in
+// order (fixed partition and order).
+__global__ void __launch_bounds__(1024)
+k_part_sum(int nblk, int nel, const float* __restrict__ part, float* __restrict__ g) {
+    __shared__ float sh[16][64];
+    const int lane = threadIdx.x & 63, r = threadIdx.x >> 6, e = blockIdx.x * 64 + lane;
     float s = 0.f;
-    for (int b = 0; b < nblk; b++) s += part[(size_t)b * nel + e];
-    g[e] += s;
-}
-
-// column sums: g[o] += sum_n dY[n][o]  (fixed chunks, then fixed order)
-__global__ void k_colsum(int n, int dout, int chunk, const float* __restrict__ dY, float* __restrict__ part) {
-    const int o = threadIdx.x;
-    if (o >= dout) return;
-    const int n0 = blockIdx.x * chunk, n1 = min(n0 + chunk, n);
-    float s = 0.f;
-    for (int i = n0; i < n1; i++) s += dY[(size_t)i * dout + o];
-    part[(size_t)blockIdx.x * dout + o] = s;
+    if (e < nel) {
+#pragma unroll 8
+        for (int b = r; b < nblk; b += 16) s += part[(size_t)b * nel + e];
+    }
+    sh[r][lane] = s;
+    __syncthreads();
+    if (r == 0 && e < nel) {
+#pragma unroll
+        for (int q = 1; q < 16; q++) s += sh[q][lane];
+        g[e] += s;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -677,29 +694,34 @@ k_loss_fin(int nparts, float scale, const double* __restrict__ partials, double*
     if (threadIdx.x == 0) lossout[0] = v[0] * (double)scale;
 }
 
-// dGs per stored lower/diagonal entry -> dphi (lower), dpsi (diag)
+// dGs per stored lower/diagonal entry -> dphi (lower), dpsi (diag); 8 lanes
+// a row, an entry each (69 -> 19 us for 97k rows against a thread a row)
 __global__ void __launch_bounds__(256)
 k_dgs(int n, int P, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
       const int32_t* __restrict__ diag, const float* __restrict__ sval, const float* __restrict__ dsq,
       const float* __restrict__ gv, const float* __restrict__ u, const float* __restrict__ v,
       const float* __restrict__ dv, const float* __restrict__ dw, float* __restrict__ dphi,
       float* __restrict__ dpsi) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t >> 3;
     if (i >= n) return;
-    for (int k = rowptr[i]; k <= diag[i]; k++) {
+    const int d = diag[i], ke = rowptr[i + 1];
+    for (int k = rowptr[i] + (t & 7); k < ke; k += 8) {
+        if (k > d) {
+            dphi[k] = 0.f;
+            continue;
+        }
         const int j = col[k];
         float s = 0.f;
         for (int p = 0; p < P; p++)
             s += dv[(size_t)i * P + p] * u[(size_t)j * P + p] + dw[(size_t)j * P + p] * v[(size_t)i * P + p];
         const float dg = s * dsq[j];
-        if (j < i) {
+        if (k < d) {
             dphi[k] = dg * sval[k];
         } else {
             dphi[k] = 0.f;
             dpsi[i] = dg * (gv[k] / dsq[i]);  // dGs_ii * Gs_ii
         }
     }
-    for (int k = diag[i] + 1; k < rowptr[i + 1]; k++) dphi[k] = 0.f;
 }
 
 // per node: dalpha (row sum of dphi), dbeta (column sum via tmap), and the
@@ -746,45 +768,98 @@ k_out_back_fin(int nparts, const double* __restrict__ partials, float* __restric
     }
 }
 
-// dU = dh_out * [Upre > 0]
-__global__ void k_relu_back(int nt, const float* __restrict__ dho, const float* __restrict__ Upre,
-                            float* __restrict__ dU) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < nt) dU[t] = Upre[t] > 0.f ? dho[t] : 0.f;
+// dU = dh_out * [Upre > 0], and its column sums over the block's nodes
+// (256 threads: 8 nodes at a time, a thread keeps one of the 32 columns)
+__global__ void __launch_bounds__(256)
+k_relu_back(int n, int chunk, const float* __restrict__ dho, const float* __restrict__ Upre,
+            float* __restrict__ dU, float* __restrict__ part) {
+    __shared__ float sh[256];
+    const int c = threadIdx.x & 31, n0 = blockIdx.x * chunk, n1 = min(n0 + chunk, n);
+    float s = 0.f;
+#pragma unroll 4
+    for (int i = n0 + (int)(threadIdx.x >> 5); i < n1; i += 8) {
+        const size_t t = (size_t)i * H + c;
+        const float d = Upre[t] > 0.f ? dho[t] : 0.f;
+        dU[t] = d;
+        s += d;
+    }
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    if (threadIdx.x < 32) {
+#pragma unroll
+        for (int q = 1; q < 8; q++) s += sh[threadIdx.x + 32 * q];
+        part[(size_t)blockIdx.x * H + threadIdx.x] = s;
+    }
 }
 
 // edge backward: dP_i = sum_j dr_ij, dQ_j = sum_i dr_ij (gathered over the
-// neighbours of j), with dr_ij = dM_i [r_ij > 0]; partials of dc1, dc2, dbm
+// neighbours of j), with dr_ij = dM_i [r_ij > 0]; partials of dc1, dc2, dbm.
+// Half a wave per row (lane = channel), a block takes rows_per consecutive
+// rows (XCD-contiguous, so the rows' gathers meet in one L2).  The row's
+// columns, values and transposed values are read once, coalesced, and handed
+// to the lanes with shuffles, so the three gathers of U edges are in flight
+// together (L2-bound: 3 x 128 B an edge; 97k rows, 1.4M entries: 144 us with
+// an edge at a time and a block per 8 rows, 62 us so).
 __global__ void __launch_bounds__(256)
-k_edge_back(int n, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
+k_edge_back(int n, int rows_per, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
             const int32_t* __restrict__ tmap, const float* __restrict__ sval, const float* __restrict__ PQ,
             const float* __restrict__ lp, const float* __restrict__ dM, float* __restrict__ dPQ,
-            float* __restrict__ part3, int chunk_rows) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = t >> 5, c = t & 31;
+            float* __restrict__ part3) {
+    const int per = (int)((gridDim.x + 7) >> 3);
+    const int blk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    const int c = threadIdx.x & 31;
     const float c1 = lp[Lay::C1 + c], c2 = lp[Lay::C2 + c], bm = lp[Lay::BM + c];
-    float dp = 0.f, dq = 0.f, g1 = 0.f, g2 = 0.f, gb = 0.f;
-    if (i < n) {
+    float g1 = 0.f, g2 = 0.f, gb = 0.f;
+    constexpr int U = 8;
+    const int r1 = min((blk + 1) * rows_per, n);
+    for (int i = blk * rows_per + (int)(threadIdx.x >> 5); i < r1; i += 8) {
         const float pi = PQ[(size_t)i * 2 * H + c];
         const float qi = PQ[(size_t)i * 2 * H + H + c];
         const float dmi = dM[(size_t)i * H + c];
-        for (int k = rowptr[i]; k < rowptr[i + 1]; k++) {
-            const int j = col[k];
-            if (j == i) continue;
-            const float s = sval[k];
-            // edge (i <- j): contributes to dP_i
-            const float qj = PQ[(size_t)j * 2 * H + H + c];
-            if (pi + qj + c1 * s + c2 * fabsf(s) + bm > 0.f) {
-                dp += dmi;
-                g1 += dmi * s;
-                g2 += dmi * fabsf(s);
-                gb += dmi;
+        const int kb = rowptr[i], ke = rowptr[i + 1];
+        float dp = 0.f, dq = 0.f;
+        for (int k0 = kb; k0 < ke; k0 += 32) {
+            const int len = min(32, ke - k0);
+            int myj = i, myt = -1;
+            float mys = 0.f;
+            if (c < len) {
+                myj = col[k0 + c];
+                mys = sval[k0 + c];
+                myt = tmap[k0 + c];
             }
-            // edge (j <- i): Q_i enters row j's message with s_ji
-            const int kt = tmap[k];
-            const float sj = kt >= 0 ? sval[kt] : 0.f;
-            const float pj = PQ[(size_t)j * 2 * H + c];
-            if (kt >= 0 && pj + qi + c1 * sj + c2 * fabsf(sj) + bm > 0.f) dq += dM[(size_t)j * H + c];
+            const float myts = myt >= 0 ? sval[myt] : 0.f;  // s_ji
+            for (int t0 = 0; t0 < len; t0 += U) {
+                int jj[U], tt[U];
+                float sv[U], st[U], qj[U], pj[U], dm[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int t = min(t0 + u, len - 1);
+                    jj[u] = __shfl(myj, t, 32);
+                    tt[u] = __shfl(myt, t, 32);
+                    sv[u] = __shfl(mys, t, 32);
+                    st[u] = __shfl(myts, t, 32);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    pj[u] = PQ[(size_t)jj[u] * 2 * H + c];
+                    qj[u] = PQ[(size_t)jj[u] * 2 * H + H + c];
+                    dm[u] = dM[(size_t)jj[u] * H + c];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const bool in = t0 + u < len && jj[u] != i;
+                    const float s = sv[u];
+                    // edge (i <- j): contributes to dP_i
+                    if (in && pi + qj[u] + c1 * s + c2 * fabsf(s) + bm > 0.f) {
+                        dp += dmi;
+                        g1 += dmi * s;
+                        g2 += dmi * fabsf(s);
+                        gb += dmi;
+                    }
+                    // edge (j <- i): Q_i enters row j's message with s_ji
+                    if (in && tt[u] >= 0 && pj[u] + qi + c1 * st[u] + c2 * fabsf(st[u]) + bm > 0.f) dq += dm[u];
+                }
+            }
         }
         dPQ[(size_t)i * 2 * H + c] = dp;
         dPQ[(size_t)i * 2 * H + H + c] = dq;
@@ -795,26 +870,13 @@ k_edge_back(int n, const int32_t* __restrict__ rowptr, const int32_t* __restrict
     sh[1][threadIdx.x] = g2;
     sh[2][threadIdx.x] = gb;
     __syncthreads();
-    if (threadIdx.x < 32) {
-        float a = 0.f, b = 0.f, d = 0.f;
-        for (int q = threadIdx.x; q < (int)blockDim.x; q += 32) {
-            a += sh[0][q];
-            b += sh[1][q];
-            d += sh[2][q];
-        }
-        part3[((size_t)blockIdx.x * 3 + 0) * H + threadIdx.x] = a;
-        part3[((size_t)blockIdx.x * 3 + 1) * H + threadIdx.x] = b;
-        part3[((size_t)blockIdx.x * 3 + 2) * H + threadIdx.x] = d;
+    if (threadIdx.x < 3 * H) {
+        const int q = threadIdx.x / H;
+        float a = 0.f;
+#pragma unroll
+        for (int r = 0; r < 8; r++) a += sh[q][r * H + c];
+        part3[(size_t)blockIdx.x * 3 * H + threadIdx.x] = a;  // C1, C2, BM are consecutive
     }
-    (void)chunk_rows;
-}
-
-__global__ void k_part3_reduce(int nblk, const float* __restrict__ part3, float* __restrict__ g) {
-    const int e = threadIdx.x;  // 0..3H-1
-    if (e >= 3 * H) return;
-    float s = 0.f;
-    for (int b = 0; b < nblk; b++) s += part3[(size_t)b * 3 * H + e];
-    g[e] += s;  // layout C1, C2, BM are consecutive
 }
 
 // dh_in += dA (N x H) + dB (N x H) elementwise helper: y += x
@@ -837,31 +899,27 @@ __global__ void k_adam(int np, float lr, float b1, float b2, float eps, float bc
 }
 
 
-// output-layer weight gradients, per node chunk: part[chunk][q][c] for
-// q = 0 (w_a), 1 (w_b), 2 (w_d); part[chunk][3][0] = sum dpsi (b_d)
-__global__ void k_outgrad(int n, int chunk, const float* __restrict__ dab, const float* __restrict__ h,
-                          float* __restrict__ part) {
-    const int t = threadIdx.x;  // 0 .. 4H-1
+// output-layer gradients, per node chunk, in the parameters' order from WOA
+// on: w_a, w_b, w_d (each summed over the chunk's nodes), then 0 for gamma1,
+// gamma2 and b_o (k_out_back_fin has them), and b_d = sum of dpsi.  128
+// threads: 3 x 32 columns, then one for b_d.
+constexpr int kOutCols = Lay::TOTAL - Lay::WOA;
+
+__global__ void __launch_bounds__(128)
+k_outgrad(int n, int chunk, const float* __restrict__ dab, const float* __restrict__ h, float* __restrict__ part) {
+    const int t = threadIdx.x;
+    if (t >= kOutCols) return;
     const int q = t / H, cc = t % H;
     const int n0 = blockIdx.x * chunk, n1 = min(n0 + chunk, n);
     float s = 0.f;
     if (q < 3) {
+#pragma unroll 8
         for (int i = n0; i < n1; i++) s += dab[3 * (size_t)i + q] * h[(size_t)i * H + cc];
-    } else if (cc == 0) {
+    } else if (t == kOutCols - 1) {
+#pragma unroll 8
         for (int i = n0; i < n1; i++) s += dab[3 * (size_t)i + 2];
     }
-    part[(size_t)blockIdx.x * 4 * H + t] = s;
-}
-
-__global__ void k_outgrad_reduce(int nchunk, const float* __restrict__ part, float* __restrict__ g) {
-    const int t = threadIdx.x;
-    float s = 0.f;
-    for (int b = 0; b < nchunk; b++) s += part[(size_t)b * 4 * H + t];
-    const int q = t / H, cc = t % H;
-    if (q == 0) g[Lay::WOA + cc] += s;
-    else if (q == 1) g[Lay::WOB + cc] += s;
-    else if (q == 2) g[Lay::WD + cc] += s;
-    else if (cc == 0) g[Lay::BD] += s;
+    part[(size_t)blockIdx.x * kOutCols + t] = s;
 }
 
 // dh += dHM[:, :H]; dM = dHM[:, H:]
@@ -873,24 +931,18 @@ __global__ void k_split_dm(int n, const float* __restrict__ dHM, float* __restri
     dM[t] = dHM[(size_t)i * 2 * H + H + cc];
 }
 
-// input layer: part[chunk][c][f] = sum dh0[n][c] feat[n][f], f = NFEAT -> bias
-__global__ void k_ingrad(int n, int chunk, const float* __restrict__ dh, const float* __restrict__ feat,
-                         float* __restrict__ part) {
+// input layer, per node chunk, in the parameters' order: W_IN[c][f] = sum
+// dh0[n][c] feat[n][f], then B_IN[c] = sum dh0[n][c]
+__global__ void __launch_bounds__(H * (NFEAT + 1))
+k_ingrad(int n, int chunk, const float* __restrict__ dh, const float* __restrict__ feat, float* __restrict__ part) {
     const int t = threadIdx.x;  // 0 .. H*(NFEAT+1)-1
-    const int cc = t / (NFEAT + 1), f = t % (NFEAT + 1);
+    const bool bias = t >= H * NFEAT;
+    const int cc = bias ? t - H * NFEAT : t / NFEAT, f = bias ? 0 : t % NFEAT;
     const int n0 = blockIdx.x * chunk, n1 = min(n0 + chunk, n);
     float s = 0.f;
-    for (int i = n0; i < n1; i++) s += dh[(size_t)i * H + cc] * (f < NFEAT ? feat[(size_t)i * NFEAT + f] : 1.f);
+#pragma unroll 8
+    for (int i = n0; i < n1; i++) s += dh[(size_t)i * H + cc] * (bias ? 1.f : feat[(size_t)i * NFEAT + f]);
     part[(size_t)blockIdx.x * H * (NFEAT + 1) + t] = s;
-}
-
-__global__ void k_ingrad_reduce(int nchunk, const float* __restrict__ part, float* __restrict__ g) {
-    const int t = threadIdx.x;
-    float s = 0.f;
-    for (int b = 0; b < nchunk; b++) s += part[(size_t)b * H * (NFEAT + 1) + t];
-    const int cc = t / (NFEAT + 1), f = t % (NFEAT + 1);
-    if (f < NFEAT) g[Lay::W_IN + cc * NFEAT + f] += s;
-    else g[Lay::B_IN + cc] += s;
 }
 
 // ---------------------------------------------------------------------------
@@ -1344,24 +1396,28 @@ static int loss_grad(flgpu_ctx* c, int P, uint64_t seed, double* loss_out) {
     // dv = G dw
     hipLaunchKernelGGL((k_batch_spmv<float>), dim3(gnp), dim3(256), 0, c->stream, n, P, c->rowptr.p, c->col.p,
                        c->diag.p, (const float*)s->gv.p, (const float*)s->dw.p, s->dv.p, 1);
-    hipLaunchKernelGGL(k_dgs, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, n, P, c->rowptr.p, c->col.p, c->diag.p,
+    hipLaunchKernelGGL(k_dgs, dim3(grid_for((int64_t)n * 8, 256)), dim3(256), 0, c->stream, n, P, c->rowptr.p, c->col.p, c->diag.p,
                        s->sval.p, s->dsq.p, s->gv.p, s->u.p, s->v.p, s->dv.p, s->dw.p, s->dphi.p, s->dpsi.p);
     const int ogrid = (int)std::min<int64_t>(kMaxVecGrid, grid_for(n, kVecBlock));
     hipLaunchKernelGGL(k_out_back, dim3(ogrid), dim3(kVecBlock), 0, c->stream, n, c->rowptr.p, c->col.p, c->diag.p,
                        s->tmap.p, s->sval.p, s->dphi.p, s->dpsi.p, s->theta.p, s->dab.p, s->dh.p, s->lpart.p);
     hipLaunchKernelGGL(k_out_back_fin, dim3(1), dim3(kVecBlock), 0, c->stream, ogrid, s->lpart.p, s->grad.p);
     // output-layer weights: grad[WOA/WOB/WD][c] = sum_n dab[n][q] h_L[n][c], b_d = sum dpsi
-    const int chunk = 4096;
+    const int chunk = sum_chunk(n);
     const int nchunk = (n + chunk - 1) / chunk;
-    FLGPU_TRY(s->wpart.alloc((size_t)nchunk * 2 * H * 2 * H));
+    // edge blocks: rows in runs of 8, a multiple of 8 blocks for the XCD mapping
+    const int rows_per = std::max(8, ((n + 2047) / 2048 + 7) & ~7);
+    const int eblk = (((n + rows_per - 1) / rows_per) + 7) & ~7;
+    FLGPU_TRY(s->wpart.reserve(std::max((size_t)nchunk * 2 * H * H, (size_t)eblk * 3 * H)));
+    auto part_sum = [&](int nblk, int nel, float* g) {
+        hipLaunchKernelGGL(k_part_sum, dim3((nel + 63) / 64), dim3(1024), 0, c->stream, nblk, nel,
+                           (const float*)s->wpart.p, g);
+    };
     const float* hL = s->h.p + (size_t)NLAYER * n * H;
-    hipLaunchKernelGGL(k_outgrad, dim3(nchunk), dim3(4 * H), 0, c->stream, n, chunk, s->dab.p, hL, s->wpart.p);
-    hipLaunchKernelGGL(k_outgrad_reduce, dim3(1), dim3(4 * H), 0, c->stream, nchunk, s->wpart.p, s->grad.p);
+    hipLaunchKernelGGL(k_outgrad, dim3(nchunk), dim3(128), 0, c->stream, n, chunk, s->dab.p, hL, s->wpart.p);
+    part_sum(nchunk, kOutCols, s->grad.p + Lay::WOA);
     // hidden layers, last to first
     FLGPU_TRY(s->dM.alloc((size_t)n * H));  // scratch for dh_in assembly
-    const int eblk = (int)grid_for((int64_t)n * 32, 256);
-    DevBuf<float> part3;
-    FLGPU_TRY(part3.alloc((size_t)eblk * 3 * H));
     for (int l = NLAYER - 1; l >= 0; l--) {
         const float* hin = s->h.p + (size_t)l * n * H;
         const float* PQ = s->PQ.p + (size_t)l * n * 2 * H;
@@ -1371,16 +1427,14 @@ static int loss_grad(flgpu_ctx* c, int P, uint64_t seed, double* loss_out) {
         const float* lp = s->theta.p + Lay::layer(l);
         float* gl = s->grad.p + Lay::layer(l);
         const int nt = n * H;
-        hipLaunchKernelGGL(k_relu_back, dim3(grid_for(nt, 256)), dim3(256), 0, c->stream, nt, s->dh.p, U, s->dU.p);
-        // Wu, b_u
-        hipLaunchKernelGGL(k_wgrad, dim3(nchunk), dim3(256), 0, c->stream, n, chunk, H, H, hin, M, H,
+        // dU and b_u
+        hipLaunchKernelGGL(k_relu_back, dim3(nchunk), dim3(256), 0, c->stream, n, chunk, (const float*)s->dh.p, U,
+                           s->dU.p, s->wpart.p);
+        part_sum(nchunk, H, gl + Lay::BU);
+        // Wu: two 32 x 32 tiles, a wave each
+        hipLaunchKernelGGL(k_wgrad, dim3(nchunk), dim3(128), 0, c->stream, n, chunk, H, H, hin, M, H,
                            (const float*)s->dU.p, s->wpart.p);
-        hipLaunchKernelGGL(k_wgrad_reduce, dim3(grid_for(H * 2 * H, 256)), dim3(256), 0, c->stream, nchunk,
-                           H * 2 * H, (const float*)s->wpart.p, gl + Lay::WU);
-        hipLaunchKernelGGL(k_colsum, dim3(nchunk), dim3(64), 0, c->stream, n, H, chunk, (const float*)s->dU.p,
-                           s->wpart.p);
-        hipLaunchKernelGGL(k_wgrad_reduce, dim3(1), dim3(H), 0, c->stream, nchunk, H, (const float*)s->wpart.p,
-                           gl + Lay::BU);
+        part_sum(nchunk, H * 2 * H, gl + Lay::WU);
         // [dh_direct | dM] = dU Wu
         hipLaunchKernelGGL((k_node_gemm<0>), dim3(gemm_grid(n, 2 * H)), dim3(256), 0, c->stream, n, H, 0,
                            (const float*)s->dU.p, (const float*)nullptr, 2 * H, wl + 2 * H * H + H * 2 * H,
@@ -1388,15 +1442,13 @@ static int loss_grad(flgpu_ctx* c, int P, uint64_t seed, double* loss_out) {
         hipLaunchKernelGGL(k_split_dm, dim3(grid_for(nt, 256)), dim3(256), 0, c->stream, n, (const float*)s->dHM.p,
                            s->dh.p, s->dM.p);
         // edge backward -> dP, dQ and (c1, c2, bm) gradients
-        hipLaunchKernelGGL(k_edge_back, dim3(eblk), dim3(256), 0, c->stream, n, c->rowptr.p, c->col.p, s->tmap.p,
-                           s->sval.p, PQ, lp, (const float*)s->dM.p, s->dPQ.p, part3.p, 0);
-        hipLaunchKernelGGL(k_part3_reduce, dim3(1), dim3(3 * H), 0, c->stream, eblk, (const float*)part3.p,
-                           gl + Lay::C1);
+        hipLaunchKernelGGL(k_edge_back, dim3(eblk), dim3(256), 0, c->stream, n, rows_per, c->rowptr.p, c->col.p,
+                           s->tmap.p, s->sval.p, PQ, lp, (const float*)s->dM.p, s->dPQ.p, s->wpart.p);
+        part_sum(eblk, 3 * H, gl + Lay::C1);
         // [Wa; Wb]
-        hipLaunchKernelGGL(k_wgrad, dim3(nchunk), dim3(256), 0, c->stream, n, chunk, H, 0, hin,
+        hipLaunchKernelGGL(k_wgrad, dim3(nchunk), dim3(128), 0, c->stream, n, chunk, H, 0, hin,
                            (const float*)nullptr, 2 * H, (const float*)s->dPQ.p, s->wpart.p);
-        hipLaunchKernelGGL(k_wgrad_reduce, dim3(grid_for(2 * H * H, 256)), dim3(256), 0, c->stream, nchunk,
-                           2 * H * H, (const float*)s->wpart.p, gl + Lay::WA);
+        part_sum(nchunk, 2 * H * H, gl + Lay::WA);
         // dh_in += dP Wa + dQ Wb
         hipLaunchKernelGGL((k_node_gemm<0>), dim3(gemm_grid(n, H)), dim3(256), 0, c->stream, n, 2 * H, 0,
                            (const float*)s->dPQ.p, (const float*)nullptr, H, wl + 2 * H * H + H * 2 * H + 2 * H * H,
@@ -1407,8 +1459,7 @@ static int loss_grad(flgpu_ctx* c, int P, uint64_t seed, double* loss_out) {
     // input layer
     hipLaunchKernelGGL(k_ingrad, dim3(nchunk), dim3(H * (NFEAT + 1)), 0, c->stream, n, chunk, (const float*)s->dh.p,
                        (const float*)s->feat.p, s->wpart.p);
-    hipLaunchKernelGGL(k_ingrad_reduce, dim3(1), dim3(H * (NFEAT + 1)), 0, c->stream, nchunk,
-                       (const float*)s->wpart.p, s->grad.p);
+    part_sum(nchunk, H * (NFEAT + 1), s->grad.p);
     FLGPU_HIP(hipGetLastError());
     if (loss_out) {
         FLGPU_HIP(hipMemcpyAsync(loss_out, s->lossbuf.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
