@@ -56,7 +56,7 @@ struct KrylovWork {
     bool use_sell = false, sell16 = false;
     int nsl = 0;
     int64_t nslot = 0;
-    DevBuf<int32_t> sptr, ssrc, scol32;
+    DevBuf<int32_t> sptr, ssrc, scol32, srows;
     DevBuf<int16_t> scol16;
     DevBuf<double> sval64;
     DevBuf<float> sval32;
@@ -733,7 +733,7 @@ static const float* sell_values(const KrylovWork* k, const float* val) {
 template <typename V, typename CT, typename XV, typename YV>
 static void sell_launch(flgpu_ctx* c, KrylovWork* k, const V* sval, const CT* col, const XV* x, YV* y,
                         const double* bsub, int want_dot, const int* done_flag) {
-    const SellOp<V, CT> m{k->nsl, c->rows, k->sptr.p, c->rowptr.p, col, sval, nullptr};
+    const SellOp<V, CT> m{k->nsl, c->rows, k->sptr.p, c->rowptr.p, col, sval, nullptr, k->srows.p};
     const int grid = sell_grid(k->nsl);
     if (want_dot)
         hipLaunchKernelGGL((k_sell<V, V, CT, XV, YV, DOT_XY>), dim3(grid), dim3(kRowBlock), 0, c->stream, m, x, y,
@@ -780,9 +780,9 @@ static int spmv(flgpu_ctx* c, KrylovWork* k, const V* val, const XV* x, YV* y, c
     return FLGPU_OK;
 }
 
-// The sliced ELL plan of the solver matrix, kept when its padding is at
-// most kSellMaxFill times the entries (FLGPU_SPMV=csr keeps the CSR
-// stream product throughout).
+// The sliced ELL plan of the solver matrix, rows in order when that pads to
+// at most kSellMaxFill times the entries, else sorted by length in windows
+// when that does (FLGPU_SPMV=csr keeps the CSR stream product throughout).
 constexpr double kSellMaxFill = 1.2;
 
 static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
@@ -790,14 +790,21 @@ static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
     k->use_sell = false;
     k->sptr.release();
     k->ssrc.release();
+    k->srows.release();
     k->scol16.release();
     k->scol32.release();
     k->sval64.release();
     k->sval32.release();
     if (e && std::string(e) == "csr") return FLGPU_OK;
+    const int32_t* rp = c->h_rowptr.data();
+    int window = 0;
+    if (sell_fill(rp, c->rows, 0) > kSellMaxFill) {
+        window = kSellWindow;
+        if (sell_fill(rp, c->rows, window) > kSellMaxFill) return FLGPU_OK;
+    }
     SellHost h;
-    sell_plan(c->h_rowptr.data(), c->h_col.data(), c->rows, nullptr, h);
-    if (h.fill(c->nnz) > kSellMaxFill) return FLGPU_OK;
+    sell_plan(rp, c->h_col.data(), c->rows, nullptr, h, window);
+    if (window) FLGPU_TRY(k->srows.upload(h.rows.data(), h.rows.size(), c->stream));
     FLGPU_TRY(k->sptr.upload(h.sptr.data(), h.sptr.size(), c->stream));
     FLGPU_TRY(k->ssrc.upload(h.src.data(), h.src.size(), c->stream));
     if (h.use16) FLGPU_TRY(k->scol16.upload(h.c16.data(), h.c16.size(), c->stream));
@@ -1655,7 +1662,8 @@ k_gm_sell(SellOp<V, CT> m, const V* __restrict__ w, V* __restrict__ v, V* __rest
     for (int g = it.b; g < it.hi; g += it.step) {
         const int sl = g * WPB + wave;
         if (sl >= m.nsl) continue;
-        const int r0 = sl * kSlice, row = r0 + lane;
+        int r0;
+        const int row = sell_row(m, sl, lane, r0);
         const int base = m.sptr[sl], wd = (m.sptr[sl + 1] - base) / kSlice;
         const int rc = min(row, m.n - 1), len = row < m.n ? m.rowptr[rc + 1] - m.rowptr[rc] : 0;
         const V wi = w[rc], di = dinv ? dinv[rc] : (V)1;
@@ -2097,11 +2105,11 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
         if (sval) {
             const int grid = sell_grid(k->nsl);
             if (k->sell16) {
-                const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol16.p, sval, nullptr};
+                const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol16.p, sval, nullptr, k->srows.p};
                 hipLaunchKernelGGL((k_gm_sell<V, int16_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
                                    d);
             } else {
-                const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol32.p, sval, nullptr};
+                const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol32.p, sval, nullptr, k->srows.p};
                 hipLaunchKernelGGL((k_gm_sell<V, int32_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
                                    d);
             }

@@ -14,6 +14,8 @@
 // plan, the solve and the pressure path.
 #include <cmath>
 #include <cstdint>
+#include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -371,6 +373,60 @@ static void check_sell(const std::vector<int32_t>& findrm, const std::vector<int
     }
 }
 
+// The same with the rows of a window sorted by length (rows of 3 to 40
+// entries alternating, sizes below, at and past a window): every row in one
+// lane of its own window, every entry in one slot, offsets from the window's
+// first row, padding as sell_fill says, the product bit for bit.
+static void check_sell_sorted(int n) {
+    std::mt19937_64 g(n);
+    std::vector<int32_t> rp(n + 1, 0), cl;
+    for (int i = 0; i < n; i++) {
+        const int len = std::min(n, i % 8 == 0 ? 40 : i % 2 ? 3 : 17);
+        std::vector<int32_t> row;
+        for (int q = 0; q < len; q++) row.push_back((i + q) % n);
+        std::sort(row.begin(), row.end());
+        cl.insert(cl.end(), row.begin(), row.end());
+        rp[i + 1] = (int32_t)cl.size();
+    }
+    std::uniform_real_distribution<double> U(-1.0, 1.0);
+    std::vector<double> val(cl.size()), x(n);
+    for (double& v : val) v = U(g);
+    for (double& v : x) v = U(g);
+    flgpu::SellHost h;
+    flgpu::sell_plan(rp.data(), cl.data(), n, nullptr, h, flgpu::kSellWindow);
+    CHECK((int)h.rows.size() == h.nsl * flgpu::kSlice, "sorted sell rows");
+    CHECK(std::fabs(h.fill((int64_t)cl.size()) - flgpu::sell_fill(rp.data(), n, flgpu::kSellWindow)) < 1e-12,
+          "sorted sell fill");
+    std::vector<int> seen(cl.size(), 0), rows(n, 0);
+    for (int sl = 0; sl < h.nsl; sl++) {
+        const int r0 = sl / (flgpu::kSellWindow / flgpu::kSlice) * flgpu::kSellWindow, base = h.sptr[sl];
+        const int w = (h.sptr[sl + 1] - base) / flgpu::kSlice;
+        for (int lane = 0; lane < flgpu::kSlice; lane++) {
+            const int row = h.rows[sl * flgpu::kSlice + lane], len = row >= 0 ? rp[row + 1] - rp[row] : 0;
+            CHECK(row < n && (row < 0 || (row >= r0 && row < r0 + flgpu::kSellWindow)), "sorted sell row in its window");
+            CHECK(len <= w, "sorted sell row longer than its slice");
+            if (row >= 0) rows[row]++;
+            double acc = 0.0, ref = 0.0;
+            for (int j = 0; j < w; j++) {
+                const int64_t slot = base + (int64_t)j * flgpu::kSlice + lane;
+                const int cj = h.use16 ? r0 + h.c16[slot] : h.c32[slot];
+                CHECK(cj >= 0 && cj < n, "sorted sell column out of range");
+                if (j >= len) {
+                    CHECK(h.src[slot] == -1, "sorted sell padding");
+                    continue;
+                }
+                CHECK(h.src[slot] == rp[row] + j && cj == cl[rp[row] + j], "sorted sell entry");
+                seen[rp[row] + j]++;
+                acc += val[h.src[slot]] * x[cj];
+                ref += val[rp[row] + j] * x[cl[rp[row] + j]];
+            }
+            CHECK(acc == ref, "sorted sell product");
+        }
+    }
+    for (int v : seen) CHECK(v == 1, "sorted sell entry in %d slots", v);
+    for (int v : rows) CHECK(v == 1, "sorted sell row in %d lanes", v);
+}
+
 int main(int argc, char** argv) {
     const bool gpu = argc > 1 && std::strcmp(argv[1], "--gpu") == 0;
     const Mesh m = kuhn_cube(gpu ? 12 : 6);
@@ -394,6 +450,7 @@ int main(int argc, char** argv) {
     std::printf("host: %d nodes, %d elements, %lld entries, %d colours\n", m.nx, m.nele, (long long)nnz, ncol);
     check_matrixdump(findrm, colm);
     check_sell(findrm, colm);
+    for (int n : {1, 63, 64, 511, 512, 513, 1000, 1537}) check_sell_sorted(n);
     check_oracle(m, findrm, colm, centrm);
     if (gpu) check_gpu(m, findrm, colm, centrm);
     std::printf("%s\n", failures ? "FAILED" : "host_check ok");
