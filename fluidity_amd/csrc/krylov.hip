@@ -65,10 +65,20 @@ struct KrylovWork {
     int nblk = 1;
     Scal* S() { return scal.p + cur; }
     double* part(int region) { return partials.p + (size_t)region * kPartStride; }
-    // multicolour SSOR: rows grouped by colour (ascending inside a colour)
-    DevBuf<int32_t> mc_rows;
-    std::vector<int32_t> mc_ptr;  // colour c owns mc_rows[mc_ptr[c] .. mc_ptr[c+1])
+    // multicolour SSOR: the rows of a colour in slices of 64 (one wave), their
+    // off-diagonal entries in slots as in a sliced ELL matrix -- those in
+    // earlier colours for the forward sweep (f), all of them for the backward (b)
+    struct SorHalf {
+        DevBuf<int32_t> ptr, len, col, src;
+        DevBuf<double> v64;
+        DevBuf<float> v32;
+    } mc_f, mc_b;
+    DevBuf<int32_t> mc_rows, mc_dsrc, mc_cptr;
+    DevBuf<double> mc_d64;
+    DevBuf<float> mc_d32;
+    std::vector<int32_t> mc_ptr;  // colour c owns slices mc_ptr[c] .. mc_ptr[c+1]
     int64_t mc_key = -1;          // sparsity generation of the colouring
+    bool mc_one = false;          // a sweep by one workgroup
     // GMRES
     DevBuf<double> V, gm_work;  // basis; block sums, Hessenberg column, rotations
     DevBuf<float> V32;
@@ -653,38 +663,123 @@ k_finish_x(int n, double* __restrict__ x, const double* __restrict__ rhs,
 // colouring of the matrix graph in row order (rows of one colour share no
 // entry, so a colour's rows update independently): the same sweep on the
 // symmetrically permuted matrix, again symmetric positive definite for an
-// SPD system, one launch per colour.
+// SPD system.
 //   forward:  z = 0; for c = 0 .. C-1:  z_i = (r_i - sum_{j != i} a_ij z_j) / a_ii
 //   backward:        for c = C-2 .. 0:  the same with the current z
-// (the last colour's backward step would recompute its forward values).
-// Each row is summed by one thread in entry order with explicit fused
+// (the last colour's backward step would recompute its forward values; the
+// forward step needs only the entries in earlier colours, the others' z being
+// 0).  Each row is summed by one thread in entry order with explicit fused
 // multiply-adds, the order of the oracle's restatement.
+// What bounds it: the chain of 2C - 1 dependent steps.  A launch per colour
+// (k_sor_slices) takes 4 us with a few thousand rows a colour (12 us reading
+// the CSR rows entry by entry); where z fits LDS and the entries are few, one
+// workgroup takes the whole sweep with a barrier per colour (k_sor_block).
+// An apply on one MI355X: 41 x 41 P2 triangles (6889 rows, 13 colours), 27
+// launches 200 us -> one launch 36 us; 45^3 x 6 P1 tetrahedra (97k rows, 9
+// colours) 205 -> 79 us.  Their time steps with GMRES: 2.42 -> 1.33 ms and
+// 3.0 -> 1.88 ms.
+
+// One sweep direction: slices ptr[sl] .. of 64 rows, len their entries.
+template <typename V>
+struct SorOp {
+    const int32_t *rows, *ptr, *len, *col;
+    const V *val, *dia;
+};
+
+constexpr int kSorBatch = 8;
+
+// What a lane needs before the first z: its row, bounds, and the first
+// batch of its entries (slots past a slice's width re-read its last one).
+template <typename V>
+struct SorLane {
+    int row, len, base, w;
+    V r, d;
+    int cj[kSorBatch];
+    V av[kSorBatch];
+};
 
 template <typename V>
-__global__ void __launch_bounds__(kVecBlock)
-k_fill_done(int n, V* __restrict__ a, const int* __restrict__ done_flag) {
-    if (done_flag && *done_flag) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) a[i] = (V)0;
+__device__ __forceinline__ void sor_batch(const SorOp<V>& m, SorLane<V>& t, int j0, int lane) {
+#pragma unroll
+    for (int u = 0; u < kSorBatch; u++) {
+        const int slot = t.base + min(j0 + u, t.w - 1) * kSlice + lane;
+        t.cj[u] = m.col[slot];
+        t.av[u] = m.val[slot];
+    }
 }
 
 template <typename V>
-__global__ void __launch_bounds__(256)
-k_sor_colour(int nr, const int32_t* __restrict__ rows, const int32_t* __restrict__ rowptr,
-             const int32_t* __restrict__ col, const V* __restrict__ val, const V* __restrict__ r, V* __restrict__ z,
-             const int* __restrict__ done_flag) {
-    if (done_flag && *done_flag) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nr) return;
-    const int i = rows[t];
-    V acc = r[i], aii = (V)0;
-    for (int k = rowptr[i]; k < rowptr[i + 1]; k++) {
-        const int j = col[k];
-        if (j == i)
-            aii = val[k];
-        else
-            acc = fma(-val[k], z[j], acc);
+__device__ __forceinline__ void sor_fetch(const SorOp<V>& m, int sl, int lane, const V* __restrict__ r, SorLane<V>& t) {
+    const int q = sl * kSlice + lane;
+    t.row = m.rows[q];
+    t.len = m.len[q];
+    t.d = m.dia[q];
+    t.base = m.ptr[sl];
+    t.w = (m.ptr[sl + 1] - t.base) / kSlice;
+    if (t.w > 0) sor_batch(m, t, 0, lane);
+    t.r = t.row >= 0 ? r[t.row] : (V)0;
+}
+
+// z of the lane's row from the fetched entries and the current z.
+template <typename V>
+__device__ __forceinline__ V sor_finish(const SorOp<V>& m, SorLane<V>& t, int lane, const V* z) {
+    V acc = t.r;
+    for (int j0 = 0; j0 < t.w; j0 += kSorBatch) {
+        if (j0 > 0) sor_batch(m, t, j0, lane);
+        V zv[kSorBatch];
+#pragma unroll
+        for (int u = 0; u < kSorBatch; u++) zv[u] = z[t.cj[u]];
+#pragma unroll
+        for (int u = 0; u < kSorBatch; u++)
+            if (j0 + u < t.len) acc = fma(-t.av[u], zv[u], acc);
     }
-    z[i] = acc / aii;
+    return acc / t.d;
+}
+
+// A colour's slices s0 .. s1, a wave each.
+template <typename V>
+__global__ void __launch_bounds__(256)
+k_sor_slices(SorOp<V> m, int s0, int s1, const V* __restrict__ r, V* z, const int* __restrict__ done_flag) {
+    if (done_flag && *done_flag) return;
+    const int sl = s0 + (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (sl >= s1) return;
+    SorLane<V> t;
+    sor_fetch(m, sl, lane, r, t);
+    const V zi = sor_finish(m, t, lane, (const V*)z);
+    if (t.row >= 0) z[t.row] = zi;
+}
+
+// Both sweeps by one workgroup, z in LDS: the entries of a wave's first slice
+// of the next colour are fetched before the barrier that ends this one.
+template <typename V>
+__global__ void __launch_bounds__(1024)
+k_sor_block(int n, int ncol, const int32_t* __restrict__ cptr, SorOp<V> f, SorOp<V> b, const V* __restrict__ r,
+            V* __restrict__ z, const int* __restrict__ done_flag) {
+    extern __shared__ double sor_lds[];
+    V* zs = reinterpret_cast<V*>(sor_lds);
+    if (done_flag && *done_flag) return;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6, np = 2 * ncol - 1;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) zs[i] = (V)0;
+    SorLane<V> t;
+    auto colour = [&](int p) { return p < ncol ? p : 2 * ncol - 2 - p; };
+    auto start = [&](int p) {
+        const int q = colour(p), sl = cptr[q] + wave;
+        if (sl < cptr[q + 1]) sor_fetch(p < ncol ? f : b, sl, lane, r, t);
+    };
+    start(0);
+    __syncthreads();
+    for (int p = 0; p < np; p++) {
+        const SorOp<V>& m = p < ncol ? f : b;
+        const int q = colour(p), s1 = cptr[q + 1];
+        for (int sl = cptr[q] + wave; sl < s1; sl += nw) {
+            if (sl != cptr[q] + wave) sor_fetch(m, sl, lane, r, t);
+            const V zi = sor_finish(m, t, lane, zs);
+            if (t.row >= 0) zs[t.row] = zi;
+        }
+        if (p + 1 < np) start(p + 1);
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < n; i += blockDim.x) z[i] = zs[i];
 }
 
 // Per-block sums r.z, z.z, z.w (w may be null: z.w = 0).
@@ -971,39 +1066,141 @@ static void colour_rows(int n, const int32_t* rowptr, const int32_t* col, std::v
     for (int i = 0; i < n; i++) rows[pos[colour[i]]++] = i;
 }
 
-static int ssor_prepare(flgpu_ctx* c, KrylovWork* k) {
-    if (k->mc_key == c->sparsity_gen) return FLGPU_OK;
+// One workgroup takes the sweeps when z fits its LDS and reading the entries
+// through one CU (about 120 GB/s) plus a barrier per step (0.8 us) costs less
+// than a launch per step (4 us).
+constexpr size_t kSorLds = 128 << 10;
+
+static int ssor_plan(flgpu_ctx* c, KrylovWork* k) {
     if (!c->all_diag) return set_error(FLGPU_EUNSUPPORTED, "sor preconditioner: a row has no diagonal entry");
-    std::vector<int32_t> rows;
-    colour_rows(c->rows, c->h_rowptr.data(), c->h_col.data(), k->mc_ptr, rows);
+    const int n = c->rows;
+    const int32_t *rp = c->h_rowptr.data(), *cl = c->h_col.data();
+    std::vector<int32_t> cp, order, colour(n), rows, dsrc, sl_of;
+    colour_rows(n, rp, cl, cp, order);
+    const int ncol = (int)cp.size() - 1;
+    for (int q = 0; q < ncol; q++)
+        for (int t = cp[q]; t < cp[q + 1]; t++) colour[order[t]] = q;
+    // slices: a colour's rows in order, longest first inside windows of kSellWindow
+    k->mc_ptr.assign(1, 0);
+    for (int q = 0; q < ncol; q++) {
+        for (int t = cp[q]; t < cp[q + 1]; t += kSellWindow)
+            std::stable_sort(order.begin() + t, order.begin() + std::min(cp[q + 1], t + kSellWindow),
+                             [&](int32_t a, int32_t b) { return rp[a + 1] - rp[a] > rp[b + 1] - rp[b]; });
+        rows.insert(rows.end(), order.begin() + cp[q], order.begin() + cp[q + 1]);
+        rows.resize((rows.size() + kSlice - 1) / kSlice * kSlice, -1);
+        k->mc_ptr.push_back((int32_t)(rows.size() / kSlice));
+    }
+    const int nsl = (int)(rows.size() / kSlice);
+    dsrc.assign(rows.size(), -1);
+    int64_t slots = 0;
+    for (int half = 0; half < 2; half++) {
+        KrylovWork::SorHalf& H = half ? k->mc_b : k->mc_f;
+        std::vector<int32_t> ptr(nsl + 1, 0), len(rows.size(), 0), col, src;
+        std::vector<std::vector<int32_t>> ent(kSlice);
+        for (int sl = 0; sl < nsl; sl++) {
+            int w = 0;
+            for (int lane = 0; lane < kSlice; lane++) {
+                const int q = sl * kSlice + lane, i = rows[q];
+                ent[lane].clear();
+                if (i < 0) continue;
+                for (int e = rp[i]; e < rp[i + 1]; e++) {
+                    if (cl[e] == i) dsrc[q] = e;
+                    else if (half || colour[cl[e]] < colour[i]) ent[lane].push_back(e);
+                }
+                len[q] = (int32_t)ent[lane].size();
+                w = std::max(w, len[q]);
+            }
+            for (int j = 0; j < w; j++)
+                for (int lane = 0; lane < kSlice; lane++) {
+                    const bool in = j < (int)ent[lane].size();
+                    src.push_back(in ? ent[lane][j] : -1);
+                    col.push_back(in ? cl[ent[lane][j]] : 0);
+                }
+            ptr[sl + 1] = (int32_t)col.size();
+        }
+        slots += (int64_t)col.size();
+        FLGPU_TRY(H.ptr.upload(ptr.data(), ptr.size(), c->stream));
+        FLGPU_TRY(H.len.upload(len.data(), len.size(), c->stream));
+        FLGPU_TRY(H.col.upload(col.data(), col.size(), c->stream));
+        FLGPU_TRY(H.src.upload(src.data(), src.size(), c->stream));
+        FLGPU_HIP(hipStreamSynchronize(c->stream));  // the vectors are freed here
+    }
     FLGPU_TRY(k->mc_rows.upload(rows.data(), rows.size(), c->stream));
-    FLGPU_HIP(hipStreamSynchronize(c->stream));  // rows is freed on return
+    FLGPU_TRY(k->mc_dsrc.upload(dsrc.data(), dsrc.size(), c->stream));
+    FLGPU_TRY(k->mc_cptr.upload(k->mc_ptr.data(), k->mc_ptr.size(), c->stream));
+    FLGPU_HIP(hipStreamSynchronize(c->stream));
+    const double steps = 2.0 * ncol - 1.0;
+    k->mc_one = sizeof(double) * (size_t)n <= kSorLds && 12.0 * (double)slots / 120e3 + 0.8 * steps < 4.0 * steps;
+    if (k->mc_one)
+        for (const void* f : {(const void*)&k_sor_block<double>, (const void*)&k_sor_block<float>})
+            FLGPU_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSorLds));
     k->mc_key = c->sparsity_gen;
+    return FLGPU_OK;
+}
+
+template <typename V>
+static const V* sor_values(KrylovWork::SorHalf& h);
+template <>
+const double* sor_values<double>(KrylovWork::SorHalf& h) { return h.v64.p; }
+template <>
+const float* sor_values<float>(KrylovWork::SorHalf& h) { return h.v32.p; }
+
+// The plan of the sparsity, and the reduced values in its slots.
+template <typename V>
+static int ssor_prepare(flgpu_ctx* c, KrylovWork* k, const V* val) {
+    if (k->mc_key != c->sparsity_gen) FLGPU_TRY(ssor_plan(c, k));
+    auto gather = [&](const DevBuf<int32_t>& src, auto& out) -> int {
+        FLGPU_TRY(out.alloc(src.n));
+        if (src.n)
+            hipLaunchKernelGGL((k_sell_gather<V, V>), dim3(grid_for((int64_t)src.n, 256)), dim3(256), 0, c->stream,
+                               (int64_t)src.n, src.p, val, out.p);
+        return FLGPU_OK;
+    };
+    if constexpr (std::is_same<V, double>::value) {
+        FLGPU_TRY(gather(k->mc_f.src, k->mc_f.v64));
+        FLGPU_TRY(gather(k->mc_b.src, k->mc_b.v64));
+        FLGPU_TRY(gather(k->mc_dsrc, k->mc_d64));
+    } else {
+        FLGPU_TRY(gather(k->mc_f.src, k->mc_f.v32));
+        FLGPU_TRY(gather(k->mc_b.src, k->mc_b.v32));
+        FLGPU_TRY(gather(k->mc_dsrc, k->mc_d32));
+    }
+    FLGPU_HIP(hipGetLastError());
     return FLGPU_OK;
 }
 
 // z = M^-1 r (the forward and backward sweeps); with done_flag set the
 // kernels return at once.
 template <typename V>
-static int ssor_sweeps(flgpu_ctx* c, KrylovWork* k, const V* val, const V* r, V* z, const int* done_flag) {
+static int ssor_sweeps(flgpu_ctx* c, KrylovWork* k, const V* r, V* z, const int* done_flag) {
     const int ncol = (int)k->mc_ptr.size() - 1;
-    hipLaunchKernelGGL((k_fill_done<V>), dim3(k->nblk), dim3(kVecBlock), 0, c->stream, c->rows, z, done_flag);
-    auto sweep = [&](int q) {
-        const int nr = k->mc_ptr[q + 1] - k->mc_ptr[q];
-        if (nr > 0)
-            hipLaunchKernelGGL((k_sor_colour<V>), dim3(grid_for(nr, 256)), dim3(256), 0, c->stream, nr,
-                               k->mc_rows.p + k->mc_ptr[q], c->rowptr.p, c->col.p, val, r, z, done_flag);
+    const V* dia;
+    if constexpr (std::is_same<V, double>::value) dia = k->mc_d64.p;
+    else dia = k->mc_d32.p;
+    const SorOp<V> f{k->mc_rows.p, k->mc_f.ptr.p, k->mc_f.len.p, k->mc_f.col.p, sor_values<V>(k->mc_f), dia};
+    const SorOp<V> b{k->mc_rows.p, k->mc_b.ptr.p, k->mc_b.len.p, k->mc_b.col.p, sor_values<V>(k->mc_b), dia};
+    if (k->mc_one) {
+        hipLaunchKernelGGL((k_sor_block<V>), dim3(1), dim3(1024), sizeof(V) * (size_t)c->rows, c->stream, c->rows,
+                           ncol, k->mc_cptr.p, f, b, r, z, done_flag);
+        FLGPU_HIP(hipGetLastError());
+        return FLGPU_OK;
+    }
+    auto sweep = [&](const SorOp<V>& m, int q) {
+        const int s0 = k->mc_ptr[q], s1 = k->mc_ptr[q + 1];
+        if (s1 > s0)
+            hipLaunchKernelGGL((k_sor_slices<V>), dim3((s1 - s0 + 3) / 4), dim3(256), 0, c->stream, m, s0, s1, r, z,
+                               done_flag);
     };
-    for (int q = 0; q < ncol; q++) sweep(q);
-    for (int q = ncol - 2; q >= 0; q--) sweep(q);
+    for (int q = 0; q < ncol; q++) sweep(f, q);
+    for (int q = ncol - 2; q >= 0; q--) sweep(b, q);
     FLGPU_HIP(hipGetLastError());
     return FLGPU_OK;
 }
 
 template <typename V>
-static int ssor_apply(flgpu_ctx* c, KrylovWork* k, const V* val, const V* r, V* z, const V* w, double* partials,
+static int ssor_apply(flgpu_ctx* c, KrylovWork* k, const V* r, V* z, const V* w, double* partials,
                       int* nparts, const int* done_flag) {
-    FLGPU_TRY(ssor_sweeps<V>(c, k, val, r, z, done_flag));
+    FLGPU_TRY(ssor_sweeps<V>(c, k, r, z, done_flag));
     hipLaunchKernelGGL((k_pc_dots<V>), dim3(k->nblk), dim3(kVecBlock), 0, c->stream, c->rows, r, z, w, partials,
                        done_flag);
     FLGPU_HIP(hipGetLastError());
@@ -1038,17 +1235,13 @@ CgVecs<float> cg_vecs<float>(KrylovWork* k) {
 // own after the residual update.
 enum PcMode { PCM_DIAG = 0, PCM_LEARNED = 1, PCM_SSOR = 2 };
 
-template <typename V>
-static int ssor_apply(flgpu_ctx* c, KrylovWork* k, const V* val, const V* r, V* z, const V* w, double* partials,
-                      int* nparts, const int* done_flag);
-
 // z = M^-1 r for the learned factor (z = G^T (G r)) or SSOR; the per-block
 // sums r.z, z.z, z.w (w = A p of this iteration) go to the PART_PC region.
 // Returns the number of partial sums in *nparts.
 template <typename V>
 static int pc_apply(flgpu_ctx* c, KrylovWork* k, const CgVecs<V>& v, PcMode mode, const int* done_flag,
                     int* nparts) {
-    if (mode == PCM_SSOR) return ssor_apply<V>(c, k, v.val, v.r, v.z, v.w, k->part(PART_PC), nparts, done_flag);
+    if (mode == PCM_SSOR) return ssor_apply<V>(c, k, v.r, v.z, v.w, k->part(PART_PC), nparts, done_flag);
     return learned_precond_apply<V>(c, v.r, v.rt, v.z, v.y, v.w, k->part(PART_PC), nparts, done_flag);
 }
 
@@ -1163,7 +1356,7 @@ static int run_cg(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_info*
                                k->dinv32.p);
         FLGPU_HIP(hipGetLastError());
     }
-    if (mode == PCM_SSOR) FLGPU_TRY(ssor_prepare(c, k));
+    if (mode == PCM_SSOR) FLGPU_TRY(ssor_prepare<V>(c, k, v.val));
     Scal& h = *k->h_scal;
     // keep the pivot computed by build_reduced
     FLGPU_TRY(read_scal(c, k));
@@ -1343,7 +1536,7 @@ static int run_cg1(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_info
                                k->dinv32.p);
         FLGPU_HIP(hipGetLastError());
     }
-    if (mode == PCM_SSOR) FLGPU_TRY(ssor_prepare(c, k));
+    if (mode == PCM_SSOR) FLGPU_TRY(ssor_prepare<V>(c, k, v.val));
     Scal& h = *k->h_scal;
     FLGPU_TRY(read_scal(c, k));
     {
@@ -2069,7 +2262,7 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
     }
     // left SSOR: the product and the residual go through tmp, then the sweeps
     const bool ssor = sp->pc == FLGPU_PC_SOR;
-    if (ssor) FLGPU_TRY(ssor_prepare(c, k));
+    if (ssor) FLGPU_TRY(ssor_prepare<V>(c, k, val));
     V* tmp = mixed ? (V*)k->rt32.p : (V*)k->rt.p;
     const int nb = std::max(1, (int)std::min<int64_t>(kGmGrid, ((int64_t)n + 511) / 512));
     const size_t mm = (size_t)m + 1;
@@ -2126,7 +2319,7 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
                 default: launch(&k_gm_csr<64, V>); break;
             }
         }
-        if (ssor) FLGPU_TRY(ssor_sweeps<V>(c, k, val, tmp, out, &d.st->done));
+        if (ssor) FLGPU_TRY(ssor_sweeps<V>(c, k, tmp, out, &d.st->done));
         return FLGPU_OK;
     };
     // Gram-Schmidt of w against nv basis vectors, twice, and |w|^2
@@ -2169,7 +2362,7 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
         hipLaunchKernelGGL((k_gm_precres_norm<V>), dim3(nb), dim3(kGmNormBlock), 0, c->stream, n, k->r.p,
                            ssor ? nullptr : k->dinv.p, ssor ? tmp : wb[0], d);
         if (ssor) {
-            FLGPU_TRY(ssor_sweeps<V>(c, k, val, tmp, wb[0], nullptr));
+            FLGPU_TRY(ssor_sweeps<V>(c, k, tmp, wb[0], nullptr));
             hipLaunchKernelGGL((k_gm_norm<V>), dim3(nb), dim3(kGmNormBlock), 0, c->stream, n, wb[0], d);
         }
         FLGPU_HIP(hipGetLastError());
@@ -2437,8 +2630,8 @@ int pc_apply_host(flgpu_ctx* c, const flgpu_solver_params* sp, const double* r, 
     const int n = c->rows;
     FLGPU_HIP(hipMemcpyAsync(k->r.p, r, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
     if (sp->pc == FLGPU_PC_SOR) {
-        FLGPU_TRY(ssor_prepare(c, k));
-        FLGPU_TRY(ssor_sweeps<double>(c, k, k->val64.p, k->r.p, k->z.p, nullptr));
+        FLGPU_TRY(ssor_prepare<double>(c, k, k->val64.p));
+        FLGPU_TRY(ssor_sweeps<double>(c, k, k->r.p, k->z.p, nullptr));
     } else if (sp->pc == FLGPU_PC_LEARNED || sp->pc == FLGPU_PC_FSAI) {
         FLGPU_TRY(learned_prepare(c, false, sp->pc == FLGPU_PC_FSAI));
         hipLaunchKernelGGL(k_scale_res, dim3(k->nblk), dim3(kVecBlock), 0, c->stream, n, k->r.p, learned_scale(c),

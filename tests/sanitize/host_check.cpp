@@ -12,10 +12,9 @@
 // With --gpu it also binds the mesh to a device context and runs the
 // blocked assembly (the host-side slab plan builder), the two-pass P2
 // plan, the solve and the pressure path.
-#include <cmath>
-#include <cstdint>
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
