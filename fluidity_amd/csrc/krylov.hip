@@ -229,39 +229,69 @@ k_build(int nrb, const int32_t* __restrict__ rb, const int32_t* __restrict__ row
 // PCG / FCG vector kernels
 // ---------------------------------------------------------------------
 
+// The scalars an iteration reads and changes, in registers of every thread
+// (the whole Scal as a local variable would go through LDS or scratch).
+struct CgState {
+    double rz, rz_old, pAp, alpha, beta, rr, zz, zw, last_norm;
+    int its, reason, done;
+};
+
+__device__ __forceinline__ CgState cg_state(const Scal* __restrict__ in) {
+    return {in->rz, in->rz_old, in->pAp, in->alpha, in->beta, in->rr, in->zz, in->zw, in->last_norm, in->its, in->reason,
+            in->done};
+}
+
+// The next slot: the state, the rest carried over.
+__device__ __forceinline__ void cg_store(const Scal* __restrict__ in, Scal* __restrict__ out, const CgState& s) {
+    *out = *in;
+    out->rz = s.rz;
+    out->rz_old = s.rz_old;
+    out->pAp = s.pAp;
+    out->alpha = s.alpha;
+    out->beta = s.beta;
+    out->rr = s.rr;
+    out->zz = s.zz;
+    out->zw = s.zw;
+    out->last_norm = s.last_norm;
+    out->its = s.its;
+    out->reason = s.reason;
+    out->done = s.done;
+}
+
 // Convergence test of KSPConvergedDefault on the norm chosen by norm_type,
 // then beta (Fletcher-Reeves, or Polak-Ribiere when flexible).
-__device__ void cg_test(Scal* sc) {
-    sc->its += 1;
-    const double nrm = sc->norm_type == FLGPU_NORM_UNPRECONDITIONED ? sqrt(sc->rr) : sqrt(sc->zz);
-    sc->last_norm = nrm;
+__device__ __forceinline__ void cg_test(CgState& s, const Scal* __restrict__ in) {
+    s.its += 1;
+    const double nrm = in->norm_type == FLGPU_NORM_UNPRECONDITIONED ? sqrt(s.rr) : sqrt(s.zz);
+    const double rnorm0 = in->rnorm0;
+    s.last_norm = nrm;
     if (nrm != nrm || isinf(nrm)) {
-        sc->reason = KSP_DIVERGED_NANORINF;
-        sc->done = 1;
-    } else if (nrm <= sc->atol) {
-        sc->reason = KSP_CONVERGED_ATOL;
-        sc->done = 1;
-    } else if (nrm <= sc->rtol * sc->rnorm0) {
-        sc->reason = KSP_CONVERGED_RTOL;
-        sc->done = 1;
-    } else if (sc->rnorm0 > 0 && nrm >= 1e5 * sc->rnorm0) {
-        sc->reason = KSP_DIVERGED_DTOL;
-        sc->done = 1;
-    } else if (sc->its >= sc->max_its) {
-        sc->reason = KSP_DIVERGED_ITS;
-        sc->done = 1;
+        s.reason = KSP_DIVERGED_NANORINF;
+        s.done = 1;
+    } else if (nrm <= in->atol) {
+        s.reason = KSP_CONVERGED_ATOL;
+        s.done = 1;
+    } else if (nrm <= in->rtol * rnorm0) {
+        s.reason = KSP_CONVERGED_RTOL;
+        s.done = 1;
+    } else if (rnorm0 > 0 && nrm >= 1e5 * rnorm0) {
+        s.reason = KSP_DIVERGED_DTOL;
+        s.done = 1;
+    } else if (s.its >= in->max_its) {
+        s.reason = KSP_DIVERGED_ITS;
+        s.done = 1;
     }
 }
 
-__device__ void cg_test_and_beta(Scal* sc) {
-    cg_test(sc);
-    if (sc->flexible)
-        sc->beta = -sc->alpha * sc->zw / sc->rz_old;  // z.(r_new - r_old) / (z_old.r_old)
+__device__ __forceinline__ void cg_test_and_beta(CgState& s, const Scal* __restrict__ in) {
+    cg_test(s, in);
+    if (in->flexible)
+        s.beta = -s.alpha * s.zw / s.rz_old;  // z.(r_new - r_old) / (z_old.r_old)
     else
-        sc->beta = sc->rz / sc->rz_old;
-    if (!sc->done && sc->rz < 0.0) {
-        sc->reason = KSP_DIVERGED_INDEFINITE_PC;
-        sc->done = 1;
+        s.beta = s.rz / s.rz_old;
+    if (!s.done && s.rz < 0.0) {
+        s.reason = KSP_DIVERGED_INDEFINITE_PC;
+        s.done = 1;
     }
 }
 
@@ -269,11 +299,6 @@ __device__ void cg_test_and_beta(Scal* sc) {
 // them reads slot "in" in every block and block 0 writes the next state
 // to slot "out", so no block can see a value written during its own
 // kernel.  A finished solve carries the state over unchanged.
-__device__ __forceinline__ bool carry_if_done(const Scal* __restrict__ in, Scal* __restrict__ out) {
-    if (!in->done) return false;
-    if (blockIdx.x == 0 && threadIdx.x == 0 && out != in) *out = *in;
-    return true;
-}
 
 // R consecutive entries as one vector load / store (R * sizeof(T) bytes;
 // the caller checks the alignment with rows_aligned)
@@ -289,6 +314,13 @@ __device__ __forceinline__ void st_rows(T* __restrict__ a, int i, const Rows<T, 
     *reinterpret_cast<Rows<T, R>*>(a + i) = v;
 }
 
+// The vector kernels of an iteration are bound by latency (a launch, the
+// partial sums, the rows): so one block per CU, every load in flight before
+// the first is used, one barrier, and the scalar step taken by every thread.
+// With 512 blocks of 512, a broadcast by thread 0 and rows loaded after it:
+// update 9.9 and p 7.2 us on 274k FP64 rows, 13.6 and 12.0 us on 1.37M FP32
+// rows with a factor; so 7.4 and 4.3, 11.2 and 6.8 us.
+//
 // pAp from the SpMV partials, alpha = rz / pAp; x += alpha p;
 // r -= alpha w; [Jacobi: z = D^-1 r]; [learned: rt = D_s r, the residual in
 // the preconditioner's scaled space]; partials r.z, r.r, z.z, z.w.  Each
@@ -302,13 +334,24 @@ k_cg_update(int n, V* __restrict__ x, const V* __restrict__ p, V* __restrict__ r
             const float* __restrict__ dsc, V* __restrict__ rt,
             const double* __restrict__ pspmv, int nspmv, double* __restrict__ pvec,
             const Scal* __restrict__ in, Scal* __restrict__ out) {
-    __shared__ double s_alpha;
-    __shared__ int s_stop;
-    if (carry_if_done(in, out)) return;
+    // The thread's first group of rows, the scalars and the partial sums are
+    // in flight together; every thread takes the scalar step itself.
+    const int ng = n / R, tid = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+    Rows<V, R> pv = {}, wv = {}, rv = {}, dv = {}, xv = {};
+    Rows<float, R> sv = {};
+    auto load = [&](int i) {
+        pv = ld_rows<R>(p, i);
+        wv = ld_rows<R>(w, i);
+        rv = ld_rows<R>((const V*)r, i);
+        xv = ld_rows<R>((const V*)x, i);
+        if (jacobi) dv = ld_rows<R>(dinv, i);
+        if (dsc) sv = ld_rows<R>(dsc, i);
+    };
+    if (tid < ng) load(tid * R);
+    CgState s = cg_state(in);
     double pap[1];
-    sum_partials<1>(pspmv, nspmv, pap);
-    if (threadIdx.x == 0) {
-        Scal s = *in;
+    part_totals<1>(pspmv, nspmv, pap);
+    if (!s.done) {
         s.pAp = pap[0];
         s.rz_old = s.rz;
         if (!(pap[0] > 0.0)) {
@@ -317,13 +360,10 @@ k_cg_update(int n, V* __restrict__ x, const V* __restrict__ p, V* __restrict__ r
         } else {
             s.alpha = s.rz / pap[0];
         }
-        s_alpha = s.alpha;
-        s_stop = s.done;
-        if (blockIdx.x == 0) *out = s;
     }
-    __syncthreads();
-    if (s_stop) return;
-    const double alpha = s_alpha;
+    if (blockIdx.x == 0 && threadIdx.x == 0) cg_store(in, out, s);
+    if (s.done) return;
+    const double alpha = s.alpha;
     const V a = (V)alpha;
     double s_rz = 0.0, s_rr = 0.0, s_zz = 0.0, s_zw = 0.0;
     auto row = [&](V& xi, V pi, V wi, V& ri, V di, float si, V& zi, V& ti) {
@@ -338,15 +378,10 @@ k_cg_update(int n, V* __restrict__ x, const V* __restrict__ p, V* __restrict__ r
         }
         s_rr += (double)ri * (double)ri;
     };
-    const int ng = n / R, tid = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
     for (int g = tid; g < ng; g += nt) {
         const int i = g * R;
-        const Rows<V, R> pv = ld_rows<R>(p, i), wv = ld_rows<R>(w, i);
-        Rows<V, R> rv = ld_rows<R>(r, i), dv = {}, zv = {}, tv = {};
-        Rows<V, R> xv = ld_rows<R>((const V*)x, i);
-        Rows<float, R> sv = {};
-        if (jacobi) dv = ld_rows<R>(dinv, i);
-        if (dsc) sv = ld_rows<R>(dsc, i);
+        if (g != tid) load(i);
+        Rows<V, R> zv = {}, tv = {};
 #pragma unroll
         for (int u = 0; u < R; u++) {
             V xi = xv[u];
@@ -382,10 +417,8 @@ template <typename V, int R>
 __global__ void __launch_bounds__(kVecBlock)
 k_cg_p(int n, const V* __restrict__ z, V* __restrict__ p, const double* __restrict__ pvec, int nvec,
        const double* __restrict__ ppc, int npc, const Scal* __restrict__ in, Scal* __restrict__ out) {
-    __shared__ double s_beta;
-    __shared__ int s_stop;
     // The thread's first group of rows does not depend on the scalars: its
-    // loads are issued before the done flag's and the partial sums', so the
+    // loads are issued before the scalars' and the partial sums', so the
     // three are in flight together (one memory round trip, not two).
     const int ng = n / R, tid = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
     Rows<V, R> zv = {}, pv = {};
@@ -394,30 +427,29 @@ k_cg_p(int n, const V* __restrict__ z, V* __restrict__ p, const double* __restri
         pv = ld_rows<R>((const V*)p, i);
     };
     if (tid < ng) load(tid * R);
-    if (carry_if_done(in, out)) return;
-    double u[4], q[3] = {0.0, 0.0, 0.0};
-    sum_partials<4>(pvec, nvec, u);
-    if (ppc) sum_partials<3>(ppc, npc, q);
-    if (threadIdx.x == 0) {
-        Scal s = *in;
-        s.rr = u[1];
-        if (ppc) {
-            s.rz = q[0];
-            s.zz = q[1];
-            s.zw = q[2];
-        } else {
-            s.rz = u[0];
-            s.zz = u[2];
-            s.zw = u[3];
-        }
-        cg_test_and_beta(&s);
-        s_beta = s.beta;
-        s_stop = s.done;
-        if (blockIdx.x == 0) *out = s;
+    CgState s = cg_state(in);
+    double u[4];
+    if (ppc) {
+        double q[3], rr[1];
+        part_totals<3>(ppc, npc, q);
+        part_totals<1>(pvec + kPartStride, nvec, rr);
+        u[0] = q[0];
+        u[1] = rr[0];
+        u[2] = q[1];
+        u[3] = q[2];
+    } else {
+        part_totals<4>(pvec, nvec, u);
     }
-    __syncthreads();
-    if (s_stop) return;
-    const V beta = (V)s_beta;
+    if (!s.done) {
+        s.rz = u[0];
+        s.rr = u[1];
+        s.zz = u[2];
+        s.zw = u[3];
+        cg_test_and_beta(s, in);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) cg_store(in, out, s);
+    if (s.done) return;
+    const V beta = (V)s.beta;
     for (int g = tid; g < ng; g += nt) {
         const int i = g * R;
         if (g != tid) load(i);
@@ -448,8 +480,6 @@ k_cg1_vec(int n, double* __restrict__ x, V* __restrict__ p, V* __restrict__ s, V
           const float* __restrict__ dsc, V* __restrict__ rt, const double* __restrict__ pspmv, int nspmv,
           const double* __restrict__ pg, int ng, int pc_layout, const double* __restrict__ prr, int nrr, int first,
           double* __restrict__ pvec, const Scal* __restrict__ in, Scal* __restrict__ out) {
-    __shared__ double s_ab[2];
-    __shared__ int s_stop;
     // the first group's loads in flight with the scalars' (as k_cg_p)
     const int ng_ = n / R, tid = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
     Rows<V, R> pv = {}, sv = {}, rv = {}, uv = {}, wv = {}, dv = {};
@@ -466,21 +496,20 @@ k_cg1_vec(int n, double* __restrict__ x, V* __restrict__ p, V* __restrict__ s, V
         if (dsc) fv = ld_rows<R>(dsc, i);
     };
     if (tid < ng_) load(tid * R);
-    if (carry_if_done(in, out)) return;
-    double dl[1], g[3] = {0.0, 0.0, 0.0}, q[3] = {0.0, 0.0, 0.0};
-    sum_partials<1>(pspmv, nspmv, dl);
+    CgState sc = cg_state(in);
+    double dl[1], g[3] = {0.0, 0.0, 0.0}, q[1] = {0.0};
+    part_totals<1>(pspmv, nspmv, dl);
     if (!first) {
-        sum_partials<3>(pg, ng, g);
-        if (pc_layout) sum_partials<3>(prr, nrr, q);
+        part_totals<3>(pg, ng, g);
+        if (pc_layout) part_totals<1>(prr + kPartStride, nrr, q);
     }
-    if (threadIdx.x == 0) {
-        Scal sc = *in;
+    if (!sc.done) {
         if (!first) {
             sc.rz_old = sc.rz;
             sc.rz = g[0];
-            sc.rr = pc_layout ? q[1] : g[1];
+            sc.rr = pc_layout ? q[0] : g[1];
             sc.zz = pc_layout ? g[1] : g[2];
-            cg_test(&sc);
+            cg_test(sc, in);
         }
         const double delta = dl[0];
         sc.pAp = delta;
@@ -498,15 +527,11 @@ k_cg1_vec(int n, double* __restrict__ x, V* __restrict__ p, V* __restrict__ s, V
                 sc.alpha = sc.rz / denom;
             }
         }
-        s_ab[0] = sc.alpha;
-        s_ab[1] = sc.beta;
-        s_stop = sc.done;
-        if (blockIdx.x == 0) *out = sc;
     }
-    __syncthreads();
-    if (s_stop) return;
-    const double alpha = s_ab[0];
-    const V a = (V)alpha, b = (V)s_ab[1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) cg_store(in, out, sc);
+    if (sc.done) return;
+    const double alpha = sc.alpha;
+    const V a = (V)alpha, b = (V)sc.beta;
     double s_g = 0.0, s_rr = 0.0, s_uu = 0.0;
     auto row = [&](double& xi, V& pi, V& si, V ui, V wi, V& ri, V di, float dsi, V& uo, V& ti) {
         pi = first ? ui : fma(b, pi, ui);
@@ -829,13 +854,11 @@ template <typename V, typename CT, typename XV, typename YV>
 static void sell_launch(flgpu_ctx* c, KrylovWork* k, const V* sval, const CT* col, const XV* x, YV* y,
                         const double* bsub, int want_dot, const int* done_flag) {
     const SellOp<V, CT> m{k->nsl, c->rows, k->sptr.p, c->rowptr.p, col, sval, nullptr, k->srows.p};
-    const int grid = sell_grid(k->nsl);
     if (want_dot)
-        hipLaunchKernelGGL((k_sell<V, V, CT, XV, YV, DOT_XY>), dim3(grid), dim3(kRowBlock), 0, c->stream, m, x, y,
-                           bsub, (const V*)nullptr, (const V*)nullptr, k->part(PART_SPMV), done_flag);
+        sell_product<V, V, CT, XV, YV, DOT_XY>(c->stream, m, x, y, bsub, nullptr, nullptr, k->part(PART_SPMV), done_flag);
     else
-        hipLaunchKernelGGL((k_sell<V, V, CT, XV, YV, DOT_NONE>), dim3(grid), dim3(kRowBlock), 0, c->stream, m, x,
-                           y, bsub, (const V*)nullptr, (const V*)nullptr, k->part(PART_SPMV), done_flag);
+        sell_product<V, V, CT, XV, YV, DOT_NONE>(c->stream, m, x, y, bsub, nullptr, nullptr, k->part(PART_SPMV),
+                                                 done_flag);
 }
 
 template <typename AV, typename CT>

@@ -32,8 +32,9 @@ struct Scal {
     int32_t norm_type, flexible, pad0, pad1;
 };
 
-constexpr int kVecBlock = 512;     // threads per block of the vector kernels (8 waves)
-constexpr int kMaxVecGrid = 512;   // their fixed grid (2 blocks per CU)
+constexpr int kVecBlock = 1024;    // threads per block of the vector kernels (16 waves)
+constexpr int kMaxVecGrid = 256;   // their fixed grid: one block per CU, so that a consumer has few
+                                   // partial sums to add
 constexpr int kRowBlock = 256;     // threads per block of the CSR row products
 constexpr int kMaxRowGrid = 2048;  // their fixed grid
 constexpr int kPartStride = 2048;  // partials[k * kPartStride + block], >= either grid
@@ -49,12 +50,30 @@ enum {
     PART_COMPONENTS = 15
 };
 
+// Sum over the wave by DPP moves (8-cycle steps instead of LDS shuffles, in
+// a fixed order), in every lane.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_total(double v) {
+    v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: the last lane of each 16 has their sum
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3, row_bcast 31 into rows 2 and 3
+    v = dpp_add<0x143, 0xc>(v);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
 // Sum over a block in a fixed order; result valid in thread 0.
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double (*sh)[NV]) {
 #pragma unroll
-    for (int k = 0; k < NV; k++)
-        for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
+    for (int k = 0; k < NV; k++) v[k] = wave_total(v[k]);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0)
 #pragma unroll
@@ -81,6 +100,32 @@ __device__ __forceinline__ void block_partials(double (&v)[NV], double* __restri
     if (threadIdx.x == 0)
 #pragma unroll
         for (int k = 0; k < NV; k++) partials[(size_t)k * kPartStride + blockIdx.x] = v[k];
+}
+
+// Totals of the nparts per-block sums of NV components, in every thread of a
+// kVecBlock block: each wave takes 64 of a component's sums at a time, so up
+// to kVecBlock / NV sums are one load, and the waves' totals are added in
+// order.  The same sums in every block.
+template <int NV>
+__device__ __forceinline__ void part_totals(const double* __restrict__ partials, int nparts, double (&out)[NV]) {
+    constexpr int G = kVecBlock / 64 / NV;  // waves per component
+    __shared__ double sh[NV][G];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (wave < G * NV) {
+        const int c = wave / G, g = wave % G;
+        double t = 0.0;
+#pragma unroll 4
+        for (int b = g * 64 + lane; b < nparts; b += 64 * G) t += partials[(size_t)c * kPartStride + b];
+        t = wave_total(t);
+        if (lane == 0) sh[c][g] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NV; c++) {
+        out[c] = sh[c][0];
+#pragma unroll
+        for (int g = 1; g < G; g++) out[c] += sh[c][g];
+    }
 }
 
 // Total of the nparts per-block sums a previous kernel wrote.  Every block
@@ -343,7 +388,7 @@ k_sell(SellOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, const dou
        const V* __restrict__ dr, const V* __restrict__ dw, double* __restrict__ partials,
        const int* __restrict__ done_flag) {
 #pragma clang fp contract(off)
-    if (done_flag && *done_flag) return;
+    const int done = done_flag ? *done_flag : 0;
     constexpr int WPB = kRowBlock / kSlice;
     constexpr int U = 8;
     const int wave = threadIdx.x / kSlice, lane = threadIdx.x % kSlice;
@@ -357,7 +402,8 @@ k_sell(SellOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, const dou
         int r0;
         const int row = sell_row(m, sl, lane, r0);
         const int base = m.sptr[sl], w = (m.sptr[sl + 1] - base) / kSlice;
-        const int len = row < m.n ? m.rowptr[row + 1] - m.rowptr[row] : 0;
+        const int rc = min(row, m.n - 1), len = row < m.n ? m.rowptr[rc + 1] - m.rowptr[rc] : 0;
+        if (done) break;  // (after the slice's own loads, which are in flight with the flag's)
         V acc = (V)0;
         for (int j0 = 0; j0 < w; j0 += U) {
             // Every load is unconditional (a step past the slice's width
@@ -398,6 +444,7 @@ k_sell(SellOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, const dou
             }
         }
     }
+    if (done) return;
     if (DOTS == DOT_XY) {
         double v[2] = {d0, d1};
         block_partials<2>(v, partials);
@@ -505,7 +552,7 @@ k_sell_gather(int64_t m, const int32_t* __restrict__ src, const SV* __restrict__
     }
 }
 
-// Fixed grid for k_sell: the slice groups through stream_grid.
+// Fixed grid of k_sell.
 inline int sell_grid(int nsl);
 
 // int16 column offsets from each row block's first row; false (and out
@@ -538,6 +585,21 @@ inline int stream_grid(int nrb) {
     return g & ~7;
 }
 
-inline int sell_grid(int nsl) { return stream_grid((nsl + kRowBlock / kSlice - 1) / (kRowBlock / kSlice)); }
+// The groups of slices over as many workgroups as give each the same number
+// of them (a workgroup with one more would double a short product's time).
+inline int sell_grid(int nsl) {
+    constexpr int per = kRowBlock / kSlice;
+    const int groups = (nsl + per - 1) / per;
+    if (groups < 8) return std::max(1, groups);
+    const int rounds = (groups + stream_grid(kMaxRowGrid) - 1) / stream_grid(kMaxRowGrid);
+    return ((groups + rounds - 1) / rounds + 7) & ~7;
+}
+
+template <typename V, typename AV, typename CT, typename XV, typename YV, int DOTS>
+inline void sell_product(hipStream_t stream, const SellOp<AV, CT>& m, const XV* x, YV* y, const double* bsub,
+                         const V* dr, const V* dw, double* partials, const int* done_flag) {
+    hipLaunchKernelGGL((k_sell<V, AV, CT, XV, YV, DOTS>), dim3(sell_grid(m.nsl)), dim3(kRowBlock), 0, stream, m, x, y,
+                       bsub, dr, dw, partials, done_flag);
+}
 
 }  // namespace flgpu

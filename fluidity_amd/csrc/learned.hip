@@ -1300,10 +1300,8 @@ static void apply_launch_sell(flgpu_ctx* c, LearnedState* s, const HV* gl, const
     const int n = c->rows;
     const SellOp<HV, LC> lo{s->nsll, n, s->lsp.p, s->lptr.p, lcol, gl, nullptr};
     const SellOp<HV, UC> up{s->nslu, n, s->usp.p, s->uptr.p, ucol, gu, s->dsq.p};
-    hipLaunchKernelGGL((k_sell<V, HV, LC, V, V, DOT_NONE>), dim3(sell_grid(s->nsll)), dim3(kRowBlock), 0, c->stream,
-                       lo, rt, y, (const double*)nullptr, (const V*)nullptr, (const V*)nullptr, partials, done);
-    hipLaunchKernelGGL((k_sell<V, HV, UC, V, V, DOT_PC>), dim3(sell_grid(s->nslu)), dim3(kRowBlock), 0, c->stream,
-                       up, (const V*)y, z, (const double*)nullptr, r, w, partials, done);
+    sell_product<V, HV, LC, V, V, DOT_NONE>(c->stream, lo, rt, y, nullptr, nullptr, nullptr, partials, done);
+    sell_product<V, HV, UC, V, V, DOT_PC>(c->stream, up, y, z, nullptr, r, w, partials, done);
 }
 
 template <typename V, typename HV>

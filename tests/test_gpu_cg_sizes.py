@@ -1,0 +1,40 @@
+"""CG, flexible CG with a factor and the single-reduction CG where the block
+sums and grids of their kernels change: one block, one row more than a
+block, one block per CU and more than one row group a thread; products of
+one slice, of uneven groups, and of several rounds.  The reference is the
+oracle's Jacobi-CG to a relative residual of 1e-13; the difference is bounded
+by cond(D^-1 A) (1e-13 + rtol), and these Poisson systems' condition numbers
+are below 0.7 (cells a side)^2.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from fluidity_amd import cg, meshgen as M
+
+pytestmark = pytest.mark.gpu
+
+METHODS = [("cg", "jacobi", "fp64"), ("cg", "jacobi", "mixed"), ("cg", "none", "fp64"), ("cg", "fsai", "fp64"),
+           ("fcg", "fsai", "mixed"), ("cg", "sor", "fp64"), ("pipecg", "jacobi", "fp64"), ("pipecg", "fsai", "mixed")]
+
+
+@pytest.mark.parametrize("scale", [2, 3, 9, 10, 39, 64])  # 27, 64, 1000, 1331, 64000 and 274625 rows
+def test_cg_against_oracle(require_gpu, scale):
+    cfg = M.config("c2", seed=23, scale=scale)
+    ref = O.reference_system(cfg)
+    xr, _, reason, _, _ = O.petsc_solve("cg", "jacobi", 1e-13, ref["sparsity"], ref["A"], ref["inactive"], ref["rhs"])
+    assert reason > 0
+    pr = cg.problem_from_config(cfg)
+    cg.assemble_advection_diffusion_cg(pr, cg.options_from_config(cfg), cfg.dt)
+    cg.apply_dirichlet_conditions(pr, cfg.mesh.boundary, 0.0, cfg.dt)
+    rtol = 1e-10
+    tol = 0.7 * max(scale, 3) ** 2 * (rtol + 1e-13)
+    for ksp, pc, precision in METHODS:
+        print(f"\n[case] {ksp} {pc} {precision} rows {cfg.mesh.nnodes}", flush=True)
+        so = cg.SolverOptions(ksp, pc, relative_error=rtol, precision=precision, norm="unpreconditioned")
+        x, info = cg.petsc_solve(pr, so)
+        assert info.reason > 0 and info.true_relres <= rtol * (1 + 1e-6), (ksp, pc, precision, info.true_relres)
+        assert np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr), (ksp, pc, precision)
+        x2, info2 = cg.petsc_solve(pr, so)
+        assert np.array_equal(x, x2) and info2.its == info.its  # fixed order of every sum
+    pr.close()
