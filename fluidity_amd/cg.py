@@ -289,9 +289,9 @@ class CGProblem:
     # -- system --------------------------------------------------------
     def matrix(self):
         """(A values, rhs, inactive mask) copied from the device."""
-        A = np.zeros(self.sparsity.nnz)
-        rhs = np.zeros(self.mesh.nnodes)
-        inact = np.zeros(self.mesh.nnodes, np.int32)
+        A = np.empty(self.sparsity.nnz)
+        rhs = np.empty(self.mesh.nnodes)
+        inact = np.empty(self.mesh.nnodes, np.int32)
         L.check(self.lib.flgpu_matrix_get(self.ctx, L.ptr(A), L.ptr(rhs), L.ptr(inact)), "flgpu_matrix_get")
         return A, rhs, inact
 
@@ -507,8 +507,8 @@ def construct_momentum_ct(problem: CGProblem, pm: PressureMesh, integrate_contin
     returns (ct_val (dim, nnz), masslump (velocity nodes))."""
     d = problem.mesh.dim
     rho = np.atleast_1d(np.ascontiguousarray(density, dtype=np.float64))
-    ct = np.zeros((d, pm.ct_colm.size))
-    ml = np.zeros(problem.mesh.nnodes)
+    ct = np.empty((d, pm.ct_colm.size))
+    ml = np.empty(problem.mesh.nnodes)
     L.check(problem.lib.flgpu_ct_assemble(problem.ctx, int(integrate_continuity_by_parts), int(rho.size == 1),
                                           L.ptr(rho), L.ptr(ct), L.ptr(ml)), "flgpu_ct_assemble")
     return ct, ml
@@ -531,7 +531,7 @@ def assemble_masslumped_cmc(problem: CGProblem, cmc_findrm: np.ndarray, cmc_colm
     velocity nodes) or None for 1/masslump in every component."""
     im = None if inverse_masslump is None else np.ascontiguousarray(
         np.asarray(inverse_masslump, np.float64).reshape(problem.mesh.dim, -1).T)
-    out = np.zeros(cmc_colm.size)
+    out = np.empty(cmc_colm.size)
     L.check(problem.lib.flgpu_cmc_assemble(problem.ctx, None if im is None else L.ptr(im), cmc_findrm.size - 1,
                                            L.ptr(cmc_findrm), L.ptr(cmc_colm), L.ptr(out)), "flgpu_cmc_assemble")
     return out

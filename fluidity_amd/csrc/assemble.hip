@@ -2118,11 +2118,10 @@ static int assemble_check(flgpu_ctx* c, int* d_err) {
 
 int assemble(flgpu_ctx* c, const flgpu_advdif_params* p) {
     c->assembled = false;  // set again only when this assembly succeeds
-    DevBuf<int> d_err;
-    FLGPU_TRY(d_err.alloc(1));
-    FLGPU_HIP(hipMemsetAsync(d_err.p, 0, sizeof(int), c->stream));
-    FLGPU_TRY(assemble_launch(c, p, d_err.p));
-    return assemble_check(c, d_err.p);
+    FLGPU_TRY(c->asm_err.alloc(1));
+    FLGPU_HIP(hipMemsetAsync(c->asm_err.p, 0, sizeof(int), c->stream));
+    FLGPU_TRY(assemble_launch(c, p, c->asm_err.p));
+    return assemble_check(c, c->asm_err.p);
 }
 
 int assembly_plan_info(flgpu_ctx* c, int64_t* info, int n, double* build_seconds) {

@@ -251,6 +251,12 @@ struct flgpu_ctx {
     bool have_inactive = false;
     bool assembled = false;
 
+    // kept between calls: assembly's error flag, the strong Dirichlet nodes
+    // and values
+    flgpu::DevBuf<int> asm_err;
+    flgpu::DevBuf<int32_t> bc_nodes;
+    flgpu::DevBuf<double> bc_values;
+
     flgpu::BlockPlan plan;
     flgpu::SurfaceState surf;
     flgpu::KrylovWork* kw = nullptr;
@@ -286,6 +292,9 @@ void learned_free(flgpu_ctx* c);
 void pressure_free(flgpu_ctx* c);
 // shared helpers
 unsigned grid_for(int64_t n, int block);
+// Device memory to the caller's pageable memory, after the work queued on
+// the context's stream; `dst` is complete once the stream is synchronised.
+int copy_out(flgpu_ctx* c, void* dst, const void* src, size_t bytes);
 // setup_gpu.hip: out[0..n) = exclusive prefix sums of in[0..n), out[n] = the total
 int exclusive_scan(hipStream_t s, const int32_t* in, int64_t n, DevBuf<int64_t>& out);
 // flgpu_context.hip: bind a colouring already known to be valid (0-based)

@@ -2463,8 +2463,7 @@ int solve(flgpu_ctx* c, const flgpu_solver_params* sp, double* x_host, flgpu_sol
     hipLaunchKernelGGL(k_finish_x, dim3(grid_for(c->rows, kVecBlock)), dim3(kVecBlock), 0, c->stream, c->rows,
                        k->x.p, c->rhs.p, c->inactive.p, c->have_inactive ? 1 : 0);
     FLGPU_HIP(hipGetLastError());
-    if (x_host)
-        FLGPU_HIP(hipMemcpyAsync(x_host, k->x.p, sizeof(double) * c->rows, hipMemcpyDeviceToHost, c->stream));
+    if (x_host) FLGPU_TRY(copy_out(c, x_host, k->x.p, sizeof(double) * c->rows));
     FLGPU_HIP(hipStreamSynchronize(c->stream));
     k->have_x = true;
     if (info_out) *info_out = info;
@@ -2617,7 +2616,7 @@ int solve_noalloc(flgpu_ctx* c, const flgpu_solver_params* sp, double* x_host, f
 
 int solution_get(flgpu_ctx* c, double* x) {
     if (!c->kw || !c->kw->have_x) return set_error(FLGPU_EINVAL, "flgpu_solution_get: no solution");
-    FLGPU_HIP(hipMemcpyAsync(x, c->kw->x.p, sizeof(double) * c->rows, hipMemcpyDeviceToHost, c->stream));
+    FLGPU_TRY(copy_out(c, x, c->kw->x.p, sizeof(double) * c->rows));
     FLGPU_HIP(hipStreamSynchronize(c->stream));
     return FLGPU_OK;
 }

@@ -25,6 +25,7 @@
 #include <cmath>
 #include <cstring>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "flgpu_internal.h"
@@ -55,6 +56,8 @@ struct PressureState {
     DevBuf<double> ct, ml;                   // ct_m (dim blocks of ct_nnz) and the lumped mass
     bool assembled = false;
     DevBuf<int32_t> cmc_rowptr, cmc_col;     // the last cmc pattern
+    DevBuf<int32_t> cmc_in;                  // the pattern being checked, then swapped with cmc_col
+    DevBuf<unsigned long long> cmc_bad;      // its first entry out of range
     int32_t cmc_rows = 0;
     int64_t cmc_nnz = -1;                    // -1: no cmc assembled yet
     DevBuf<double> cmc, inv;
@@ -347,6 +350,17 @@ __global__ void __launch_bounds__(256) k_invert_ml(int n, const double* __restri
     for (int d = 0; d < DIM; d++) inv[(int64_t)i * DIM + d] = v;
 }
 
+// 1-based column indices to 0-based, in place; the smallest position whose
+// index is outside 1..ncols goes to *bad.
+__global__ void __launch_bounds__(256)
+k_zero_based(int64_t nnz, int ncols, int32_t* __restrict__ col, unsigned long long* __restrict__ bad) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nnz) return;
+    const int32_t v = col[k];
+    if (v < 1 || v > ncols) atomicMin(bad, (unsigned long long)k);
+    col[k] = v - 1;
+}
+
 // C_P^T M_l^-1 C a wave per cmc row i: row i of ct (columns, the dim
 // values and the inverse lumped mass of each column) staged in the wave's
 // LDS slice once, then each lane takes an entry (i, j) and walks row j of
@@ -550,8 +564,8 @@ int ct_assemble(flgpu_ctx* c, PressureState& S, int ibp, int density_const, cons
     int h_err = 0;
     FLGPU_HIP(hipMemcpyAsync(&h_err, S.err.p, sizeof(int), hipMemcpyDeviceToHost, s));
     if (ct_out)
-        FLGPU_HIP(hipMemcpyAsync(ct_out, S.ct.p, sizeof(double) * S.ct_nnz * dim, hipMemcpyDeviceToHost, s));
-    if (ml_out) FLGPU_HIP(hipMemcpyAsync(ml_out, S.ml.p, sizeof(double) * c->nnodes, hipMemcpyDeviceToHost, s));
+        FLGPU_TRY(copy_out(c, ct_out, S.ct.p, sizeof(double) * S.ct_nnz * dim));
+    if (ml_out) FLGPU_TRY(copy_out(c, ml_out, S.ml.p, sizeof(double) * c->nnodes));
     FLGPU_HIP(hipStreamSynchronize(s));
     if (h_err) return set_error(FLGPU_EPATTERN, "Attempting to set value in matrix outside sparsity pattern.");
     S.assembled = true;
@@ -571,16 +585,27 @@ int cmc_assemble(flgpu_ctx* c, PressureState& S, const double* inverse_masslump,
         if (i > 0 && rp[i] < rp[i - 1]) return set_error(FLGPU_EINVAL, "flgpu_cmc_assemble: findrm decreases at %d", i);
     }
     const int64_t nnz = rp[rows];
-    std::vector<int32_t> cl((size_t)nnz);
-    for (int64_t k = 0; k < nnz; k++) {
-        const int v = colm[k] - 1;
-        if (v < 0 || v >= S.p_nodes)
-            return set_error(FLGPU_EINVAL, "flgpu_cmc_assemble: colm(%lld) = %d out of 1..%d", (long long)k + 1,
-                             colm[k], S.p_nodes);
-        cl[k] = v;
+    // the columns are checked and shifted to 0-based on the device; an
+    // accepted pattern replaces the last one
+    const unsigned long long none = ~0ull;
+    unsigned long long bad = none;
+    FLGPU_TRY(S.cmc_in.alloc((size_t)std::max<int64_t>(nnz, 1)));
+    FLGPU_TRY(S.cmc_bad.alloc(1));
+    FLGPU_HIP(hipMemcpyAsync(S.cmc_bad.p, &none, sizeof none, hipMemcpyHostToDevice, s));
+    if (nnz > 0) {
+        FLGPU_HIP(hipMemcpyAsync(S.cmc_in.p, colm, sizeof(int32_t) * (size_t)nnz, hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(k_zero_based, dim3(grid_for(nnz, 256)), dim3(256), 0, s, nnz, S.p_nodes, S.cmc_in.p,
+                           S.cmc_bad.p);
+        FLGPU_HIP(hipGetLastError());
     }
+    FLGPU_HIP(hipMemcpyAsync(&bad, S.cmc_bad.p, sizeof bad, hipMemcpyDeviceToHost, s));
+    FLGPU_HIP(hipStreamSynchronize(s));
+    if (bad != none)
+        return set_error(FLGPU_EINVAL, "flgpu_cmc_assemble: colm(%lld) = %d out of 1..%d", (long long)bad + 1,
+                         colm[bad], S.p_nodes);
+    std::swap(S.cmc_col.p, S.cmc_in.p);
+    std::swap(S.cmc_col.n, S.cmc_in.n);
     FLGPU_TRY(S.cmc_rowptr.upload(rp.data(), rp.size(), s));
-    FLGPU_TRY(S.cmc_col.upload(cl.data(), cl.size(), s));
     FLGPU_TRY(S.cmc.alloc((size_t)std::max<int64_t>(nnz, 1)));
     FLGPU_TRY(S.inv.alloc((size_t)c->nnodes * dim));
     if (inverse_masslump)
@@ -589,8 +614,8 @@ int cmc_assemble(flgpu_ctx* c, PressureState& S, const double* inverse_masslump,
     S.cmc_rows = rows;
     S.cmc_nnz = nnz;
     FLGPU_TRY(cmc_launch(c, S, !inverse_masslump));
-    if (out && nnz > 0) FLGPU_HIP(hipMemcpyAsync(out, S.cmc.p, sizeof(double) * nnz, hipMemcpyDeviceToHost, s));
-    FLGPU_HIP(hipStreamSynchronize(s));  // rp, cl and the host arrays
+    if (out && nnz > 0) FLGPU_TRY(copy_out(c, out, S.cmc.p, sizeof(double) * nnz));
+    FLGPU_HIP(hipStreamSynchronize(s));  // rp and the host arrays
     return FLGPU_OK;
 }
 
