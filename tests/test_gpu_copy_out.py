@@ -55,10 +55,11 @@ def test_two_contexts_on_two_threads(require_gpu):
         p.close()
 
 
-def test_cmc_pattern_checked_on_the_device(require_gpu):
+@pytest.mark.parametrize("n", [4, 8])  # checked on the host, on the device
+def test_cmc_pattern_check(require_gpu, n):
     """The first column out of range is named, and the last accepted pattern
     stays in place."""
-    mesh = M.cube_tets(4)
+    mesh = M.cube_tets(n)
     pr = cg.CGProblem(mesh)
     pm = cg.vertex_pressure_mesh(pr)
     cg.bind_pressure_mesh(pr, pm)
