@@ -19,7 +19,12 @@ pytestmark = pytest.mark.gpu
 # name, cells a side, restart, precision, preconditioner, rtol, tolerance on x
 CASES = [
     ("c1", 2, 30, "fp64", "jacobi", 1e-11, 1e-8),     # 9 rows: one partly filled block
-    ("c1", 22, 30, "fp64", "jacobi", 1e-11, 1e-8),    # 529 rows: two blocks
+    ("c1", 21, 30, "fp64", "jacobi", 1e-11, 1e-8),    # 484 rows: one workgroup, one row a thread
+    ("c1", 22, 30, "fp64", "jacobi", 1e-11, 1e-8),    # 529 rows: more
+    ("c1", 22, 7, "mixed", "none", 1e-9, 1e-6),       # and several cycles
+    ("c1", 45, 32, "fp64", "jacobi", 1e-11, 1e-8),    # 2116 rows: the most
+    ("c1", 47, 30, "fp64", "jacobi", 1e-11, 1e-8),    # 2304 rows: a launch a step
+    ("c1p2", 9, 30, "fp64", "jacobi", 1e-11, 1e-8),   # quadratic triangles, rows sorted by length
     ("c1", 90, 30, "fp64", "jacobi", 1e-11, 1e-8),    # 8281 rows: 17 blocks
     ("c1", 90, 1, "fp64", "jacobi", 1e-9, 1e-6),      # a cycle an iteration
     ("c1", 40, 8, "fp64", "jacobi", 1e-11, 1e-8),     # register bases of 8 and cycles of exactly that
