@@ -56,7 +56,8 @@ struct KrylovWork {
     bool use_sell = false, sell16 = false;
     int nsl = 0;
     int64_t nslot = 0;
-    DevBuf<int32_t> sptr, ssrc, scol32, srows;
+    DevBuf<int32_t> sptr, ssrc, scol32, srows, soff;
+    DevBuf<uint64_t> smask;
     DevBuf<int16_t> scol16;
     DevBuf<double> sval64;
     DevBuf<float> sval32;
@@ -853,7 +854,8 @@ static const float* sell_values(const KrylovWork* k, const float* val) {
 template <typename V, typename CT, typename XV, typename YV>
 static void sell_launch(flgpu_ctx* c, KrylovWork* k, const V* sval, const CT* col, const XV* x, YV* y,
                         const double* bsub, int want_dot, const int* done_flag) {
-    const SellOp<V, CT> m{k->nsl, c->rows, k->sptr.p, c->rowptr.p, col, sval, nullptr, k->srows.p};
+    const SellOp<V, CT> m{k->nsl, c->rows, k->sptr.p, col, sval, nullptr, k->srows.p, k->soff.p,
+                                                    k->smask.p};
     if (want_dot)
         sell_product<V, V, CT, XV, YV, DOT_XY>(c->stream, m, x, y, bsub, nullptr, nullptr, k->part(PART_SPMV), done_flag);
     else
@@ -909,6 +911,8 @@ static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
     k->sptr.release();
     k->ssrc.release();
     k->srows.release();
+    k->soff.release();
+    k->smask.release();
     k->scol16.release();
     k->scol32.release();
     k->sval64.release();
@@ -921,8 +925,10 @@ static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
         if (sell_fill(rp, c->rows, window) > kSellMaxFill) return FLGPU_OK;
     }
     SellHost h;
-    sell_plan(rp, c->h_col.data(), c->rows, nullptr, h, window);
+    sell_plan(rp, c->h_col.data(), c->rows, nullptr, h, window, true);
     if (window) FLGPU_TRY(k->srows.upload(h.rows.data(), h.rows.size(), c->stream));
+    FLGPU_TRY(k->soff.upload(h.off.data(), h.off.size(), c->stream));
+    FLGPU_TRY(k->smask.upload(h.mask.data(), h.mask.size(), c->stream));
     FLGPU_TRY(k->sptr.upload(h.sptr.data(), h.sptr.size(), c->stream));
     FLGPU_TRY(k->ssrc.upload(h.src.data(), h.src.size(), c->stream));
     if (h.use16) FLGPU_TRY(k->scol16.upload(h.c16.data(), h.c16.size(), c->stream));
@@ -1872,37 +1878,19 @@ k_gm_sell(SellOp<V, CT> m, const V* __restrict__ w, V* __restrict__ v, V* __rest
     const double share = gm_share(d.pn, d.nb);
     if (gm_done(d)) return;
     constexpr int WPB = kRowBlock / kSlice;
-    constexpr int U = 8;
-    const int wave = threadIdx.x / kSlice, lane = threadIdx.x % kSlice;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kSlice), lane = threadIdx.x % kSlice;
     const RowBlocks it((m.nsl + WPB - 1) / WPB);
     for (int g = it.b; g < it.hi; g += it.step) {
         const int sl = g * WPB + wave;
         if (sl >= m.nsl) continue;
-        int r0;
-        const int row = sell_row(m, sl, lane, r0);
-        const int base = m.sptr[sl], wd = (m.sptr[sl + 1] - base) / kSlice;
-        const int rc = min(row, m.n - 1), len = row < m.n ? m.rowptr[rc + 1] - m.rowptr[rc] : 0;
+        const SellSlice c = sell_slice(m, sl, lane);
+        const int rc = min(c.row, m.n - 1);
         const V wi = w[rc], di = dinv ? dinv[rc] : (V)1;
-        V acc = (V)0;
-        for (int j0 = 0; j0 < wd; j0 += U) {  // loads batched as in k_sell
-            int cj[U];
-            V av[U], xv[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int slot = base + min(j0 + u, wd - 1) * kSlice + lane;
-                cj[u] = csr_col(m.col, slot, r0);
-                av[u] = m.val[slot];
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) xv[u] = w[cj[u]];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                if (j0 + u < len) acc += av[u] * xv[u];
-        }
+        const V acc = sell_row_sum<V>(m, c, lane, w);
         const double s = gm_scale(share);
-        if (row < m.n) {
-            v[row] = (V)((double)wi * s);
-            y[row] = di * (V)((double)acc * s);
+        if (c.row < m.n) {
+            v[c.row] = (V)((double)wi * s);
+            y[c.row] = di * (V)((double)acc * s);
         }
     }
 }
@@ -2339,28 +2327,11 @@ k_gm_small(SellOp<V, CT> m, size_t ldv, V* __restrict__ Vb, const double* __rest
             w[i] = v;
         }
         __syncthreads();
-        for (int sl = wave; sl < m.nsl; sl += B / 64) {
-            int r0;
-            const int row = sell_row(m, sl, lane, r0);
-            const int base = m.sptr[sl], wd = (m.sptr[sl + 1] - base) / kSlice;
-            const int rc = min(row, n - 1), len = row < n ? m.rowptr[rc + 1] - m.rowptr[rc] : 0;
-            const V di = dinv[rc];
-            V acc = (V)0;
-            constexpr int U = 8;
-            for (int j0 = 0; j0 < wd; j0 += U) {
-                int cj[U];
-                V av[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const int slot = base + min(j0 + u, wd - 1) * kSlice + lane;
-                    cj[u] = csr_col(m.col, slot, r0);
-                    av[u] = m.val[slot];
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (j0 + u < len) acc += av[u] * w[cj[u]];
-            }
-            if (row < n) w2[row] = di * acc;
+        for (int sl = __builtin_amdgcn_readfirstlane(wave); sl < m.nsl; sl += B / 64) {
+            const SellSlice c = sell_slice(m, sl, lane);
+            const V di = dinv[min(c.row, n - 1)];
+            const V acc = sell_row_sum<V>(m, c, lane, (const V*)w);
+            if (c.row < n) w2[c.row] = di * acc;
         }
         __syncthreads();
         V* q = w;
@@ -2523,11 +2494,13 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
         if (sval) {
             const int grid = sell_grid(k->nsl);
             if (k->sell16) {
-                const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol16.p, sval, nullptr, k->srows.p};
+                const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, k->scol16.p, sval, nullptr, k->srows.p, k->soff.p,
+                                                    k->smask.p};
                 hipLaunchKernelGGL((k_gm_sell<V, int16_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
                                    d);
             } else {
-                const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol32.p, sval, nullptr, k->srows.p};
+                const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, k->scol32.p, sval, nullptr, k->srows.p, k->soff.p,
+                                                    k->smask.p};
                 hipLaunchKernelGGL((k_gm_sell<V, int32_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
                                    d);
             }
@@ -2592,10 +2565,12 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
         };
         const bool one = n <= kGmSmallBlock;
         if (k->sell16) {
-            const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol16.p, sval, nullptr, k->srows.p};
+            const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, k->scol16.p, sval, nullptr, k->srows.p, k->soff.p,
+                                                    k->smask.p};
             return one ? launch(&k_gm_small<V, int16_t, true>, op) : launch(&k_gm_small<V, int16_t, false>, op);
         }
-        const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, c->rowptr.p, k->scol32.p, sval, nullptr, k->srows.p};
+        const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, k->scol32.p, sval, nullptr, k->srows.p, k->soff.p,
+                                                    k->smask.p};
         return one ? launch(&k_gm_small<V, int32_t, true>, op) : launch(&k_gm_small<V, int32_t, false>, op);
     };
     for (;;) {

@@ -97,8 +97,9 @@ struct LearnedState {
     bool sell = false, ls16 = false, us16 = false;
     int nsll = 0, nslu = 0;
     int64_t nslotl = 0, nslotu = 0;
-    DevBuf<int32_t> lsp, usp, lss, uss, lsc32, usc32;
+    DevBuf<int32_t> lsp, usp, lss, uss, lsc32, usc32, lso, uso;
     DevBuf<int16_t> lsc16, usc16;
+    DevBuf<uint64_t> lsm, usm;  // diagonal slices: lso/uso offsets, lsm/usm masks
     // factor of the scaled matrix, Gs: FP16 for the mixed solve, FP64 for
     // the FP64 solve; the scaling D is applied by the products
     DevBuf<_Float16> gl16, gu16;
@@ -1219,13 +1220,17 @@ static int lu_prepare(flgpu_ctx* c, LearnedState* s) {
     const char* e = getenv("FLGPU_SPMV");
     s->sell = false;
     if (!(e && std::string(e) == "csr")) {
-        sell_plan(lp.data(), lc.data(), n, ls.data(), hl);
-        sell_plan(up.data(), uc.data(), n, us.data(), hu);
+        sell_plan(lp.data(), lc.data(), n, ls.data(), hl, 0, true);
+        sell_plan(up.data(), uc.data(), n, us.data(), hu, 0, true);
         s->sell = hl.fill((int64_t)lc.size()) <= kSellMaxFillHalf && hu.fill((int64_t)uc.size()) <= kSellMaxFillHalf;
     }
     if (s->sell) {
         FLGPU_TRY(s->lsp.upload(hl.sptr.data(), hl.sptr.size(), c->stream));
         FLGPU_TRY(s->usp.upload(hu.sptr.data(), hu.sptr.size(), c->stream));
+        FLGPU_TRY(s->lso.upload(hl.off.data(), hl.off.size(), c->stream));
+        FLGPU_TRY(s->uso.upload(hu.off.data(), hu.off.size(), c->stream));
+        FLGPU_TRY(s->lsm.upload(hl.mask.data(), hl.mask.size(), c->stream));
+        FLGPU_TRY(s->usm.upload(hu.mask.data(), hu.mask.size(), c->stream));
         FLGPU_TRY(s->lss.upload(hl.src.data(), hl.src.size(), c->stream));
         FLGPU_TRY(s->uss.upload(hu.src.data(), hu.src.size(), c->stream));
         if (hl.use16) FLGPU_TRY(s->lsc16.upload(hl.c16.data(), hl.c16.size(), c->stream));
@@ -1298,8 +1303,8 @@ static void apply_launch_sell(flgpu_ctx* c, LearnedState* s, const HV* gl, const
                               const UC* ucol, const V* r, const V* rt, V* z, V* y, const V* w, double* partials,
                               const int* done) {
     const int n = c->rows;
-    const SellOp<HV, LC> lo{s->nsll, n, s->lsp.p, s->lptr.p, lcol, gl, nullptr};
-    const SellOp<HV, UC> up{s->nslu, n, s->usp.p, s->uptr.p, ucol, gu, s->dsq.p};
+    const SellOp<HV, LC> lo{s->nsll, n, s->lsp.p, lcol, gl, nullptr, nullptr, s->lso.p, s->lsm.p};
+    const SellOp<HV, UC> up{s->nslu, n, s->usp.p, ucol, gu, s->dsq.p, nullptr, s->uso.p, s->usm.p};
     sell_product<V, HV, LC, V, V, DOT_NONE>(c->stream, lo, rt, y, nullptr, nullptr, nullptr, partials, done);
     sell_product<V, HV, UC, V, V, DOT_PC>(c->stream, up, y, z, nullptr, r, w, partials, done);
 }

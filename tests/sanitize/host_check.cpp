@@ -426,6 +426,70 @@ static void check_sell_sorted(int n) {
     for (int v : rows) CHECK(v == 1, "sorted sell row in %d lanes", v);
 }
 
+// Diagonal slices, walked as the kernel does (masks and offsets read up to
+// kSellAhead past a slice): in order and sorted, every entry in one slot,
+// every x index in range, the product bit for bit.  The matrix has a regular
+// part (shared offsets) and, from row `regular` on, rows of scattered columns.
+static int check_sell_diagonal(int n, int regular, bool sorted) {
+    std::mt19937_64 g(n + regular);
+    std::vector<int32_t> rp(n + 1, 0), cl;
+    for (int i = 0; i < n; i++) {
+        std::vector<int32_t> row;
+        if (i < regular) {
+            for (int d : {-31, -5, -1, 0, 1, 5, 31})
+                if (i + d >= 0 && i + d < n && !(sorted && i % 3 == 0 && d % 5 == 0 && d)) row.push_back(i + d);
+        } else {
+            for (int q = 0; q < 6; q++) row.push_back((int32_t)(g() % n));
+            row.push_back(i);
+        }
+        std::sort(row.begin(), row.end());
+        row.erase(std::unique(row.begin(), row.end()), row.end());
+        cl.insert(cl.end(), row.begin(), row.end());
+        rp[i + 1] = (int32_t)cl.size();
+    }
+    std::uniform_real_distribution<double> U(-1.0, 1.0);
+    std::vector<double> val(cl.size()), x(n);
+    for (double& v : val) v = U(g);
+    for (double& v : x) v = U(g);
+    flgpu::SellHost h;
+    const int window = sorted ? flgpu::kSellWindow : 0;
+    flgpu::sell_plan(rp.data(), cl.data(), n, nullptr, h, window, true);
+    std::vector<int> seen(cl.size(), 0), rows(n, 0);
+    int dia = 0;
+    for (int sl = 0; sl < h.nsl; sl++) {
+        const int b = h.sptr[sl], base = b & ~(flgpu::kSlice - 1), w = (h.sptr[sl + 1] - base) / flgpu::kSlice;
+        CHECK((b & (flgpu::kSlice - 2)) == 0, "diagonal sell slice start");
+        dia += b & 1;
+        const int r0 = sorted ? sl / (flgpu::kSellWindow / flgpu::kSlice) * flgpu::kSellWindow : sl * flgpu::kSlice;
+        for (int lane = 0; lane < flgpu::kSlice; lane++) {
+            const int q = sl * flgpu::kSlice + lane, row = sorted ? h.rows[q] : q < n ? q : -1;
+            const int rc = row < 0 ? n - 1 : row;
+            if (row >= 0) rows[row]++;
+            double acc = 0.0, ref = 0.0;
+            for (int j = 0; j < (w + flgpu::kSellAhead - 1) / flgpu::kSellAhead * flgpu::kSellAhead; j++) {
+                const size_t at = (size_t)base / flgpu::kSlice + j;
+                CHECK(at < h.mask.size() && (!(b & 1) || at < h.off.size()), "diagonal sell reads past its arrays");
+                const bool in = j < w && (h.mask[at] >> lane & 1);
+                const size_t slot = (size_t)base + (size_t)std::min(j, w - 1) * flgpu::kSlice + lane;
+                const int cj = b & 1 ? (in ? rc + h.off[at] : rc) : h.use16 ? r0 + h.c16[slot] : h.c32[slot];
+                CHECK(cj >= 0 && cj < n, "diagonal sell column out of range");
+                if (j >= w) continue;
+                CHECK((h.src[slot] >= 0) == in, "diagonal sell mask");
+                if (!in) continue;
+                CHECK(row >= 0 && h.src[slot] >= rp[row] && h.src[slot] < rp[row + 1] && cl[h.src[slot]] == cj,
+                      "diagonal sell entry");
+                seen[h.src[slot]]++;
+                acc += val[h.src[slot]] * x[cj];
+            }
+            for (int k = row < 0 ? 0 : rp[row]; row >= 0 && k < rp[row + 1]; k++) ref += val[k] * x[cl[k]];
+            CHECK(acc == ref, "diagonal sell product");
+        }
+    }
+    for (int v : seen) CHECK(v == 1, "diagonal sell entry in %d slots", v);
+    for (int v : rows) CHECK(v == 1, "diagonal sell row in %d lanes", v);
+    return dia;
+}
+
 int main(int argc, char** argv) {
     const bool gpu = argc > 1 && std::strcmp(argv[1], "--gpu") == 0;
     const Mesh m = kuhn_cube(gpu ? 12 : 6);
@@ -449,7 +513,14 @@ int main(int argc, char** argv) {
     std::printf("host: %d nodes, %d elements, %lld entries, %d colours\n", m.nx, m.nele, (long long)nnz, ncol);
     check_matrixdump(findrm, colm);
     check_sell(findrm, colm);
-    for (int n : {1, 63, 64, 511, 512, 513, 1000, 1537}) check_sell_sorted(n);
+    for (int n : {1, 63, 64, 511, 512, 513, 1000, 1537, 2047, 2048, 2049, 6000}) check_sell_sorted(n);
+    for (bool sorted : {false, true})
+        for (int n : {1, 63, 64, 65, 640, 2047, 2048, 2049, 5000}) {
+            check_sell_diagonal(n, 0, sorted);
+            check_sell_diagonal(n, n / 2, sorted);
+            const int dia = check_sell_diagonal(n, n, sorted);
+            CHECK(n < 640 || dia > n / flgpu::kSlice / 2, "only %d diagonal slices", dia);
+        }
     check_oracle(m, findrm, colm, centrm);
     if (gpu) check_gpu(m, findrm, colm, centrm);
     std::printf("%s\n", failures ? "FAILED" : "host_check ok");

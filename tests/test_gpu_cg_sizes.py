@@ -38,3 +38,45 @@ def test_cg_against_oracle(require_gpu, scale):
         x2, info2 = cg.petsc_solve(pr, so)
         assert np.array_equal(x, x2) and info2.its == info.its  # fixed order of every sum
     pr.close()
+
+
+def renumbered(cfg, seed):
+    """The linear mesh with its nodes numbered at random: rows share no
+    column offsets, so the products keep their column indices."""
+    m = cfg.mesh
+    perm = np.random.default_rng(seed).permutation(m.nnodes)  # old node -> new
+    inv = np.argsort(perm)
+    assert np.array_equal(m.ndglno, m.ndglno_x)
+    m.ndglno = (perm[m.ndglno - 1] + 1).astype(m.ndglno.dtype)
+    m.ndglno_x = m.ndglno.copy()
+    m.X, m.node_pos = m.X[inv].copy(), m.node_pos[inv].copy()
+    m.boundary = np.sort(perm[m.boundary - 1] + 1).astype(m.boundary.dtype)
+    cfg.T = cfg.T[inv].copy()
+    if cfg.U is not None:
+        cfg.U = cfg.U[inv].copy()
+    return cfg
+
+
+# rows in order with and without shared column offsets, and quadratic rows
+# sorted in one window, at a window's 2048 rows and over several.  The
+# quadratic systems are mass-dominated: condition numbers below 1e3.
+@pytest.mark.parametrize("name,scale,shuffle", [("c2", 3, True), ("c2", 13, True), ("c2", 13, False),
+                                                ("c3", 5, False), ("c3", 7, False), ("c3", 9, False)])
+def test_products_by_numbering(require_gpu, name, scale, shuffle):
+    cfg = M.config(name, seed=29, scale=scale)
+    if shuffle:
+        cfg = renumbered(cfg, 5)
+    print(f"\n[case] {name} rows {cfg.mesh.nnodes} shuffled {shuffle}", flush=True)
+    ref = O.reference_system(cfg)
+    meth = "cg" if name == "c2" else "gmres"
+    xr, _, reason, _, _ = O.petsc_solve(meth, "jacobi", 1e-13, ref["sparsity"], ref["A"], ref["inactive"], ref["rhs"])
+    assert reason > 0
+    pr = cg.problem_from_config(cfg)
+    cg.assemble_advection_diffusion_cg(pr, cg.options_from_config(cfg), cfg.dt)
+    cg.apply_dirichlet_conditions(pr, cfg.mesh.boundary, 0.0, cfg.dt)
+    tol = (0.7 * max(scale, 3) ** 2 if name == "c2" else 1e3) * (1e-10 + 1e-13)
+    for precision in ("fp64", "mixed"):
+        x, info = cg.petsc_solve(pr, cg.SolverOptions(meth, "jacobi", relative_error=1e-10, precision=precision,
+                                                      norm="unpreconditioned" if meth == "cg" else "preconditioned"))
+        assert info.reason > 0 and np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr), precision
+    pr.close()
