@@ -581,6 +581,7 @@ inline bool sell_offsets(const int32_t* rowptr, const int32_t* col, const int32_
 
 inline void sell_plan(const int32_t* rowptr, const int32_t* col, int n, const int32_t* vmap, SellHost& h,
                       int window = 0, bool diagonals = false) {
+    diagonals = diagonals && rowptr[n] < 1 << 30;  // (their extra steps keep within 32-bit slots)
     h.nsl = (n + kSlice - 1) / kSlice;
     h.rows.clear();
     h.off.clear();
@@ -629,10 +630,23 @@ inline void sell_plan(const int32_t* rowptr, const int32_t* col, int n, const in
     }
     h.nslot = h.sptr[h.nsl];
     h.src.assign((size_t)h.nslot, -1);
-    h.c32.assign((size_t)h.nslot, 0);
+    // the columns' width first, so that only one array is written
+    bool fits = true;
+    for (int sl = 0; fits && sl < h.nsl; sl++) {
+        const int r0 = first(sl);
+        for (int lane = 0; !dia[sl] && lane < kSlice; lane++) {
+            const int r = row_of(sl, lane);
+            if (r < 0) continue;
+            bool far = r - r0 > 32767;  // (its padding's column)
+            for (int k = rowptr[r]; k < rowptr[r + 1]; k++) far |= col[k] - r0 < -32768 || col[k] - r0 > 32767;
+            fits = fits && !far;
+        }
+    }
+    h.use16 = fits;
+    h.c16.assign(fits ? (size_t)h.nslot : 0, 0);
+    h.c32.assign(fits ? 0 : (size_t)h.nslot, 0);
     if (!alloff.empty()) h.off.assign((size_t)h.nslot / kSlice + kSellAhead, 0);
     h.mask.assign((size_t)h.nslot / kSlice + kSellAhead, 0);
-    bool fits = true;
     size_t at = 0;
     for (int sl = 0; sl < h.nsl; sl++) {
         const int r0 = first(sl), w = (h.sptr[sl + 1] - h.sptr[sl]) / kSlice;
@@ -657,25 +671,19 @@ inline void sell_plan(const int32_t* rowptr, const int32_t* col, int n, const in
             const int len = r >= 0 ? rowptr[r + 1] - rowptr[r] : 0;
             for (int j = 0; j < w; j++) {
                 const size_t slot = (size_t)h.sptr[sl] + (size_t)j * kSlice + lane;
+                int cj = r >= 0 ? r : r0;
                 if (j < len) {
                     const int k = rowptr[r] + j;
                     h.src[slot] = vmap ? vmap[k] : k;
                     h.mask[slot / kSlice] |= (uint64_t)1 << lane;
-                    h.c32[slot] = col[k];
-                } else {
-                    h.c32[slot] = r >= 0 ? r : r0;
+                    cj = col[k];
                 }
-                const int d = h.c32[slot] - r0;
-                if (d < -32768 || d > 32767) fits = false;
+                if (fits)
+                    h.c16[slot] = (int16_t)(cj - r0);
+                else
+                    h.c32[slot] = cj;
             }
         }
-    }
-    h.use16 = fits;
-    if (fits) {
-        h.c16.assign((size_t)h.nslot, 0);
-        for (int sl = 0; sl < h.nsl; sl++)
-            for (int64_t q = h.sptr[sl]; !dia[sl] && q < h.sptr[sl + 1]; q++) h.c16[q] = (int16_t)(h.c32[q] - first(sl));
-        std::vector<int32_t>().swap(h.c32);
     }
     for (int sl = 0; sl < h.nsl; sl++) h.sptr[sl] |= dia[sl];
 }
