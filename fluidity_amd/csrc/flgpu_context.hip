@@ -7,11 +7,11 @@
 #include <cstdarg>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
 #include "flgpu_internal.h"
+#include "host_stage.h"
 
 namespace flgpu {
 
@@ -35,15 +35,12 @@ unsigned grid_for(int64_t n, int block) {
 // Pinned slots through which large results go to the caller's memory: one
 // set per GPU (12 MiB, allocated at the first large copy), shared by its
 // contexts, one copy at a time, and freed with the last context.
-constexpr size_t kStageSlot = 1 << 20;
-constexpr size_t kStageMin = 4 << 20;              // smaller copies go the runtime's way
-constexpr int kStageThreads = 4, kStageDepth = 3;  // slots in flight per thread
 constexpr int kStageDevices = 64;
 struct HostStage {
     std::mutex mu;
     int users = 0;  // contexts
     unsigned char* buf = nullptr;
-    hipEvent_t ev[kStageThreads * kStageDepth] = {};
+    hipEvent_t ev[kStageSlots] = {};
 };
 static HostStage g_stage[kStageDevices];
 
@@ -66,13 +63,30 @@ static void stage_leave(int device) {
     st.buf = nullptr;
 }
 
-// A large copy to pageable memory goes through pinned slots, each thread
-// taking every T-th megabyte: the transfer (55 GB/s into pinned memory) then
-// overlaps the copies to the destination, and several threads share the page
-// faults of memory the caller has just allocated.  The runtime's own copy
-// pins such pages first.  32 MB: 1.9 -> 1.1 ms, 122 MB of fresh memory 11.8
-// -> 4.1 ms; 4 MB and less gain nothing.  With the slots taken by another
-// thread's copy, the runtime's.
+// The runtime's part of a copy through the slots.
+struct StageIo {
+    using Err = hipError_t;
+    flgpu_ctx* c;
+    HostStage& st;
+    const unsigned char* src;
+    Err begin() { return hipSetDevice(c->device); }
+    Err queue(int s, size_t at, size_t len) {
+        const Err e = hipMemcpyAsync(slot(s), src + at, len, hipMemcpyDeviceToHost, c->stream);
+        return e == hipSuccess ? hipEventRecord(st.ev[s], c->stream) : e;
+    }
+    Err wait(int s) { return hipEventSynchronize(st.ev[s]); }
+    void drain() { (void)hipStreamSynchronize(c->stream); }
+    unsigned char* slot(int s) { return st.buf + (size_t)s * kStageSlot; }
+    template <typename F>
+    std::thread thread(F f) {
+        return std::thread(f);
+    }
+};
+
+// A large copy to pageable memory goes through pinned slots (staged_copy).
+// The runtime's own copy pins such pages first.  32 MB: 1.9 -> 1.1 ms, 122 MB
+// of fresh memory 11.8 -> 4.1 ms; 4 MB and less gain nothing.  With the slots
+// taken by another thread's copy, the runtime's.
 int copy_out(flgpu_ctx* c, void* dst, const void* src, size_t bytes) {
     std::unique_lock<std::mutex> lk;
     if (bytes > kStageMin && c->device < kStageDevices)
@@ -82,45 +96,11 @@ int copy_out(flgpu_ctx* c, void* dst, const void* src, size_t bytes) {
         return FLGPU_OK;
     }
     HostStage& st = g_stage[c->device];
-    constexpr int kSlots = kStageThreads * kStageDepth;
-    if (!st.buf) FLGPU_HIP(hipHostMalloc((void**)&st.buf, kStageSlot * kSlots, hipHostMallocDefault));
+    if (!st.buf) FLGPU_HIP(hipHostMalloc((void**)&st.buf, kStageSlot * kStageSlots, hipHostMallocDefault));
     for (hipEvent_t& e : st.ev)
         if (!e) FLGPU_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    const int64_t nch = (int64_t)((bytes + kStageSlot - 1) / kStageSlot);
-    const int T = (int)std::min<int64_t>(kStageThreads, (nch + 1) / 2);
-    hipError_t err[kStageThreads] = {};
-    auto size = [&](int64_t ch) { return std::min(kStageSlot, bytes - (size_t)ch * kStageSlot); };
-    auto work = [&](int t) {
-        auto slot = [&](int64_t q) { return t * kStageDepth + (int)(q % kStageDepth); };
-        hipError_t e = hipSetDevice(c->device);
-        const int64_t mine = (nch - t + T - 1) / T;
-        for (int64_t q = 0; q < mine + kStageDepth - 1 && e == hipSuccess; q++) {
-            if (q < mine) {  // queue chunk q of this thread
-                const int64_t ch = t + q * T;
-                e = hipMemcpyAsync(st.buf + slot(q) * kStageSlot, (const unsigned char*)src + ch * kStageSlot, size(ch),
-                                   hipMemcpyDeviceToHost, c->stream);
-                if (e == hipSuccess) e = hipEventRecord(st.ev[slot(q)], c->stream);
-            }
-            const int64_t r = q - (kStageDepth - 1);
-            if (r >= 0 && r < mine && e == hipSuccess) {  // and take the one queued kStageDepth - 1 before it
-                const int64_t ch = t + r * T;
-                e = hipEventSynchronize(st.ev[slot(r)]);
-                if (e == hipSuccess)
-                    std::memcpy((unsigned char*)dst + ch * kStageSlot, st.buf + slot(r) * kStageSlot, size(ch));
-            }
-        }
-        err[t] = e;
-    };
-    std::thread pool[kStageThreads];
-    int started = 1;
-    try {
-        for (; started < T; started++) pool[started] = std::thread(work, started);
-    } catch (const std::system_error&) {  // no more threads: this one takes their share
-    }
-    work(0);
-    for (int t = 1; t < started; t++) pool[t].join();
-    for (int t = started; t < T; t++) work(t);
-    for (int t = 0; t < T; t++) FLGPU_HIP(err[t]);
+    StageIo io{c, st, (const unsigned char*)src};
+    FLGPU_HIP(staged_copy(io, dst, bytes));
     return FLGPU_OK;
 }
 

@@ -4,6 +4,7 @@
 // tests/test_host_sanitizers.py on the CPU:
 //   - make_sparsity and colour_mesh on a jittered-free Kuhn cube mesh;
 //   - the sliced ELL plan of the solver's SpMV against its CSR source;
+//   - copies through the pinned slots with a transfer or a wait that fails;
 //   - the matrix-dump writer and reader, then the reader on every
 //     truncation of a dump and on dumps with corrupted headers, counts,
 //     row lengths and column indices (each must fail cleanly or succeed);
@@ -19,9 +20,12 @@
 #include <cstdlib>
 #include <cstring>
 #include <random>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
+#include "../../fluidity_amd/csrc/host_stage.h"
 #include "../../fluidity_amd/csrc/krylov_common.h"
 #include "../../include/flgpu.h"
 #include "../../oracle/fl_oracle.h"
@@ -490,6 +494,80 @@ static int check_sell_diagonal(int n, int regular, bool sorted) {
     return dia;
 }
 
+// A stream that carries its transfers out in order and no sooner than it
+// has to: when a slot is waited for, or all of them are.  `fail` >= 0 makes
+// the fail-th queue (or, past 1000, the fail-1000th wait) an error.
+struct FakeIo {
+    using Err = int;
+    struct Transfer {
+        int slot;
+        size_t at, len;
+    };
+    const std::vector<unsigned char>& src;
+    int fail = -1;
+    int queued = 0, waited = 0;
+    std::mutex mu;
+    std::vector<Transfer> pending;
+    std::vector<unsigned char> slots = std::vector<unsigned char>(flgpu::kStageSlot * flgpu::kStageSlots);
+    explicit FakeIo(const std::vector<unsigned char>& s) : src(s) {}
+    void carry_out(size_t n) {
+        for (size_t q = 0; q < n; q++) std::memcpy(slot(pending[q].slot), &src[pending[q].at], pending[q].len);
+        pending.erase(pending.begin(), pending.begin() + n);
+    }
+    Err begin() { return 0; }
+    Err queue(int s, size_t at, size_t len) {
+        std::lock_guard<std::mutex> lk(mu);
+        if (queued++ == fail) return 7;
+        pending.push_back({s, at, len});
+        return 0;
+    }
+    Err wait(int s) {
+        std::lock_guard<std::mutex> lk(mu);
+        if (1000 + waited++ == fail) return 8;
+        for (size_t q = 0; q < pending.size(); q++)
+            if (pending[q].slot == s) {
+                carry_out(q + 1);
+                return 0;
+            }
+        return 0;
+    }
+    void drain() {
+        std::lock_guard<std::mutex> lk(mu);
+        carry_out(pending.size());
+    }
+    unsigned char* slot(int s) { return &slots[(size_t)s * flgpu::kStageSlot]; }
+    template <typename F>
+    std::thread thread(F f) {
+        return std::thread(f);
+    }
+};
+
+static std::vector<unsigned char> stage_bytes(size_t n) {
+    std::vector<unsigned char> v(n);
+    for (size_t q = 0; q < n; q++) v[q] = (unsigned char)(q * 2654435761u >> 13);
+    return v;
+}
+
+// Copies of one chunk, of a short last one, and of more chunks than slots
+// arrive whole; when any one transfer or wait fails, the error is returned
+// and no transfer is left that could still write into a slot.
+static void check_stage() {
+    for (size_t bytes : {(size_t)1, flgpu::kStageSlot, 2 * flgpu::kStageSlot + 5, 29 * flgpu::kStageSlot + 17}) {
+        const std::vector<unsigned char> src = stage_bytes(bytes);
+        const int chunks = (int)((bytes + flgpu::kStageSlot - 1) / flgpu::kStageSlot);
+        for (int fail = -1; fail < chunks; fail++)
+            for (int wait = 0; wait < (fail < 0 ? 1 : 2); wait++) {
+                FakeIo io(src);
+                io.fail = fail < 0 ? -1 : fail + 1000 * wait;
+                std::vector<unsigned char> dst(bytes);
+                const int e = flgpu::staged_copy(io, dst.data(), bytes);
+                CHECK(e == (fail < 0 ? 0 : wait ? 8 : 7), "staged copy of %zu bytes: error %d", bytes, e);
+                CHECK(io.pending.empty(), "%zu transfers in flight after a staged copy", io.pending.size());
+                CHECK(fail >= 0 || dst == src, "staged copy of %zu bytes differs", bytes);
+            }
+    }
+}
+
 int main(int argc, char** argv) {
     const bool gpu = argc > 1 && std::strcmp(argv[1], "--gpu") == 0;
     const Mesh m = kuhn_cube(gpu ? 12 : 6);
@@ -513,6 +591,7 @@ int main(int argc, char** argv) {
     std::printf("host: %d nodes, %d elements, %lld entries, %d colours\n", m.nx, m.nele, (long long)nnz, ncol);
     check_matrixdump(findrm, colm);
     check_sell(findrm, colm);
+    check_stage();
     for (int n : {1, 63, 64, 511, 512, 513, 1000, 1537, 2047, 2048, 2049, 6000}) check_sell_sorted(n);
     for (bool sorted : {false, true})
         for (int n : {1, 63, 64, 65, 640, 2047, 2048, 2049, 5000}) {
