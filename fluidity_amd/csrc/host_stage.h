@@ -14,7 +14,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace flgpu {
@@ -60,7 +60,7 @@ typename Io::Err staged_copy(Io& io, void* dst, size_t bytes) {
     int started = 1;
     try {
         for (; started < T; started++) pool[started] = io.thread([&work, started] { work(started); });
-    } catch (const std::system_error&) {  // no more threads: this one takes their share
+    } catch (const std::exception&) {  // no more threads, or no memory for one: this one takes their share
     }
     work(0);
     for (int t = 1; t < started; t++) pool[t].join();

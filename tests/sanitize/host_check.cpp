@@ -21,7 +21,9 @@
 #include <cstring>
 #include <random>
 #include <mutex>
+#include <new>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -536,9 +538,13 @@ struct FakeIo {
         carry_out(pending.size());
     }
     unsigned char* slot(int s) { return &slots[(size_t)s * flgpu::kStageSlot]; }
+    int threads = 3;          // that can be had
+    bool no_memory = false;   // the next one throws bad_alloc, else system_error
     template <typename F>
     std::thread thread(F f) {
-        return std::thread(f);
+        if (threads-- > 0) return std::thread(f);
+        if (no_memory) throw std::bad_alloc();
+        throw std::system_error(std::make_error_code(std::errc::resource_unavailable_try_again));
     }
 };
 
@@ -566,6 +572,17 @@ static void check_stage() {
                 CHECK(fail >= 0 || dst == src, "staged copy of %zu bytes differs", bytes);
             }
     }
+    // fewer threads than asked for, for either reason: the caller's takes their share
+    const std::vector<unsigned char> src = stage_bytes(29 * flgpu::kStageSlot + 17);
+    for (int threads = 0; threads < 3; threads++)
+        for (bool no_memory : {false, true}) {
+            FakeIo io(src);
+            io.threads = threads;
+            io.no_memory = no_memory;
+            std::vector<unsigned char> dst(src.size());
+            CHECK(flgpu::staged_copy(io, dst.data(), src.size()) == 0 && dst == src,
+                  "staged copy with %d threads", threads);
+        }
 }
 
 int main(int argc, char** argv) {
