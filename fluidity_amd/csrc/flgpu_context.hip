@@ -35,23 +35,20 @@ unsigned grid_for(int64_t n, int block) {
 // Pinned slots through which large results go to the caller's memory: one
 // set per GPU (12 MiB, allocated at the first large copy), shared by its
 // contexts, one copy at a time, and freed with the last context.
-constexpr int kStageDevices = 64;
 struct HostStage {
     std::mutex mu;
     int users = 0;  // contexts
     unsigned char* buf = nullptr;
     hipEvent_t ev[kStageSlots] = {};
 };
-static HostStage g_stage[kStageDevices];
+static HostStage g_stage[kMaxDevices];
 
 static void stage_join(int device) {
-    if (device >= kStageDevices) return;
     std::lock_guard<std::mutex> lk(g_stage[device].mu);
     g_stage[device].users++;
 }
 
 static void stage_leave(int device) {
-    if (device >= kStageDevices) return;
     HostStage& st = g_stage[device];
     std::lock_guard<std::mutex> lk(st.mu);
     if (--st.users > 0) return;
@@ -69,6 +66,15 @@ struct StageIo {
     flgpu_ctx* c;
     HostStage& st;
     const unsigned char* src;
+    Err plain(void* dst, size_t bytes) { return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream); }
+    bool ready() {
+        bool ok = st.buf || hipHostMalloc((void**)&st.buf, kStageSlot * kStageSlots, hipHostMallocDefault) == hipSuccess;
+        if (!ok) st.buf = nullptr;
+        for (hipEvent_t& e : st.ev)
+            if (ok && !e) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        if (!ok) (void)hipGetLastError();  // the launches that follow ask for it
+        return ok;
+    }
     Err begin() { return hipSetDevice(c->device); }
     Err queue(int s, size_t at, size_t len) {
         const Err e = hipMemcpyAsync(slot(s), src + at, len, hipMemcpyDeviceToHost, c->stream);
@@ -83,24 +89,13 @@ struct StageIo {
     }
 };
 
-// A large copy to pageable memory goes through pinned slots (staged_copy).
+// A large copy to pageable memory goes through pinned slots (copy_to_host).
 // The runtime's own copy pins such pages first.  32 MB: 1.9 -> 1.1 ms, 122 MB
-// of fresh memory 11.8 -> 4.1 ms; 4 MB and less gain nothing.  With the slots
-// taken by another thread's copy, the runtime's.
+// of fresh memory 11.8 -> 4.1 ms; 4 MB and less gain nothing.
 int copy_out(flgpu_ctx* c, void* dst, const void* src, size_t bytes) {
-    std::unique_lock<std::mutex> lk;
-    if (bytes > kStageMin && c->device < kStageDevices)
-        lk = std::unique_lock<std::mutex>(g_stage[c->device].mu, std::try_to_lock);
-    if (!lk.owns_lock()) {
-        if (bytes) FLGPU_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-        return FLGPU_OK;
-    }
     HostStage& st = g_stage[c->device];
-    if (!st.buf) FLGPU_HIP(hipHostMalloc((void**)&st.buf, kStageSlot * kStageSlots, hipHostMallocDefault));
-    for (hipEvent_t& e : st.ev)
-        if (!e) FLGPU_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     StageIo io{c, st, (const unsigned char*)src};
-    FLGPU_HIP(staged_copy(io, dst, bytes));
+    FLGPU_HIP(copy_to_host(io, st.mu, dst, bytes));
     return FLGPU_OK;
 }
 

@@ -15,6 +15,7 @@ namespace flgpu {
 constexpr int kMaxLoc = 10;   // P2 tetrahedron
 constexpr int kMaxGi = 11;    // degree-4 tetrahedron rule
 constexpr int kMaxDim = 3;
+constexpr int kMaxDevices = 64;  // GPUs the library keeps state for; flgpu_init refuses others
 
 int set_error(int code, const char* fmt, ...);
 

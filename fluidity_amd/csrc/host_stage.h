@@ -3,6 +3,8 @@
 // slot, waiting for it) is an Io, so that the order can be checked on the
 // host without a GPU:
 //   Err                        an error, Err{} for none
+//   Err plain(dst, bytes)      the runtime's own copy
+//   bool ready()               the slots are there, or could be made
 //   Err begin()                once in every thread, before its transfers
 //   Err queue(slot, at, len)   starts the transfer of len bytes at offset at
 //   Err wait(slot)             waits for the slot's last transfer
@@ -15,6 +17,7 @@
 #include <cstdint>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <thread>
 
 namespace flgpu {
@@ -71,6 +74,18 @@ typename Io::Err staged_copy(Io& io, void* dst, size_t bytes) {
             return err[t];
         }
     return Err{};
+}
+
+// A copy of any size: through the slots, guarded by mu, when it is large and
+// they can be had; the runtime's way when another thread has them or the
+// memory for them is not to be had.
+template <class Io>
+typename Io::Err copy_to_host(Io& io, std::mutex& mu, void* dst, size_t bytes) {
+    if (bytes > kStageMin) {
+        std::unique_lock<std::mutex> lk(mu, std::try_to_lock);
+        if (lk.owns_lock() && io.ready()) return staged_copy(io, dst, bytes);
+    }
+    return bytes ? io.plain(dst, bytes) : typename Io::Err{};
 }
 
 }  // namespace flgpu

@@ -2703,15 +2703,14 @@ void krylov_free(flgpu_ctx* c) {
 // shares that GPU's array, so solves that overlap on one GPU race.
 
 constexpr size_t kNoAllocBytes = (size_t)64 << 20;
-constexpr int kNoAllocDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 static std::mutex g_scratch_mu;
-static unsigned char* g_scratch_ptr[kNoAllocDevices] = {};
+static unsigned char* g_scratch_ptr[kMaxDevices] = {};
 
 int noalloc_setup(int device) {
-    if (device < 0 || device >= kNoAllocDevices)
+    if (device < 0 || device >= kMaxDevices)
         return set_error(FLGPU_EUNSUPPORTED, "flgpu_init: device %d beyond the %d the library tracks", device,
-                         kNoAllocDevices);
+                         kMaxDevices);
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     if (g_scratch_ptr[device]) return FLGPU_OK;
     void* p = nullptr;
@@ -2722,7 +2721,7 @@ int noalloc_setup(int device) {
 }
 
 static unsigned char* noalloc_ptr(int device) {
-    if (device < 0 || device >= kNoAllocDevices) return nullptr;
+    if (device < 0 || device >= kMaxDevices) return nullptr;
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     return g_scratch_ptr[device];
 }

@@ -516,6 +516,14 @@ struct FakeIo {
         for (size_t q = 0; q < n; q++) std::memcpy(slot(pending[q].slot), &src[pending[q].at], pending[q].len);
         pending.erase(pending.begin(), pending.begin() + n);
     }
+    bool have_slots = true;
+    int plain_copies = 0;
+    bool ready() { return have_slots; }
+    Err plain(void* dst, size_t bytes) {
+        plain_copies++;
+        std::memcpy(dst, src.data(), bytes);
+        return 0;
+    }
     Err begin() { return 0; }
     Err queue(int s, size_t at, size_t len) {
         std::lock_guard<std::mutex> lk(mu);
@@ -585,6 +593,27 @@ static void check_stage() {
         }
 }
 
+// Which copies take the slots: the large ones, while nobody else has them and
+// they can be had at all; every other one is the runtime's.
+static void check_stage_route() {
+    const std::vector<unsigned char> src = stage_bytes(flgpu::kStageMin + 9);
+    for (size_t bytes : {(size_t)0, (size_t)100, flgpu::kStageMin, src.size()})
+        for (bool busy : {false, true})
+            for (bool have_slots : {true, false}) {
+                FakeIo io(src);
+                io.have_slots = have_slots;
+                std::mutex mu;
+                std::vector<unsigned char> dst(bytes);
+                std::unique_lock<std::mutex> other(mu, std::defer_lock);
+                if (busy) other.lock();
+                int e = -1;
+                std::thread([&] { e = flgpu::copy_to_host(io, mu, dst.data(), bytes); }).join();
+                const bool staged = bytes > flgpu::kStageMin && !busy && have_slots;
+                CHECK(e == 0 && std::equal(dst.begin(), dst.end(), src.begin()), "copy of %zu bytes", bytes);
+                CHECK((io.queued > 0) == staged && io.plain_copies == (bytes > 0 && !staged), "route of %zu bytes", bytes);
+            }
+}
+
 int main(int argc, char** argv) {
     const bool gpu = argc > 1 && std::strcmp(argv[1], "--gpu") == 0;
     const Mesh m = kuhn_cube(gpu ? 12 : 6);
@@ -609,6 +638,7 @@ int main(int argc, char** argv) {
     check_matrixdump(findrm, colm);
     check_sell(findrm, colm);
     check_stage();
+    check_stage_route();
     for (int n : {1, 63, 64, 511, 512, 513, 1000, 1537, 2047, 2048, 2049, 6000}) check_sell_sorted(n);
     for (bool sorted : {false, true})
         for (int n : {1, 63, 64, 65, 640, 2047, 2048, 2049, 5000}) {
