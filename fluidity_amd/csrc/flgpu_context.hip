@@ -66,6 +66,12 @@ struct StageIo {
     flgpu_ctx* c;
     HostStage& st;
     const unsigned char* src;
+    bool pinned(const void* dst) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, dst) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+        (void)hipGetLastError();  // memory that the runtime does not know: pageable
+        return false;
+    }
     Err plain(void* dst, size_t bytes) { return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream); }
     bool ready() {
         bool ok = st.buf || hipHostMalloc((void**)&st.buf, kStageSlot * kStageSlots, hipHostMallocDefault) == hipSuccess;

@@ -4,6 +4,7 @@
 // host without a GPU:
 //   Err                        an error, Err{} for none
 //   Err plain(dst, bytes)      the runtime's own copy
+//   bool pinned(dst)           the destination is pinned memory
 //   bool ready()               the slots are there, or could be made
 //   Err begin()                once in every thread, before its transfers
 //   Err queue(slot, at, len)   starts the transfer of len bytes at offset at
@@ -77,11 +78,12 @@ typename Io::Err staged_copy(Io& io, void* dst, size_t bytes) {
 }
 
 // A copy of any size: through the slots, guarded by mu, when it is large and
-// they can be had; the runtime's way when another thread has them or the
-// memory for them is not to be had.
+// goes to pageable memory; the runtime's way to pinned memory (one direct
+// transfer), and when another thread has the slots or the memory for them is
+// not to be had.
 template <class Io>
 typename Io::Err copy_to_host(Io& io, std::mutex& mu, void* dst, size_t bytes) {
-    if (bytes > kStageMin) {
+    if (bytes > kStageMin && !io.pinned(dst)) {
         std::unique_lock<std::mutex> lk(mu, std::try_to_lock);
         if (lk.owns_lock() && io.ready()) return staged_copy(io, dst, bytes);
     }

@@ -516,7 +516,8 @@ struct FakeIo {
         for (size_t q = 0; q < n; q++) std::memcpy(slot(pending[q].slot), &src[pending[q].at], pending[q].len);
         pending.erase(pending.begin(), pending.begin() + n);
     }
-    bool have_slots = true;
+    bool have_slots = true, is_pinned = false;
+    bool pinned(const void*) { return is_pinned; }
     int plain_copies = 0;
     bool ready() { return have_slots; }
     Err plain(void* dst, size_t bytes) {
@@ -593,22 +594,23 @@ static void check_stage() {
         }
 }
 
-// Which copies take the slots: the large ones, while nobody else has them and
-// they can be had at all; every other one is the runtime's.
+// Which copies take the slots: the large ones to pageable memory, while nobody
+// else has them and they can be had at all; every other one is the runtime's.
 static void check_stage_route() {
     const std::vector<unsigned char> src = stage_bytes(flgpu::kStageMin + 9);
     for (size_t bytes : {(size_t)0, (size_t)100, flgpu::kStageMin, src.size()})
         for (bool busy : {false, true})
-            for (bool have_slots : {true, false}) {
+            for (int kind = 0; kind < 3; kind++) {
                 FakeIo io(src);
-                io.have_slots = have_slots;
+                io.have_slots = kind != 1;
+                io.is_pinned = kind == 2;
                 std::mutex mu;
                 std::vector<unsigned char> dst(bytes);
                 std::unique_lock<std::mutex> other(mu, std::defer_lock);
                 if (busy) other.lock();
                 int e = -1;
                 std::thread([&] { e = flgpu::copy_to_host(io, mu, dst.data(), bytes); }).join();
-                const bool staged = bytes > flgpu::kStageMin && !busy && have_slots;
+                const bool staged = bytes > flgpu::kStageMin && !busy && kind == 0;
                 CHECK(e == 0 && std::equal(dst.begin(), dst.end(), src.begin()), "copy of %zu bytes", bytes);
                 CHECK((io.queued > 0) == staged && io.plain_copies == (bytes > 0 && !staged), "route of %zu bytes", bytes);
             }

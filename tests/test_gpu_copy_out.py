@@ -73,3 +73,23 @@ def test_cmc_pattern_check(require_gpu, n):
             cg.assemble_masslumped_cmc(pr, f, broken)
     assert np.array_equal(cg.assemble_masslumped_cmc(pr, f, c), good)
     pr.close()
+
+
+def test_pinned_destination(require_gpu):
+    """Memory that the caller has pinned, at an offset too, takes the direct
+    transfer at every size."""
+    import ctypes as C
+    pr, nnz = bound(520)
+    path = next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln)  # the library's runtime
+    hip = C.CDLL(path)
+    p = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(p), C.c_size_t(8 * (nnz + 3)), 0) == 0
+    dst = np.frombuffer((C.c_double * (nnz + 3)).from_address(p.value), np.float64)
+    A = np.random.default_rng(4).standard_normal(nnz)
+    L.check(pr.lib.flgpu_matrix_set(pr.ctx, L.ptr(A), L.ptr(np.zeros(pr.mesh.nnodes)), None), "flgpu_matrix_set")
+    for off in (0, 3):
+        dst[:] = -1.0
+        L.check(pr.lib.flgpu_matrix_get(pr.ctx, C.c_void_p(p.value + 8 * off), None, None), "flgpu_matrix_get")
+        assert np.array_equal(dst[off:off + nnz], A)
+    pr.close()
+    assert hip.hipHostFree(p) == 0
