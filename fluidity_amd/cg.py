@@ -128,6 +128,18 @@ class Sparsity:
         return int(self.colm.size)
 
 
+def _pattern_result(findrm: np.ndarray, colm: np.ndarray, blocks: int = 1) -> np.ndarray:
+    """The array that the values of a pattern are copied to, `blocks` values
+    an entry: as long as the column array, zero past the pattern's entries
+    (the library writes no others)."""
+    written = max(int(findrm[-1]) - 1, 0) if findrm.size else 0
+    if written > colm.size:
+        raise ValueError(f"a pattern of {written} entries with {colm.size} columns")
+    out = np.empty(blocks * colm.size)
+    out[blocks * written:] = 0.0
+    return out
+
+
 def make_sparsity(mesh: Mesh) -> Sparsity:
     """make_sparsity(mesh, mesh) through the library's host helper."""
     lib = L.load()
@@ -289,7 +301,7 @@ class CGProblem:
     # -- system --------------------------------------------------------
     def matrix(self):
         """(A values, rhs, inactive mask) copied from the device."""
-        A = np.empty(self.sparsity.nnz)
+        A = _pattern_result(self.sparsity.findrm, self.sparsity.colm)
         rhs = np.empty(self.mesh.nnodes)
         inact = np.empty(self.mesh.nnodes, np.int32)
         L.check(self.lib.flgpu_matrix_get(self.ctx, L.ptr(A), L.ptr(rhs), L.ptr(inact)), "flgpu_matrix_get")
@@ -507,7 +519,7 @@ def construct_momentum_ct(problem: CGProblem, pm: PressureMesh, integrate_contin
     returns (ct_val (dim, nnz), masslump (velocity nodes))."""
     d = problem.mesh.dim
     rho = np.atleast_1d(np.ascontiguousarray(density, dtype=np.float64))
-    ct = np.empty((d, pm.ct_colm.size))
+    ct = _pattern_result(pm.ct_findrm, pm.ct_colm, d).reshape(d, -1)
     ml = np.empty(problem.mesh.nnodes)
     L.check(problem.lib.flgpu_ct_assemble(problem.ctx, int(integrate_continuity_by_parts), int(rho.size == 1),
                                           L.ptr(rho), L.ptr(ct), L.ptr(ml)), "flgpu_ct_assemble")
@@ -531,7 +543,7 @@ def assemble_masslumped_cmc(problem: CGProblem, cmc_findrm: np.ndarray, cmc_colm
     velocity nodes) or None for 1/masslump in every component."""
     im = None if inverse_masslump is None else np.ascontiguousarray(
         np.asarray(inverse_masslump, np.float64).reshape(problem.mesh.dim, -1).T)
-    out = np.empty(cmc_colm.size)
+    out = _pattern_result(cmc_findrm, cmc_colm)
     L.check(problem.lib.flgpu_cmc_assemble(problem.ctx, None if im is None else L.ptr(im), cmc_findrm.size - 1,
                                            L.ptr(cmc_findrm), L.ptr(cmc_colm), L.ptr(out)), "flgpu_cmc_assemble")
     return out
