@@ -1866,16 +1866,42 @@ __device__ __forceinline__ double gm_scale(double share) {
     return nrm > 0.0 ? 1.0 / nrm : 0.0;
 }
 
+// w / |w| from |w|^2's block sums, in two steps.  The product takes FP32
+// entries scaled by the power of two next to 1 / |w| (exact), so that its
+// range is the matrix's, whatever the units and the size of the residual (a
+// product that left it lost the solve); what remains, between 1/2 and 1, is
+// applied to the row's sum.  FP64 has the range, and takes the whole scale
+// at the end.  Normalising every gathered FP32 entry in FP64 instead: 1% of
+// a step on 104k quadratic rows.
+template <typename V>
+struct GmUnit {
+    double share, s, t;
+    int e;
+    __device__ __forceinline__ explicit GmUnit(double sh) : share(sh), s(0.0), t(0.0), e(0) {}
+    __device__ __forceinline__ void begin() {
+        s = t = gm_scale(share);
+        if (sizeof(V) == 4) {
+            e = __builtin_amdgcn_frexp_exp(s);
+            t = __builtin_amdgcn_ldexp(s, -e);
+        }
+    }
+    __device__ __forceinline__ V operator()(V w) const {  // an entry for the product
+        if constexpr (sizeof(V) == 4) return __builtin_amdgcn_ldexpf(w, e);
+        else return w;
+    }
+    __device__ __forceinline__ V row(V acc) const { return (V)((double)acc * t); }  // its sum
+    __device__ __forceinline__ V entry(V w) const { return (V)((double)w * s); }    // of the basis vector
+};
+
 // v = w / |w| and y = D^-1 A v (D^-1 absent: y = A v) over the slices of the
-// solver matrix.  The row
-// sums are formed from w and scaled at the end, so the norm's block sums are
-// in flight with the first slice.  The kernel holds nothing else: closing the
-// column here took it from 8 to 5 waves a SIMD (15 -> 22 us on 373k rows).
+// solver matrix.  The scale is formed with the first slice's loads in flight.
+// The kernel holds nothing else: closing the column here took it from 8 to 5
+// waves a SIMD (15 -> 22 us on 373k rows).
 template <typename V, typename CT>
 __global__ void __launch_bounds__(kRowBlock)
 k_gm_sell(SellOp<V, CT> m, const V* __restrict__ w, V* __restrict__ v, V* __restrict__ y,
           const V* __restrict__ dinv, GmDev d) {
-    const double share = gm_share(d.pn, d.nb);
+    GmUnit<V> unit(gm_share(d.pn, d.nb));
     if (gm_done(d)) return;
     constexpr int WPB = kRowBlock / kSlice;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kSlice), lane = threadIdx.x % kSlice;
@@ -1886,11 +1912,11 @@ k_gm_sell(SellOp<V, CT> m, const V* __restrict__ w, V* __restrict__ v, V* __rest
         const SellSlice c = sell_slice(m, sl, lane);
         const int rc = min(c.row, m.n - 1);
         const V wi = w[rc], di = dinv ? dinv[rc] : (V)1;
-        const V acc = sell_row_sum<V>(m, c, lane, w);
-        const double s = gm_scale(share);
+        if (c.w == 0) unit.begin();
+        const V acc = sell_row_sum<V>(m, c, lane, w, unit);
         if (c.row < m.n) {
-            v[c.row] = (V)((double)wi * s);
-            y[c.row] = di * (V)((double)acc * s);
+            v[c.row] = unit.entry(wi);
+            y[c.row] = di * unit.row(acc);
         }
     }
 }
@@ -1900,20 +1926,20 @@ template <int L, typename V>
 __global__ void __launch_bounds__(kRowBlock)
 k_gm_csr(int n, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col, const V* __restrict__ val,
          const V* __restrict__ w, V* __restrict__ v, V* __restrict__ y, const V* __restrict__ dinv, GmDev d) {
-    const double share = gm_share(d.pn, d.nb);
+    GmUnit<V> unit(gm_share(d.pn, d.nb));
     if (gm_done(d)) return;
-    const double s = gm_scale(share);
+    unit.begin();
     constexpr int ROWS = kRowBlock / L;
     const int lane = threadIdx.x % L, rloc = threadIdx.x / L;
     for (int grp = blockIdx.x; grp * ROWS < n; grp += gridDim.x) {
         const int row = grp * ROWS + rloc;
         V acc = (V)0;
         if (row < n)
-            for (int k = rowptr[row] + lane; k < rowptr[row + 1]; k += L) acc += val[k] * w[col[k]];
+            for (int k = rowptr[row] + lane; k < rowptr[row + 1]; k += L) acc += val[k] * unit(w[col[k]]);
         for (int off = L >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
         if (row < n && lane == 0) {
-            v[row] = (V)((double)w[row] * s);
-            y[row] = (dinv ? dinv[row] : (V)1) * (V)((double)acc * s);
+            v[row] = unit.entry(w[row]);
+            y[row] = (dinv ? dinv[row] : (V)1) * unit.row(acc);
         }
     }
 }
@@ -2330,7 +2356,8 @@ k_gm_small(SellOp<V, CT> m, size_t ldv, V* __restrict__ Vb, const double* __rest
         for (int sl = __builtin_amdgcn_readfirstlane(wave); sl < m.nsl; sl += B / 64) {
             const SellSlice c = sell_slice(m, sl, lane);
             const V di = dinv[min(c.row, n - 1)];
-            const V acc = sell_row_sum<V>(m, c, lane, (const V*)w);
+            SellX fx;
+            const V acc = sell_row_sum<V>(m, c, lane, (const V*)w, fx);
             if (c.row < n) w2[c.row] = di * acc;
         }
         __syncthreads();

@@ -414,13 +414,23 @@ __device__ __forceinline__ SellSlice sell_slice(const SellOp<AV, CT>& m, int sl,
     return s;
 }
 
+// What a product takes of x: the values as they are, or (GMRES) scaled ones,
+// the scale formed by begin() while the first step's loads are in flight.
+struct SellX {
+    __device__ __forceinline__ void begin() {}
+    template <typename V>
+    __device__ __forceinline__ V operator()(V v) const {
+        return v;
+    }
+};
+
 // The lane's row sum: its products in entry order, each rounded before the
 // addition (no contraction), the same sums as k_csr_stream.  Every load is
 // unconditional (a step past the slice's width re-reads its last slot,
 // padding holds an in-range column), so the U loads of a step are all in
 // flight together; only the additions are predicated.
-template <typename V, typename AV, typename CT, typename XV>
-__device__ __forceinline__ V sell_row_sum(const SellOp<AV, CT>& m, const SellSlice& s, int lane, const XV* x) {
+template <typename V, typename AV, typename CT, typename XV, typename F>
+__device__ __forceinline__ V sell_row_sum(const SellOp<AV, CT>& m, const SellSlice& s, int lane, const XV* x, F& fx) {
 #pragma clang fp contract(off)
     // (past a slice's last step: the next slice's, or the arrays' padding)
     const uint64_t* mask = m.mask + s.base / kSlice;
@@ -441,9 +451,10 @@ __device__ __forceinline__ V sell_row_sum(const SellOp<AV, CT>& m, const SellSli
                 av[u] = m.val[s.base + min(j0 + u, s.w - 1) * kSlice + lane];
                 xv[u] = x[in[u] ? rc + d : rc];
             }
+            if (j0 == 0) fx.begin();
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const V pv = (V)av[u] * (V)xv[u];
+                const V pv = (V)av[u] * fx((V)xv[u]);
                 if (in[u]) acc += pv;
             }
         }
@@ -463,9 +474,10 @@ __device__ __forceinline__ V sell_row_sum(const SellOp<AV, CT>& m, const SellSli
         }
 #pragma unroll
         for (int u = 0; u < U; u++) xv[u] = x[cj[u]];
+        if (j0 == 0) fx.begin();
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const V pv = (V)av[u] * (V)xv[u];
+            const V pv = (V)av[u] * fx((V)xv[u]);
             if (in[u]) acc += pv;
         }
     }
@@ -491,7 +503,8 @@ k_sell(SellOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, const dou
         if (sl >= m.nsl) continue;
         const SellSlice s = sell_slice(m, sl, lane);
         if (done) break;  // (after the slice's own loads, which are in flight with the flag's)
-        V acc = sell_row_sum<V>(m, s, lane, x);
+        SellX fx;
+        V acc = sell_row_sum<V>(m, s, lane, x, fx);
         const int row = s.row;
         if (row < m.n) {
             if (m.rs) acc = acc * (V)m.rs[row];

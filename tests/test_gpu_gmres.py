@@ -77,3 +77,33 @@ def test_gmres_iteration_limit_and_zero_rhs(require_gpu):
     x, info = cg.petsc_solve(pr, cg.SolverOptions("gmres", "jacobi", relative_error=1e-10))
     assert info.reason == 3 and info.its == 0 and not np.any(x)
     pr.close()
+
+
+# A matrix scaled by 2^a and a solution by 2^x change no rounding in the
+# solver while nothing leaves the range: the same iterations and exactly the
+# scaled solution, also where the FP32 residual times the matrix would leave
+# it (below 1e-38 once the residual has fallen, above 3e38).
+@pytest.mark.parametrize("n,spmv", [(40, ""), (90, ""), (47, "csr")])
+@pytest.mark.parametrize("a,x", [(-60, -40), (60, 85)])
+def test_mixed_gmres_in_any_units(require_gpu, monkeypatch, n, spmv, a, x):
+    from fluidity_amd import lib as L
+    print(f"\n[case] mixed gmres {n} {spmv} matrix 2^{a} solution 2^{x}", flush=True)
+    if spmv:
+        monkeypatch.setenv("FLGPU_SPMV", spmv)
+    cfg = M.config("c1", seed=17, scale=n)
+    pr = cg.problem_from_config(cfg)
+    cg.assemble_advection_diffusion_cg(pr, cg.options_from_config(cfg), cfg.dt)
+    cg.apply_dirichlet_conditions(pr, cfg.mesh.boundary, 0.0, cfg.dt)
+    so = cg.SolverOptions("gmres", "jacobi", relative_error=1e-9, precision="mixed")
+    A, rhs, inact = pr.matrix()
+    # entries of one size (the prescribed values, taken as they are, zero), so that none is below the range by itself
+    rhs = np.where(inact != 0, 0.0, np.max(np.abs(rhs)) * np.random.default_rng(3).uniform(0.5, 1.5, rhs.size))
+    for sa, sb in ((0, 0), (a, a + x)):
+        As, bs = np.ldexp(A, sa), np.ldexp(rhs, sb)
+        L.check(pr.lib.flgpu_matrix_set(pr.ctx, L.ptr(As), L.ptr(bs), L.ptr(inact)), "flgpu_matrix_set")
+        got, info = cg.petsc_solve(pr, so)
+        if sa == 0:
+            want, its = got, info.its
+    assert info.reason == 2 and info.its == its
+    assert np.array_equal(got, np.ldexp(want, x))
+    pr.close()
