@@ -900,11 +900,8 @@ static int spmv(flgpu_ctx* c, KrylovWork* k, const V* val, const XV* x, YV* y, c
     return FLGPU_OK;
 }
 
-// The sliced ELL plan of the solver matrix, rows in order when that pads to
-// at most kSellMaxFill times the entries, else sorted by length in windows
-// when that does (FLGPU_SPMV=csr keeps the CSR stream product throughout).
-constexpr double kSellMaxFill = 1.2;
-
+// The sliced ELL plan of the solver matrix, where sell_order gives it one
+// (FLGPU_SPMV=csr keeps the CSR products throughout).
 static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
     const char* e = getenv("FLGPU_SPMV");
     k->use_sell = false;
@@ -919,11 +916,9 @@ static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
     k->sval32.release();
     if (e && std::string(e) == "csr") return FLGPU_OK;
     const int32_t* rp = c->h_rowptr.data();
-    int window = 0;
-    if (sell_fill(rp, c->rows, 0) > kSellMaxFill) {
-        window = kSellWindow;
-        if (sell_fill(rp, c->rows, window) > kSellMaxFill) return FLGPU_OK;
-    }
+    const SellOrder order = sell_order(rp, c->rows);
+    if (order == SELL_NONE) return FLGPU_OK;
+    const int window = order == SELL_SORTED ? kSellWindow : 0;
     SellHost h;
     sell_plan(rp, c->h_col.data(), c->rows, nullptr, h, window, true);
     if (window) FLGPU_TRY(k->srows.upload(h.rows.data(), h.rows.size(), c->stream));
@@ -1099,6 +1094,7 @@ static void colour_rows(int n, const int32_t* rowptr, const int32_t* col, std::v
 // through one CU (about 120 GB/s) plus a barrier per step (0.8 us) costs less
 // than a launch per step (4 us).
 constexpr size_t kSorLds = 128 << 10;
+constexpr int kSorWindow = 2048;  // rows of a colour that are sorted by length together
 
 static int ssor_plan(flgpu_ctx* c, KrylovWork* k) {
     if (!c->all_diag) return set_error(FLGPU_EUNSUPPORTED, "sor preconditioner: a row has no diagonal entry");
@@ -1109,11 +1105,11 @@ static int ssor_plan(flgpu_ctx* c, KrylovWork* k) {
     const int ncol = (int)cp.size() - 1;
     for (int q = 0; q < ncol; q++)
         for (int t = cp[q]; t < cp[q + 1]; t++) colour[order[t]] = q;
-    // slices: a colour's rows in order, longest first inside windows of kSellWindow
+    // slices: a colour's rows in order, longest first inside windows of kSorWindow
     k->mc_ptr.assign(1, 0);
     for (int q = 0; q < ncol; q++) {
-        for (int t = cp[q]; t < cp[q + 1]; t += kSellWindow)
-            std::stable_sort(order.begin() + t, order.begin() + std::min(cp[q + 1], t + kSellWindow),
+        for (int t = cp[q]; t < cp[q + 1]; t += kSorWindow)
+            std::stable_sort(order.begin() + t, order.begin() + std::min(cp[q + 1], t + kSorWindow),
                              [&](int32_t a, int32_t b) { return rp[a + 1] - rp[a] > rp[b + 1] - rp[b]; });
         rows.insert(rows.end(), order.begin() + cp[q], order.begin() + cp[q + 1]);
         rows.resize((rows.size() + kSlice - 1) / kSlice * kSlice, -1);

@@ -340,13 +340,12 @@ k_csr_stream(CsrOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, cons
 // offsets is one contiguous line per wave, with no row bounds, no LDS and
 // no barrier.  A slice is as wide as its longest row; the slots past a
 // row's end are padding (value 0, column the row itself) and are skipped.
-// Meshes numbered in space-filling order give slices of near-equal rows,
-// so the padding is small.  Where rows of very different length alternate
-// (quadratic elements: 19 to 65 entries, padding 1.53) the rows of a window
-// of kSellWindow are first sorted by length and column offsets: the slice
-// then lists its rows, column indices count from the window's first row, and
-// the padding is 1.02.  sell_fill tells the padding beforehand and the caller
-// keeps the CSR stream product where neither is small.
+// Meshes numbered in space-filling order give slices of near-equal rows, so
+// the padding is small.  Where rows of different length alternate (quadratic
+// elements, unstructured meshes) the rows of a window of kSellWindow are
+// first sorted by length, equal ones in order: the slice then lists its rows,
+// and column indices count from the window's first row.  sell_order says which
+// form a matrix takes, if any.
 //
 // A slice keeps a 64-bit lane mask per step, the rows that have an entry
 // there.
@@ -355,21 +354,21 @@ k_csr_stream(CsrOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, cons
 // extruded meshes) the rows of a slice share their column offsets col - row.
 // A slice whose rows have at most 1/8 more distinct offsets than its longest
 // row has entries keeps one offset per step instead of 64 column indices: 98
-// of 100 slices of linear meshes, 89 of quadratic ones sorted in windows of
-// 2048 (72 in windows of 512).  Its x addresses come from scalar loads, so
-// the x loads leave with the values' (one dependent memory round trip less)
-// and read contiguous lines; 2 of 6 (FP32), 4 (FP16) or 10 (FP64) bytes an
-// entry are not read at all.  A row's entries stay in order: the same sums.
+// of 100 slices of linear lattices, 27 to 62 of quadratic ones sorted by
+// length.  Its x addresses come from scalar loads, so the x loads leave with
+// the values' (one dependent memory round trip less) and read contiguous
+// lines; 2 of 6 (FP32), 4 (FP16) or 10 (FP64) bytes an entry are not read at
+// all.  A row's entries stay in order: the same sums.
 // Against column indices: 1.37M rows FP64 33.6 -> 27.9 us, FP32 20.3 -> 18.1
 // us, a factor's FP16 halves 13.5 and 15.8 -> 10.5 and 12.6 us (of which the
-// masks in place of row lengths made 1 us); 275k rows FP64 10.7 -> 7.7 us;
-// quadratic, 531k rows, 37.8 -> 34.2 and 27.8 -> 23.0 us.  1/8 more steps
-// cost at most 1 byte an entry (FP64), half of what its index takes.  Slices
-// of unstructured numberings find no shared offsets and keep their indices.
+// masks in place of row lengths made 1 us); 275k rows FP64 10.7 -> 7.7 us.
+// 1/8 more steps cost at most 1 byte an entry (FP64), half of what its index
+// takes.  Slices of unstructured numberings find no shared offsets and keep
+// their indices.
 // Slower: 12 or 16 steps in flight (8 here), values loaded past the caches
 // (28 -> 41 us), the next slice's bounds fetched early (no gain).
 constexpr int kSlice = 64;
-constexpr int kSellWindow = 2048;
+constexpr int kSellWindow = 256;
 constexpr int kSellAhead = 8;  // masks and offsets read past the last slice's
 
 template <typename AV, typename CT>
@@ -549,6 +548,35 @@ inline double sell_fill(const int32_t* rowptr, int n, int window) {
     return n > 0 && rowptr[n] > 0 ? (double)slots / (double)rowptr[n] : 1.0;
 }
 
+// The form that a matrix's products take.  In order where that pads to at
+// most kSellMaxFill times the entries; sorted where that does and either
+//   - the order itself pads to at most 1.75: linear tetrahedra and triangles
+//     of unstructured meshes (1.30 to 1.37), quadratic elements of lattices
+//     (1.28 to 1.68), whose rows move little; or
+//   - the matrix has at most a million entries: then every x is near, and the
+//     CSR product is bound by its chain of barriers (8.5 us) and not by loads;
+// and the CSR stream product otherwise.  Quadratic elements of unstructured
+// meshes pad to 2.07 (triangles) and 2.98 (tetrahedra) in order; sorted, the
+// rows of a slice come from all over the window and no two lanes share a line
+// of x.  CSR against sorted slices, FP64 and FP32: linear tetrahedra, 301k
+// rows, 18.7 and 16.0 -> 15.0 and 11.1 us, 804k rows 35.8 and 32.9 -> 34.4
+// and 25.7; a lattice's quadratic ones, 531k rows, 41.0 and 38.8 -> 34.7 and
+// 25.1; quadratic triangles, 40k rows, 9.0 and 9.0 -> 5.0 and 4.8, but 1.2M
+// rows 36.4 and 32.8 -> 41.0 and 31.7, numbered at random 398k rows 28.4 and
+// 25.0 -> 36.8 and 28.5.  Windows of 512 and 2048 keep more of the tetrahedra
+// within the padding and are slower: unstructured quadratic ones, 223k rows,
+// CSR 23.4 and 22.4, sorted 30.8 and 24.2, and 54.2 and 37.0 us; linear ones,
+// 804k rows, 36.5 and 25.9, and 49.0 and 32.0 us.
+constexpr double kSellMaxFill = 1.2;
+enum SellOrder { SELL_NONE, SELL_IN_ORDER, SELL_SORTED };
+
+inline SellOrder sell_order(const int32_t* rowptr, int n) {
+    const double fill = sell_fill(rowptr, n, 0);
+    if (fill <= kSellMaxFill) return SELL_IN_ORDER;
+    if (fill > 1.75 && rowptr[n] > 1000000) return SELL_NONE;
+    return sell_fill(rowptr, n, kSellWindow) <= kSellMaxFill ? SELL_SORTED : SELL_NONE;
+}
+
 // Host-side plan of a sliced ELL operand: slot offsets, column indices
 // (int16 offsets from the slice's first row, or its window's, when they all
 // fit) and, per slot, the entry of the source value array it takes (vmap[k]
@@ -600,21 +628,11 @@ inline void sell_plan(const int32_t* rowptr, const int32_t* col, int n, const in
     h.off.clear();
     h.mask.clear();
     if (window) {
-        // by length, then by column offsets (a hash of them), then in order
-        std::vector<uint64_t> key((size_t)n);
-        for (int r = 0; r < n; r++) {
-            uint64_t k = 0;
-            for (int e = rowptr[r]; diagonals && e < rowptr[r + 1]; e++)
-                k = (k ^ (uint64_t)(uint32_t)(col[e] - r)) * 0x9E3779B97F4A7C15ull;
-            key[r] = k;
-        }
         h.rows.assign((size_t)h.nsl * kSlice, -1);
         for (int r = 0; r < n; r++) h.rows[r] = r;
         for (int w0 = 0; w0 < n; w0 += window)
-            std::stable_sort(h.rows.begin() + w0, h.rows.begin() + std::min(n, w0 + window), [&](int32_t a, int32_t b) {
-                const int la = rowptr[a + 1] - rowptr[a], lb = rowptr[b + 1] - rowptr[b];
-                return la != lb ? la > lb : key[a] < key[b];
-            });
+            std::stable_sort(h.rows.begin() + w0, h.rows.begin() + std::min(n, w0 + window),
+                             [&](int32_t a, int32_t b) { return rowptr[a + 1] - rowptr[a] > rowptr[b + 1] - rowptr[b]; });
     }
     auto row_of = [&](int sl, int lane) {
         const int q = sl * kSlice + lane;

@@ -432,6 +432,28 @@ static void check_sell_sorted(int n) {
     for (int v : rows) CHECK(v == 1, "sorted sell row in %d lanes", v);
 }
 
+// Which form a matrix takes, from its row lengths: rows of one length in
+// order; of alternating lengths sorted while that moves rows little or the
+// matrix is small; of very different lengths, and above a million entries of
+// moderately different ones, not sliced.
+static void check_sell_order() {
+    auto order = [](int n, std::vector<int> lens) {
+        std::vector<int32_t> rp(n + 1, 0);
+        for (int i = 0; i < n; i++) rp[i + 1] = rp[i] + lens[i % lens.size()];
+        return flgpu::sell_order(rp.data(), n);
+    };
+    CHECK(order(1000, {15}) == flgpu::SELL_IN_ORDER, "equal rows");
+    CHECK(order(500000, {13, 15, 17}) == flgpu::SELL_IN_ORDER, "near-equal rows");
+    const std::vector<int> moderate = {10, 10, 16}, wide = {9, 9, 9, 25};  // 1.33 and 1.92 times in order
+    for (int n : {3000, 80000, 500000}) CHECK(order(n, moderate) == flgpu::SELL_SORTED, "moderately different rows, %d", n);
+    CHECK(order(76923, wide) == flgpu::SELL_SORTED, "999987 entries");
+    CHECK(order(76924, wide) == flgpu::SELL_NONE, "1000012 entries");
+    CHECK(order(500000, wide) == flgpu::SELL_NONE, "very different rows");
+    std::vector<int> lens;
+    for (int q = 0; q < 256; q++) lens.push_back(q < 230 ? 5 : 150);  // a window's mean slice pads 2.6 times
+    CHECK(order(256, lens) == flgpu::SELL_NONE, "few long rows in a small matrix");
+}
+
 // Diagonal slices, walked as the kernel does (masks and offsets read up to
 // kSellAhead past a slice): in order and sorted, every entry in one slot,
 // every x index in range, the product bit for bit.  The matrix has a regular
@@ -639,6 +661,7 @@ int main(int argc, char** argv) {
     std::printf("host: %d nodes, %d elements, %lld entries, %d colours\n", m.nx, m.nele, (long long)nnz, ncol);
     check_matrixdump(findrm, colm);
     check_sell(findrm, colm);
+    check_sell_order();
     check_stage();
     check_stage_route();
     for (int n : {1, 63, 64, 511, 512, 513, 1000, 1537, 2047, 2048, 2049, 6000}) check_sell_sorted(n);

@@ -80,3 +80,30 @@ def test_products_by_numbering(require_gpu, name, scale, shuffle):
                                                       norm="unpreconditioned" if meth == "cg" else "preconditioned"))
         assert info.reason > 0 and np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr), precision
     pr.close()
+
+
+# Quadratic elements numbered at random on both sides of a million entries:
+# rows sorted into slices, and the CSR products.
+@pytest.mark.parametrize("scale", [15, 17])  # 29791 rows of 807661 entries; 42875 rows of 1170281
+def test_quadratic_products_numbered_at_random(require_gpu, scale):
+    cfg = M.config("c3", seed=31, scale=scale)
+    m = cfg.mesh
+    perm = np.random.default_rng(7).permutation(m.nnodes)
+    inv = np.argsort(perm)
+    m.ndglno = (perm[m.ndglno - 1] + 1).astype(m.ndglno.dtype)
+    m.node_pos = m.node_pos[inv].copy()
+    m.boundary = np.sort(perm[m.boundary - 1] + 1).astype(m.boundary.dtype)
+    cfg.T, cfg.U = cfg.T[inv].copy(), cfg.U[inv].copy()
+    print(f"\n[case] c3 numbered at random, rows {m.nnodes}", flush=True)
+    ref = O.reference_system(cfg)
+    xr, _, reason, _, _ = O.petsc_solve("gmres", "jacobi", 1e-13, ref["sparsity"], ref["A"], ref["inactive"],
+                                        ref["rhs"])
+    assert reason > 0
+    pr = cg.problem_from_config(cfg)
+    cg.assemble_advection_diffusion_cg(pr, cg.options_from_config(cfg), cfg.dt)
+    cg.apply_dirichlet_conditions(pr, cfg.mesh.boundary, 0.0, cfg.dt)
+    for precision in ("fp64", "mixed"):
+        x, info = cg.petsc_solve(pr, cg.SolverOptions("gmres", "jacobi", relative_error=1e-10, precision=precision))
+        # mass-dominated: condition numbers below 1e3
+        assert info.reason > 0 and np.linalg.norm(x - xr) <= 1e3 * 1e-10 * np.linalg.norm(xr), precision
+    pr.close()
