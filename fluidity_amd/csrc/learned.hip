@@ -1158,9 +1158,6 @@ int learned_prepare(flgpu_ctx* c, bool mixed, bool fsai) {
 
 // Compact lower/upper CSR of A's pattern (positions into A for the values)
 // and their stream row blocks; rebuilt when the sparsity changes.
-// The factor halves take the sliced ELL product when each pads at most this much.
-constexpr double kSellMaxFillHalf = 1.2;
-
 static int lu_prepare(flgpu_ctx* c, LearnedState* s) {
     if (s->lu_key == c->sparsity_gen) return FLGPU_OK;
     const int n = c->rows;
@@ -1215,16 +1212,14 @@ static int lu_prepare(flgpu_ctx* c, LearnedState* s) {
     s->u16 = compress_columns(up.data(), uc.data(), rbu, u16);
     if (s->l16) FLGPU_TRY(s->lcol16.upload(l16.data(), l16.size(), c->stream));
     if (s->u16) FLGPU_TRY(s->ucol16.upload(u16.data(), u16.size(), c->stream));
-    // sliced ELL plans of both halves, the slots mapped to the factor's entries
+    // sliced ELL plans of both halves when both fit in order, the slots mapped
+    // to the factor's entries
     SellHost hl, hu;
     const char* e = getenv("FLGPU_SPMV");
-    s->sell = false;
-    if (!(e && std::string(e) == "csr")) {
+    s->sell = !(e && std::string(e) == "csr") && sell_fits(lp.data(), n) && sell_fits(up.data(), n);
+    if (s->sell) {
         sell_plan(lp.data(), lc.data(), n, ls.data(), hl, 0, true);
         sell_plan(up.data(), uc.data(), n, us.data(), hu, 0, true);
-        s->sell = hl.fill((int64_t)lc.size()) <= kSellMaxFillHalf && hu.fill((int64_t)uc.size()) <= kSellMaxFillHalf;
-    }
-    if (s->sell) {
         FLGPU_TRY(s->lsp.upload(hl.sptr.data(), hl.sptr.size(), c->stream));
         FLGPU_TRY(s->usp.upload(hu.sptr.data(), hu.sptr.size(), c->stream));
         FLGPU_TRY(s->lso.upload(hl.off.data(), hl.off.size(), c->stream));

@@ -454,6 +454,23 @@ static void check_sell_order() {
     CHECK(order(256, lens) == flgpu::SELL_NONE, "few long rows in a small matrix");
 }
 
+// Diagonal slices may pad a matrix past the limit that its rows keep within:
+// it is sliced all the same.
+static void check_sell_fits_by_rows() {
+    const int n = 6400;
+    std::vector<int32_t> rp(n + 1, 0), cl;
+    for (int i = 0; i < n; i++) {  // 9 of 9 or 10 shared offsets; a fifth of the rows has 4
+        const int len = i % 5 ? 9 : 4, skip = i % 64 % 10;
+        for (int d = 0, k = 0; d < 10 && k < len; d++)
+            if (d != skip && i + 3 * d < n) cl.push_back(i + 3 * d), k++;
+        rp[i + 1] = (int32_t)cl.size();
+    }
+    flgpu::SellHost h;
+    flgpu::sell_plan(rp.data(), cl.data(), n, nullptr, h, 0, true);
+    CHECK(h.fill((int64_t)cl.size()) > flgpu::kSellMaxFill, "diagonal padding %.3f", h.fill((int64_t)cl.size()));
+    CHECK(flgpu::sell_fits(rp.data(), n), "rows' padding %.3f", flgpu::sell_fill(rp.data(), n, 0));
+}
+
 // Diagonal slices, walked as the kernel does (masks and offsets read up to
 // kSellAhead past a slice): in order and sorted, every entry in one slot,
 // every x index in range, the product bit for bit.  The matrix has a regular
@@ -662,6 +679,7 @@ int main(int argc, char** argv) {
     check_matrixdump(findrm, colm);
     check_sell(findrm, colm);
     check_sell_order();
+    check_sell_fits_by_rows();
     check_stage();
     check_stage_route();
     for (int n : {1, 63, 64, 511, 512, 513, 1000, 1537, 2047, 2048, 2049, 6000}) check_sell_sorted(n);
