@@ -808,6 +808,72 @@ k_sor_block(int n, int ncol, const int32_t* __restrict__ cptr, SorOp<V> f, SorOp
     for (int i = threadIdx.x; i < n; i += blockDim.x) z[i] = zs[i];
 }
 
+// The slices of a plan, a thread a slot of 64-row slices (rows: -1 past a
+// colour's last), in two passes over the CSR rows: the entries of each sweep
+// and the slices' widths (in steps), then the entries at their slots.  Built
+// by the host, the plan of 1.37M rows of 15 entries took 240 ms, most of the
+// first solve; so 4 (and 12 for the colouring, which is the host's).
+__global__ void __launch_bounds__(256)
+k_sor_count(int nslot, const int32_t* __restrict__ rows, const int32_t* __restrict__ rowptr,
+            const int32_t* __restrict__ col, const int32_t* __restrict__ colour, int32_t* __restrict__ lenf,
+            int32_t* __restrict__ lenb, int32_t* __restrict__ dsrc, int32_t* __restrict__ wf,
+            int32_t* __restrict__ wb) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nslot) return;  // whole waves
+    const int i = rows[q];
+    int nf = 0, nb = 0, d = -1;
+    if (i >= 0) {
+        const int ci = colour[i];
+        for (int e = rowptr[i]; e < rowptr[i + 1]; e++) {
+            const int j = col[e];
+            if (j == i) d = e;
+            else {
+                nb++;
+                nf += colour[j] < ci;
+            }
+        }
+    }
+    lenf[q] = nf;
+    lenb[q] = nb;
+    dsrc[q] = d;
+    for (int off = 32; off > 0; off >>= 1) {
+        nf = max(nf, __shfl_xor(nf, off, 64));
+        nb = max(nb, __shfl_xor(nb, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        wf[q / kSlice] = nf;
+        wb[q / kSlice] = nb;
+    }
+}
+
+__global__ void __launch_bounds__(256)
+k_sor_fill(int nslot, const int32_t* __restrict__ rows, const int32_t* __restrict__ rowptr,
+           const int32_t* __restrict__ col, const int32_t* __restrict__ colour, const int32_t* __restrict__ ptrf,
+           const int32_t* __restrict__ ptrb, int32_t* __restrict__ colf, int32_t* __restrict__ srcf,
+           int32_t* __restrict__ colb, int32_t* __restrict__ srcb) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nslot) return;
+    const int i = rows[q], sl = q / kSlice;
+    int f = ptrf[sl] + q % kSlice, b = ptrb[sl] + q % kSlice;
+    if (i >= 0) {
+        const int ci = colour[i];
+        for (int e = rowptr[i]; e < rowptr[i + 1]; e++) {
+            const int j = col[e];
+            if (j == i) continue;
+            colb[b] = j;
+            srcb[b] = e;
+            b += kSlice;
+            if (colour[j] < ci) {
+                colf[f] = j;
+                srcf[f] = e;
+                f += kSlice;
+            }
+        }
+    }
+    for (; f < ptrf[sl + 1]; f += kSlice) colf[f] = 0, srcf[f] = -1;
+    for (; b < ptrb[sl + 1]; b += kSlice) colb[b] = 0, srcb[b] = -1;
+}
+
 // Per-block sums r.z, z.z, z.w (w may be null: z.w = 0).
 template <typename V>
 __global__ void __launch_bounds__(kVecBlock)
@@ -1066,8 +1132,9 @@ static int norm_b(flgpu_ctx* c, KrylovWork* k) {
 // takes the smallest colour that none of its columns j < i holds.  Rows are
 // then listed colour by colour, ascending inside a colour.
 static void colour_rows(int n, const int32_t* rowptr, const int32_t* col, std::vector<int32_t>& ptr,
-                 std::vector<int32_t>& rows) {
-    std::vector<int32_t> colour(n, -1), mark;  // mark[q] == i: colour q is taken next to row i
+                        std::vector<int32_t>& rows, std::vector<int32_t>& colour) {
+    std::vector<int32_t> mark;  // mark[q] == i: colour q is taken next to row i
+    colour.assign(n, -1);
     int ncol = 0;
     for (int i = 0; i < n; i++) {
         for (int k = rowptr[i]; k < rowptr[i + 1]; k++) {
@@ -1096,64 +1163,73 @@ static void colour_rows(int n, const int32_t* rowptr, const int32_t* col, std::v
 constexpr size_t kSorLds = 128 << 10;
 constexpr int kSorWindow = 2048;  // rows of a colour that are sorted by length together
 
+// Rows longest first, equal ones in order (a counting sort).
+static void sort_by_length(const int32_t* rowptr, int32_t* rows, int n, std::vector<int32_t>& count,
+                           std::vector<int32_t>& tmp) {
+    int top = 0;
+    for (int t = 0; t < n; t++) top = std::max(top, rowptr[rows[t] + 1] - rowptr[rows[t]]);
+    count.assign((size_t)top + 2, 0);  // count[d + 1]: rows that are d shorter than the longest
+    for (int t = 0; t < n; t++) count[top - (rowptr[rows[t] + 1] - rowptr[rows[t]]) + 1]++;
+    for (int d = 0; d < top; d++) count[d + 1] += count[d];
+    tmp.assign(rows, rows + n);
+    for (int t = 0; t < n; t++) rows[count[top - (rowptr[tmp[t] + 1] - rowptr[tmp[t]])]++] = tmp[t];
+}
+
 static int ssor_plan(flgpu_ctx* c, KrylovWork* k) {
     if (!c->all_diag) return set_error(FLGPU_EUNSUPPORTED, "sor preconditioner: a row has no diagonal entry");
     const int n = c->rows;
+    if (c->cols > n) return set_error(FLGPU_EUNSUPPORTED, "sor preconditioner: a column past the rows");
     const int32_t *rp = c->h_rowptr.data(), *cl = c->h_col.data();
-    std::vector<int32_t> cp, order, colour(n), rows, dsrc, sl_of;
-    colour_rows(n, rp, cl, cp, order);
+    std::vector<int32_t> cp, order, colour, rows, count, tmp;
+    colour_rows(n, rp, cl, cp, order, colour);
     const int ncol = (int)cp.size() - 1;
-    for (int q = 0; q < ncol; q++)
-        for (int t = cp[q]; t < cp[q + 1]; t++) colour[order[t]] = q;
     // slices: a colour's rows in order, longest first inside windows of kSorWindow
     k->mc_ptr.assign(1, 0);
+    rows.reserve((size_t)n + (size_t)ncol * kSlice);
     for (int q = 0; q < ncol; q++) {
         for (int t = cp[q]; t < cp[q + 1]; t += kSorWindow)
-            std::stable_sort(order.begin() + t, order.begin() + std::min(cp[q + 1], t + kSorWindow),
-                             [&](int32_t a, int32_t b) { return rp[a + 1] - rp[a] > rp[b + 1] - rp[b]; });
+            sort_by_length(rp, order.data() + t, std::min(cp[q + 1] - t, kSorWindow), count, tmp);
         rows.insert(rows.end(), order.begin() + cp[q], order.begin() + cp[q + 1]);
         rows.resize((rows.size() + kSlice - 1) / kSlice * kSlice, -1);
         k->mc_ptr.push_back((int32_t)(rows.size() / kSlice));
     }
-    const int nsl = (int)(rows.size() / kSlice);
-    dsrc.assign(rows.size(), -1);
+    const int nslot = (int)rows.size(), nsl = nslot / kSlice;
+    KrylovWork::SorHalf *F = &k->mc_f, *B = &k->mc_b;
+    DevBuf<int32_t> dcolour, width;
+    FLGPU_TRY(dcolour.upload(colour.data(), colour.size(), c->stream));
+    FLGPU_TRY(width.alloc(2 * (size_t)nsl));
+    FLGPU_TRY(k->mc_rows.upload(rows.data(), rows.size(), c->stream));
+    FLGPU_TRY(k->mc_cptr.upload(k->mc_ptr.data(), k->mc_ptr.size(), c->stream));
+    FLGPU_TRY(k->mc_dsrc.alloc(rows.size()));
+    FLGPU_TRY(F->len.alloc(rows.size()));
+    FLGPU_TRY(B->len.alloc(rows.size()));
+    const unsigned grid = grid_for(nslot, 256);
+    hipLaunchKernelGGL(k_sor_count, dim3(grid), dim3(256), 0, c->stream, nslot, k->mc_rows.p, c->rowptr.p, c->col.p,
+                       dcolour.p, F->len.p, B->len.p, k->mc_dsrc.p, width.p, width.p + nsl);
+    FLGPU_HIP(hipGetLastError());
+    std::vector<int32_t> w(2 * (size_t)nsl), ptr[2];
+    FLGPU_HIP(hipMemcpyAsync(w.data(), width.p, sizeof(int32_t) * w.size(), hipMemcpyDeviceToHost, c->stream));
+    FLGPU_HIP(hipStreamSynchronize(c->stream));
     int64_t slots = 0;
     for (int half = 0; half < 2; half++) {
-        KrylovWork::SorHalf& H = half ? k->mc_b : k->mc_f;
-        std::vector<int32_t> ptr(nsl + 1, 0), len(rows.size(), 0), col, src;
-        std::vector<std::vector<int32_t>> ent(kSlice);
+        int64_t at = 0;
+        ptr[half].assign(1, 0);
         for (int sl = 0; sl < nsl; sl++) {
-            int w = 0;
-            for (int lane = 0; lane < kSlice; lane++) {
-                const int q = sl * kSlice + lane, i = rows[q];
-                ent[lane].clear();
-                if (i < 0) continue;
-                for (int e = rp[i]; e < rp[i + 1]; e++) {
-                    if (cl[e] == i) dsrc[q] = e;
-                    else if (half || colour[cl[e]] < colour[i]) ent[lane].push_back(e);
-                }
-                len[q] = (int32_t)ent[lane].size();
-                w = std::max(w, len[q]);
-            }
-            for (int j = 0; j < w; j++)
-                for (int lane = 0; lane < kSlice; lane++) {
-                    const bool in = j < (int)ent[lane].size();
-                    src.push_back(in ? ent[lane][j] : -1);
-                    col.push_back(in ? cl[ent[lane][j]] : 0);
-                }
-            ptr[sl + 1] = (int32_t)col.size();
+            at += (int64_t)w[half * nsl + sl] * kSlice;
+            ptr[half].push_back((int32_t)at);
         }
-        slots += (int64_t)col.size();
-        FLGPU_TRY(H.ptr.upload(ptr.data(), ptr.size(), c->stream));
-        FLGPU_TRY(H.len.upload(len.data(), len.size(), c->stream));
-        FLGPU_TRY(H.col.upload(col.data(), col.size(), c->stream));
-        FLGPU_TRY(H.src.upload(src.data(), src.size(), c->stream));
-        FLGPU_HIP(hipStreamSynchronize(c->stream));  // the vectors are freed here
+        if (at > INT32_MAX)
+            return set_error(FLGPU_EUNSUPPORTED, "sor preconditioner: %lld slots of entries", (long long)at);
+        KrylovWork::SorHalf& H = half ? k->mc_b : k->mc_f;
+        FLGPU_TRY(H.ptr.upload(ptr[half].data(), ptr[half].size(), c->stream));
+        FLGPU_TRY(H.col.alloc((size_t)at));
+        FLGPU_TRY(H.src.alloc((size_t)at));
+        slots += at;
     }
-    FLGPU_TRY(k->mc_rows.upload(rows.data(), rows.size(), c->stream));
-    FLGPU_TRY(k->mc_dsrc.upload(dsrc.data(), dsrc.size(), c->stream));
-    FLGPU_TRY(k->mc_cptr.upload(k->mc_ptr.data(), k->mc_ptr.size(), c->stream));
-    FLGPU_HIP(hipStreamSynchronize(c->stream));
+    hipLaunchKernelGGL(k_sor_fill, dim3(grid), dim3(256), 0, c->stream, nslot, k->mc_rows.p, c->rowptr.p, c->col.p,
+                       dcolour.p, F->ptr.p, B->ptr.p, F->col.p, F->src.p, B->col.p, B->src.p);
+    FLGPU_HIP(hipGetLastError());
+    FLGPU_HIP(hipStreamSynchronize(c->stream));  // the vectors and dcolour are freed here
     const double steps = 2.0 * ncol - 1.0;
     k->mc_one = sizeof(double) * (size_t)n <= kSorLds && 12.0 * (double)slots / 120e3 + 0.8 * steps < 4.0 * steps;
     if (k->mc_one)
