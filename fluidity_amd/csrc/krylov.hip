@@ -986,7 +986,7 @@ static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
     if (order == SELL_NONE) return FLGPU_OK;
     const int window = order == SELL_SORTED ? kSellWindow : 0;
     SellHost h;
-    sell_plan(rp, c->h_col.data(), c->rows, nullptr, h, window, true);
+    sell_plan(rp, c->h_col.data(), c->rows, nullptr, h, window, true, sell_run(c->rows));
     if (window) FLGPU_TRY(k->srows.upload(h.rows.data(), h.rows.size(), c->stream));
     FLGPU_TRY(k->soff.upload(h.off.data(), h.off.size(), c->stream));
     FLGPU_TRY(k->smask.upload(h.mask.data(), h.mask.size(), c->stream));

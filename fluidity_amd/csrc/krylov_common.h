@@ -342,10 +342,10 @@ k_csr_stream(CsrOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, cons
 // row's end are padding (value 0, column the row itself) and are skipped.
 // Meshes numbered in space-filling order give slices of near-equal rows, so
 // the padding is small.  Where rows of different length alternate (quadratic
-// elements, unstructured meshes) the rows of a window of kSellWindow are
-// first sorted by length, equal ones in order: the slice then lists its rows,
-// and column indices count from the window's first row.  sell_order says which
-// form a matrix takes, if any.
+// elements, unstructured meshes) the rows are first sorted by length within
+// runs (sell_run), equal ones in order: the slice then lists its rows, and
+// column indices count from the first row of its window of kSellWindow rows.
+// sell_order says which form a matrix takes, if any.
 //
 // A slice keeps a 64-bit lane mask per step, the rows that have an entry
 // there.
@@ -368,7 +368,8 @@ k_csr_stream(CsrOp<AV, CT> m, const XV* __restrict__ x, YV* __restrict__ y, cons
 // Slower: 12 or 16 steps in flight (8 here), values loaded past the caches
 // (28 -> 41 us), the next slice's bounds fetched early (no gain).
 constexpr int kSlice = 64;
-constexpr int kSellWindow = 256;
+constexpr int kSellWindow = 2048;
+constexpr int kSellRun = 256;
 constexpr int kSellAhead = 8;  // masks and offsets read past the last slice's
 
 template <typename AV, typename CT>
@@ -563,10 +564,13 @@ inline double sell_fill(const int32_t* rowptr, int n, int window) {
 // and 25.7; a lattice's quadratic ones, 531k rows, 41.0 and 38.8 -> 34.7 and
 // 25.1; quadratic triangles, 40k rows, 9.0 and 9.0 -> 5.0 and 4.8, but 1.2M
 // rows 36.4 and 32.8 -> 41.0 and 31.7, numbered at random 398k rows 28.4 and
-// 25.0 -> 36.8 and 28.5.  Windows of 512 and 2048 keep more of the tetrahedra
-// within the padding and are slower: unstructured quadratic ones, 223k rows,
-// CSR 23.4 and 22.4, sorted 30.8 and 24.2, and 54.2 and 37.0 us; linear ones,
-// 804k rows, 36.5 and 25.9, and 49.0 and 32.0 us.
+// 25.0 -> 36.8 and 28.5.  Runs of 512 and 2048 rows keep more of the
+// tetrahedra within the padding and are slower: unstructured quadratic ones,
+// 223k rows, CSR 23.4 and 22.4, sorted 30.8 and 24.2, and 54.2 and 37.0 us;
+// linear ones, 804k rows, 36.5 and 25.9, and 49.0 and 32.0 us.  A matrix of
+// one window is one run: its x is in one CU's cache, and short runs' remainders
+// would pad it past the limit (324 rows: the one-workgroup GMRES cycle, 0.32
+// against 0.57 ms a step, takes slices).
 constexpr double kSellMaxFill = 1.2;
 enum SellOrder { SELL_NONE, SELL_IN_ORDER, SELL_SORTED };
 
@@ -578,11 +582,14 @@ inline bool sell_fits(const int32_t* rowptr, int n, double* fill = nullptr) {
     return f <= kSellMaxFill;
 }
 
+// Rows that are sorted together.
+inline int sell_run(int n) { return n <= kSellWindow ? kSellWindow : kSellRun; }
+
 inline SellOrder sell_order(const int32_t* rowptr, int n) {
     double fill;
     if (sell_fits(rowptr, n, &fill)) return SELL_IN_ORDER;
     if (fill > 1.75 && rowptr[n] > 1000000) return SELL_NONE;
-    return sell_fill(rowptr, n, kSellWindow) <= kSellMaxFill ? SELL_SORTED : SELL_NONE;
+    return sell_fill(rowptr, n, sell_run(n)) <= kSellMaxFill ? SELL_SORTED : SELL_NONE;
 }
 
 // Host-side plan of a sliced ELL operand: slot offsets, column indices
@@ -629,7 +636,7 @@ inline bool sell_offsets(const int32_t* rowptr, const int32_t* col, const int32_
 }
 
 inline void sell_plan(const int32_t* rowptr, const int32_t* col, int n, const int32_t* vmap, SellHost& h,
-                      int window = 0, bool diagonals = false) {
+                      int window = 0, bool diagonals = false, int run = 0) {
     diagonals = diagonals && rowptr[n] < 1 << 30;  // (their extra steps keep within 32-bit slots)
     h.nsl = (n + kSlice - 1) / kSlice;
     h.rows.clear();
@@ -638,8 +645,9 @@ inline void sell_plan(const int32_t* rowptr, const int32_t* col, int n, const in
     if (window) {
         h.rows.assign((size_t)h.nsl * kSlice, -1);
         for (int r = 0; r < n; r++) h.rows[r] = r;
-        for (int w0 = 0; w0 < n; w0 += window)
-            std::stable_sort(h.rows.begin() + w0, h.rows.begin() + std::min(n, w0 + window),
+        if (!run) run = window;
+        for (int w0 = 0; w0 < n; w0 += run)
+            std::stable_sort(h.rows.begin() + w0, h.rows.begin() + std::min(n, w0 + run),
                              [&](int32_t a, int32_t b) { return rowptr[a + 1] - rowptr[a] > rowptr[b + 1] - rowptr[b]; });
     }
     auto row_of = [&](int sl, int lane) {

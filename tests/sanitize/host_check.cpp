@@ -452,6 +452,15 @@ static void check_sell_order() {
     std::vector<int> lens;
     for (int q = 0; q < 256; q++) lens.push_back(q < 230 ? 5 : 150);  // a window's mean slice pads 2.6 times
     CHECK(order(256, lens) == flgpu::SELL_NONE, "few long rows in a small matrix");
+    // triangulated lattices of few rows, whose last run would be mostly padding
+    for (int p : {18, 20, 30, 45}) {
+        std::vector<int> l;
+        for (int j = 0; j < p; j++)
+            for (int i = 0; i < p; i++)
+                l.push_back(1 + (i > 0) + (i + 1 < p) + (j > 0) + (j + 1 < p) + (i > 0 && j > 0) +
+                            (i + 1 < p && j + 1 < p));
+        CHECK(order(p * p, l) != flgpu::SELL_NONE, "lattice of %d rows", p * p);
+    }
 }
 
 // Diagonal slices may pad a matrix past the limit that its rows keep within:
