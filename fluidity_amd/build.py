@@ -35,7 +35,7 @@ EXTRA = {
     "pressure.hip": ["-ffp-contract=off"],
 }
 SOURCES = ["flgpu_context.hip", "assemble.hip", "surface.hip", "krylov.hip", "learned.hip", "matrixdump.hip",
-           "setup_gpu.hip", "pressure.hip"]
+           "setup_gpu.hip", "pressure.hip", "sell_plan.hip"]
 
 
 def _compile(src: str) -> str:

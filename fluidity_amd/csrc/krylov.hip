@@ -30,6 +30,7 @@
 #include "flgpu_internal.h"
 #include "krylov_common.h"
 #include "learned.h"
+#include "sell_plan.h"
 
 namespace flgpu {
 
@@ -52,13 +53,8 @@ struct KrylovWork {
     bool use16 = false;
     int nrb = 0;
     int64_t rb_key = -1;     // sparsity generation rb was built for
-    // sliced ELL copy of the solver matrix, used by spmv when its padding is small
-    bool use_sell = false, sell16 = false;
-    int nsl = 0;
-    int64_t nslot = 0;
-    DevBuf<int32_t> sptr, ssrc, scol32, srows, soff;
-    DevBuf<uint64_t> smask;
-    DevBuf<int16_t> scol16;
+    // sliced ELL copy of the solver matrix, used by spmv when there is a plan
+    SellPlan sell;
     DevBuf<double> sval64;
     DevBuf<float> sval32;
     Scal* h_scal = nullptr;  // host copy of the current slot (pinned when h_scal_owned)
@@ -905,23 +901,22 @@ static int lanes_for(const flgpu_ctx* c) {
 }
 
 static int spmv_grid(const flgpu_ctx* c) {
-    return c->kw->use_sell ? sell_grid(c->kw->nsl) : stream_grid(c->kw->nrb);
+    return c->kw->sell.nsl ? sell_grid(c->kw->sell.nsl) : stream_grid(c->kw->nrb);
 }
 
 // The sliced ELL values matching a CSR value array of the solver matrix
 // (null for any other array, which takes the CSR product).
 static const double* sell_values(const KrylovWork* k, const double* val) {
-    return k->use_sell && val == k->val64.p ? k->sval64.p : nullptr;
+    return k->sell.nsl && val == k->val64.p ? k->sval64.p : nullptr;
 }
 static const float* sell_values(const KrylovWork* k, const float* val) {
-    return k->use_sell && val == k->val32.p ? k->sval32.p : nullptr;
+    return k->sell.nsl && val == k->val32.p ? k->sval32.p : nullptr;
 }
 
 template <typename V, typename CT, typename XV, typename YV>
 static void sell_launch(flgpu_ctx* c, KrylovWork* k, const V* sval, const CT* col, const XV* x, YV* y,
                         const double* bsub, int want_dot, const int* done_flag) {
-    const SellOp<V, CT> m{k->nsl, c->rows, k->sptr.p, col, sval, nullptr, k->srows.p, k->soff.p,
-                                                    k->smask.p};
+    const SellOp<V, CT> m = sell_op(k->sell, c->rows, sval, col);
     if (want_dot)
         sell_product<V, V, CT, XV, YV, DOT_XY>(c->stream, m, x, y, bsub, nullptr, nullptr, k->part(PART_SPMV), done_flag);
     else
@@ -954,10 +949,10 @@ template <typename V, typename XV, typename YV>
 static int spmv(flgpu_ctx* c, KrylovWork* k, const V* val, const XV* x, YV* y, const double* bsub,
                 int want_dot, const int* done_flag) {
     if (const V* sv = sell_values(k, val)) {
-        if (k->sell16)
-            sell_launch<V, int16_t, XV, YV>(c, k, sv, k->scol16.p, x, y, bsub, want_dot, done_flag);
+        if (k->sell.use16)
+            sell_launch<V, int16_t, XV, YV>(c, k, sv, k->sell.col16.p, x, y, bsub, want_dot, done_flag);
         else
-            sell_launch<V, int32_t, XV, YV>(c, k, sv, k->scol32.p, x, y, bsub, want_dot, done_flag);
+            sell_launch<V, int32_t, XV, YV>(c, k, sv, k->sell.col32.p, x, y, bsub, want_dot, done_flag);
     } else if (k->use16)
         spmv_launch<V, int16_t, XV, YV>(c, k, val, k->col16.p, x, y, bsub, want_dot, done_flag);
     else
@@ -970,36 +965,13 @@ static int spmv(flgpu_ctx* c, KrylovWork* k, const V* val, const XV* x, YV* y, c
 // (FLGPU_SPMV=csr keeps the CSR products throughout).
 static int sell_setup(flgpu_ctx* c, KrylovWork* k) {
     const char* e = getenv("FLGPU_SPMV");
-    k->use_sell = false;
-    k->sptr.release();
-    k->ssrc.release();
-    k->srows.release();
-    k->soff.release();
-    k->smask.release();
-    k->scol16.release();
-    k->scol32.release();
+    k->sell.release();
     k->sval64.release();
     k->sval32.release();
     if (e && std::string(e) == "csr") return FLGPU_OK;
-    const int32_t* rp = c->h_rowptr.data();
-    const SellOrder order = sell_order(rp, c->rows);
+    const SellOrder order = sell_order(c->h_rowptr.data(), c->rows);
     if (order == SELL_NONE) return FLGPU_OK;
-    const int window = order == SELL_SORTED ? kSellWindow : 0;
-    SellHost h;
-    sell_plan(rp, c->h_col.data(), c->rows, nullptr, h, window, true, sell_run(c->rows));
-    if (window) FLGPU_TRY(k->srows.upload(h.rows.data(), h.rows.size(), c->stream));
-    FLGPU_TRY(k->soff.upload(h.off.data(), h.off.size(), c->stream));
-    FLGPU_TRY(k->smask.upload(h.mask.data(), h.mask.size(), c->stream));
-    FLGPU_TRY(k->sptr.upload(h.sptr.data(), h.sptr.size(), c->stream));
-    FLGPU_TRY(k->ssrc.upload(h.src.data(), h.src.size(), c->stream));
-    if (h.use16) FLGPU_TRY(k->scol16.upload(h.c16.data(), h.c16.size(), c->stream));
-    else FLGPU_TRY(k->scol32.upload(h.c32.data(), h.c32.size(), c->stream));
-    FLGPU_HIP(hipStreamSynchronize(c->stream));  // h is freed on return
-    k->nsl = h.nsl;
-    k->nslot = h.nslot;
-    k->sell16 = h.use16;
-    k->use_sell = true;
-    return FLGPU_OK;
+    return sell_build(c->stream, c->rows, c->nnz, c->rowptr.p, c->col.p, nullptr, order == SELL_SORTED, k->sell);
 }
 
 static int ensure_work(flgpu_ctx* c, bool mixed) {
@@ -1046,9 +1018,9 @@ static int ensure_work(flgpu_ctx* c, bool mixed) {
         FLGPU_TRY(sell_setup(c, k));
         k->rb_key = c->sparsity_gen;
     }
-    if (k->use_sell) {
-        FLGPU_TRY(k->sval64.alloc((size_t)k->nslot));
-        if (mixed) FLGPU_TRY(k->sval32.alloc((size_t)k->nslot));
+    if (k->sell.nsl) {
+        FLGPU_TRY(k->sval64.alloc((size_t)k->sell.nslot));
+        if (mixed) FLGPU_TRY(k->sval32.alloc((size_t)k->sell.nslot));
     }
     FLGPU_TRY(k->scal.alloc(2));
     if (!k->h_scal) {
@@ -1090,13 +1062,14 @@ static int build_reduced(flgpu_ctx* c, KrylovWork* k, bool mixed, bool zero_x) {
                        c->rowptr.p, c->col.p, c->A.p, c->rhs.p, c->inactive.p, c->have_inactive ? 1 : 0, k->S(),
                        k->val64.p, mixed ? k->val32.p : nullptr, k->b.p, k->dinv.p, mixed ? k->dinv32.p : nullptr,
                        k->x.p, zero_x ? 1 : 0);
-    if (k->use_sell) {
-        const unsigned g = grid_for(k->nslot, 256);
-        hipLaunchKernelGGL((k_sell_gather<double, double>), dim3(g), dim3(256), 0, c->stream, k->nslot, k->ssrc.p,
+    if (k->sell.nsl) {
+        const SellPlan& p = k->sell;
+        const unsigned g = grid_for(p.nslot, 256);
+        hipLaunchKernelGGL((k_sell_gather<double, double>), dim3(g), dim3(256), 0, c->stream, p.nslot, p.src.p,
                            k->val64.p, k->sval64.p);
         if (mixed)
-            hipLaunchKernelGGL((k_sell_gather<float, float>), dim3(g), dim3(256), 0, c->stream, k->nslot,
-                               k->ssrc.p, k->val32.p, k->sval32.p);
+            hipLaunchKernelGGL((k_sell_gather<float, float>), dim3(g), dim3(256), 0, c->stream, p.nslot, p.src.p,
+                               k->val32.p, k->sval32.p);
     }
     FLGPU_HIP(hipGetLastError());
     return FLGPU_OK;
@@ -2506,7 +2479,7 @@ k_gm_small(SellOp<V, CT> m, size_t ldv, V* __restrict__ Vb, const double* __rest
 // 20 us of the four launches (P1 triangles: up to 2200 rows).
 static bool gm_small_fits(const KrylovWork* k, int n, int64_t nnz, int m, size_t value) {
     const double bytes = (double)nnz * (double)(value + 2) + 30.0 * (double)n * (double)value;
-    return k->use_sell && m <= kGmReg && 2 * value * ((size_t)n + 2) <= ((size_t)96 << 10) && 6.0 + bytes / 55e3 < 18.0;
+    return k->sell.nsl && m <= kGmReg && 2 * value * ((size_t)n + 2) <= ((size_t)96 << 10) && 6.0 + bytes / 55e3 < 18.0;
 }
 
 // Waits until the device has closed `its` columns or the solve is done; a
@@ -2591,15 +2564,13 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
         const V* dv = ssor ? nullptr : dinv;
         V* y = ssor ? tmp : out;
         if (sval) {
-            const int grid = sell_grid(k->nsl);
-            if (k->sell16) {
-                const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, k->scol16.p, sval, nullptr, k->srows.p, k->soff.p,
-                                                    k->smask.p};
+            const int grid = sell_grid(k->sell.nsl);
+            if (k->sell.use16) {
+                const SellOp<V, int16_t> op = sell_op(k->sell, n, sval, k->sell.col16.p);
                 hipLaunchKernelGGL((k_gm_sell<V, int16_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
                                    d);
             } else {
-                const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, k->scol32.p, sval, nullptr, k->srows.p, k->soff.p,
-                                                    k->smask.p};
+                const SellOp<V, int32_t> op = sell_op(k->sell, n, sval, k->sell.col32.p);
                 hipLaunchKernelGGL((k_gm_sell<V, int32_t>), dim3(grid), dim3(kRowBlock), 0, c->stream, op, w, v, y, dv,
                                    d);
             }
@@ -2663,13 +2634,11 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
             return FLGPU_OK;
         };
         const bool one = n <= kGmSmallBlock;
-        if (k->sell16) {
-            const SellOp<V, int16_t> op{k->nsl, n, k->sptr.p, k->scol16.p, sval, nullptr, k->srows.p, k->soff.p,
-                                                    k->smask.p};
+        if (k->sell.use16) {
+            const SellOp<V, int16_t> op = sell_op(k->sell, n, sval, k->sell.col16.p);
             return one ? launch(&k_gm_small<V, int16_t, true>, op) : launch(&k_gm_small<V, int16_t, false>, op);
         }
-        const SellOp<V, int32_t> op{k->nsl, n, k->sptr.p, k->scol32.p, sval, nullptr, k->srows.p, k->soff.p,
-                                                    k->smask.p};
+        const SellOp<V, int32_t> op = sell_op(k->sell, n, sval, k->sell.col32.p);
         return one ? launch(&k_gm_small<V, int32_t, true>, op) : launch(&k_gm_small<V, int32_t, false>, op);
     };
     for (;;) {

@@ -29,6 +29,7 @@
 #include "flgpu_internal.h"
 #include "krylov_common.h"
 #include "learned.h"
+#include "sell_plan.h"
 
 namespace flgpu {
 
@@ -93,13 +94,9 @@ struct LearnedState {
     int nrbl = 0, nrbu = 0;
     int64_t nnzl = 0, nnzu = 0;
     // the halves as sliced ELL operands (when both pad little): the value
-    // arrays gl/gu then hold slots, gathered from the factor through lss/uss
-    bool sell = false, ls16 = false, us16 = false;
-    int nsll = 0, nslu = 0;
-    int64_t nslotl = 0, nslotu = 0;
-    DevBuf<int32_t> lsp, usp, lss, uss, lsc32, usc32, lso, uso;
-    DevBuf<int16_t> lsc16, usc16;
-    DevBuf<uint64_t> lsm, usm;  // diagonal slices: lso/uso offsets, lsm/usm masks
+    // arrays gl/gu then hold slots, gathered from the factor through src
+    bool sell = false;
+    SellPlan lsell, usell;
     // factor of the scaled matrix, Gs: FP16 for the mixed solve, FP64 for
     // the FP64 solve; the scaling D is applied by the products
     DevBuf<_Float16> gl16, gu16;
@@ -1214,30 +1211,14 @@ static int lu_prepare(flgpu_ctx* c, LearnedState* s) {
     if (s->u16) FLGPU_TRY(s->ucol16.upload(u16.data(), u16.size(), c->stream));
     // sliced ELL plans of both halves when both fit in order, the slots mapped
     // to the factor's entries
-    SellHost hl, hu;
     const char* e = getenv("FLGPU_SPMV");
     s->sell = !(e && std::string(e) == "csr") && sell_fits(lp.data(), n) && sell_fits(up.data(), n);
+    s->lsell.release();
+    s->usell.release();
     if (s->sell) {
-        sell_plan(lp.data(), lc.data(), n, ls.data(), hl, 0, true);
-        sell_plan(up.data(), uc.data(), n, us.data(), hu, 0, true);
-        FLGPU_TRY(s->lsp.upload(hl.sptr.data(), hl.sptr.size(), c->stream));
-        FLGPU_TRY(s->usp.upload(hu.sptr.data(), hu.sptr.size(), c->stream));
-        FLGPU_TRY(s->lso.upload(hl.off.data(), hl.off.size(), c->stream));
-        FLGPU_TRY(s->uso.upload(hu.off.data(), hu.off.size(), c->stream));
-        FLGPU_TRY(s->lsm.upload(hl.mask.data(), hl.mask.size(), c->stream));
-        FLGPU_TRY(s->usm.upload(hu.mask.data(), hu.mask.size(), c->stream));
-        FLGPU_TRY(s->lss.upload(hl.src.data(), hl.src.size(), c->stream));
-        FLGPU_TRY(s->uss.upload(hu.src.data(), hu.src.size(), c->stream));
-        if (hl.use16) FLGPU_TRY(s->lsc16.upload(hl.c16.data(), hl.c16.size(), c->stream));
-        else FLGPU_TRY(s->lsc32.upload(hl.c32.data(), hl.c32.size(), c->stream));
-        if (hu.use16) FLGPU_TRY(s->usc16.upload(hu.c16.data(), hu.c16.size(), c->stream));
-        else FLGPU_TRY(s->usc32.upload(hu.c32.data(), hu.c32.size(), c->stream));
-        s->ls16 = hl.use16;
-        s->us16 = hu.use16;
-        s->nsll = hl.nsl;
-        s->nslu = hu.nsl;
-        s->nslotl = hl.nslot;
-        s->nslotu = hu.nslot;
+        FLGPU_TRY(sell_build(c->stream, n, (int64_t)lc.size(), s->lptr.p, s->lcol.p, s->lsrc.p, false, s->lsell));
+        FLGPU_TRY(sell_build(c->stream, n, (int64_t)uc.size(), s->uptr.p, s->ucol.p, s->usrc.p, false, s->usell));
+        s->sell = s->lsell.nsl && s->usell.nsl;
     }
     FLGPU_HIP(hipStreamSynchronize(c->stream));
     s->nnzl = (int64_t)lc.size();
@@ -1252,12 +1233,13 @@ template <typename GV, typename HV>
 static int split_halves(flgpu_ctx* c, LearnedState* s, const GV* gv, DevBuf<HV>& gl, DevBuf<HV>& gu) {
     FLGPU_TRY(lu_prepare(c, s));
     if (s->sell) {
-        FLGPU_TRY(gl.alloc(s->nslotl));
-        FLGPU_TRY(gu.alloc(s->nslotu));
-        hipLaunchKernelGGL((k_sell_gather<GV, HV>), dim3(grid_for(s->nslotl, 256)), dim3(256), 0, c->stream,
-                           s->nslotl, s->lss.p, gv, gl.p);
-        hipLaunchKernelGGL((k_sell_gather<GV, HV>), dim3(grid_for(s->nslotu, 256)), dim3(256), 0, c->stream,
-                           s->nslotu, s->uss.p, gv, gu.p);
+        const SellPlan &l = s->lsell, &u = s->usell;
+        FLGPU_TRY(gl.alloc(l.nslot));
+        FLGPU_TRY(gu.alloc(u.nslot));
+        hipLaunchKernelGGL((k_sell_gather<GV, HV>), dim3(grid_for(l.nslot, 256)), dim3(256), 0, c->stream, l.nslot,
+                           l.src.p, gv, gl.p);
+        hipLaunchKernelGGL((k_sell_gather<GV, HV>), dim3(grid_for(u.nslot, 256)), dim3(256), 0, c->stream, u.nslot,
+                           u.src.p, gv, gu.p);
         FLGPU_HIP(hipGetLastError());
         return FLGPU_OK;
     }
@@ -1298,8 +1280,8 @@ static void apply_launch_sell(flgpu_ctx* c, LearnedState* s, const HV* gl, const
                               const UC* ucol, const V* r, const V* rt, V* z, V* y, const V* w, double* partials,
                               const int* done) {
     const int n = c->rows;
-    const SellOp<HV, LC> lo{s->nsll, n, s->lsp.p, lcol, gl, nullptr, nullptr, s->lso.p, s->lsm.p};
-    const SellOp<HV, UC> up{s->nslu, n, s->usp.p, ucol, gu, s->dsq.p, nullptr, s->uso.p, s->usm.p};
+    const SellOp<HV, LC> lo = sell_op(s->lsell, n, gl, lcol);
+    const SellOp<HV, UC> up = sell_op(s->usell, n, gu, ucol, s->dsq.p);
     sell_product<V, HV, LC, V, V, DOT_NONE>(c->stream, lo, rt, y, nullptr, nullptr, nullptr, partials, done);
     sell_product<V, HV, UC, V, V, DOT_PC>(c->stream, up, y, z, nullptr, r, w, partials, done);
 }
@@ -1308,19 +1290,16 @@ template <typename V, typename HV>
 static int apply_impl(flgpu_ctx* c, LearnedState* s, const HV* gl, const HV* gu, const V* r, const V* rt, V* z,
                       V* y, const V* w, double* partials, int* nparts, const int* done) {
     if (s->sell) {
-        *nparts = sell_grid(s->nslu);
-        if (s->ls16 && s->us16)
-            apply_launch_sell<V, HV, int16_t, int16_t>(c, s, gl, gu, s->lsc16.p, s->usc16.p, r, rt, z, y, w,
-                                                       partials, done);
-        else if (s->ls16)
-            apply_launch_sell<V, HV, int16_t, int32_t>(c, s, gl, gu, s->lsc16.p, s->usc32.p, r, rt, z, y, w,
-                                                       partials, done);
-        else if (s->us16)
-            apply_launch_sell<V, HV, int32_t, int16_t>(c, s, gl, gu, s->lsc32.p, s->usc16.p, r, rt, z, y, w,
-                                                       partials, done);
+        const SellPlan &l = s->lsell, &u = s->usell;
+        *nparts = sell_grid(u.nsl);
+        if (l.use16 && u.use16)
+            apply_launch_sell<V, HV>(c, s, gl, gu, l.col16.p, u.col16.p, r, rt, z, y, w, partials, done);
+        else if (l.use16)
+            apply_launch_sell<V, HV>(c, s, gl, gu, l.col16.p, u.col32.p, r, rt, z, y, w, partials, done);
+        else if (u.use16)
+            apply_launch_sell<V, HV>(c, s, gl, gu, l.col32.p, u.col16.p, r, rt, z, y, w, partials, done);
         else
-            apply_launch_sell<V, HV, int32_t, int32_t>(c, s, gl, gu, s->lsc32.p, s->usc32.p, r, rt, z, y, w,
-                                                       partials, done);
+            apply_launch_sell<V, HV>(c, s, gl, gu, l.col32.p, u.col32.p, r, rt, z, y, w, partials, done);
         FLGPU_HIP(hipGetLastError());
         return FLGPU_OK;
     }

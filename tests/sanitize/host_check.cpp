@@ -31,6 +31,7 @@
 #include "../../fluidity_amd/csrc/krylov_common.h"
 #include "../../include/flgpu.h"
 #include "../../oracle/fl_oracle.h"
+#include "sell_reference.h"
 
 static int failures = 0;
 #define CHECK(cond, ...)                                  \
