@@ -2356,9 +2356,9 @@ __device__ __forceinline__ double gm_small_orth(int n, size_t ldv, int nv, const
     return total;
 }
 
-template <typename V, typename CT, bool ONE>
+template <typename V, bool ONE>
 __global__ void __launch_bounds__(kGmSmallBlock)
-k_gm_small(SellOp<V, CT> m, size_t ldv, V* __restrict__ Vb, const double* __restrict__ r64,
+k_gm_small(SellOp<V, int16_t> m, size_t ldv, V* __restrict__ Vb, const double* __restrict__ r64,
            const double* __restrict__ dinv64, const V* __restrict__ dinv, double* __restrict__ x, GmDev d) {
     constexpr int B = kGmSmallBlock, N = kGmReg;
     extern __shared__ double gm_lds[];
@@ -2476,10 +2476,11 @@ k_gm_small(SellOp<V, CT> m, size_t ldv, V* __restrict__ Vb, const double* __rest
 // A cycle goes to one workgroup when its vectors fit LDS, the basis its
 // registers, and an iteration -- 6 us of block sums, then the matrix and
 // three passes over ten vectors read by one CU at 55 GB/s -- stays below the
-// 20 us of the four launches (P1 triangles: up to 2200 rows).
+// 20 us of the four launches (P1 triangles: up to 2200 rows).  Column indices
+// of so few rows have 16 bits.
 static bool gm_small_fits(const KrylovWork* k, int n, int64_t nnz, int m, size_t value) {
     const double bytes = (double)nnz * (double)(value + 2) + 30.0 * (double)n * (double)value;
-    return k->sell.nsl && m <= kGmReg && 2 * value * ((size_t)n + 2) <= ((size_t)96 << 10) && 6.0 + bytes / 55e3 < 18.0;
+    return k->sell.nsl && k->sell.use16 && m <= kGmReg && 2 * value * ((size_t)n + 2) <= ((size_t)96 << 10) && 6.0 + bytes / 55e3 < 18.0;
 }
 
 // Waits until the device has closed `its` columns or the solve is done; a
@@ -2625,7 +2626,8 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
     const bool small = !ssor && sval && gm_small_fits(k, n, c->nnz, m, sizeof(V));
     auto small_cycle = [&]() -> int {
         const size_t lds = 2 * sizeof(V) * (((size_t)n + 1) & ~(size_t)1);
-        auto launch = [&](auto kern, auto op) -> int {
+        const SellOp<V, int16_t> op = sell_op(k->sell, n, sval, (const int16_t*)k->sell.col16.p);
+        auto launch = [&](auto kern) -> int {
             FLGPU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, 100 << 10));
             hipLaunchKernelGGL(kern, dim3(1), dim3(kGmSmallBlock), lds, c->stream, op, ldv, Vb, (const double*)k->r.p,
@@ -2633,13 +2635,7 @@ static int run_gmres(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_in
             FLGPU_HIP(hipGetLastError());
             return FLGPU_OK;
         };
-        const bool one = n <= kGmSmallBlock;
-        if (k->sell.use16) {
-            const SellOp<V, int16_t> op = sell_op(k->sell, n, sval, k->sell.col16.p);
-            return one ? launch(&k_gm_small<V, int16_t, true>, op) : launch(&k_gm_small<V, int16_t, false>, op);
-        }
-        const SellOp<V, int32_t> op = sell_op(k->sell, n, sval, k->sell.col32.p);
-        return one ? launch(&k_gm_small<V, int32_t, true>, op) : launch(&k_gm_small<V, int32_t, false>, op);
+        return n <= kGmSmallBlock ? launch(&k_gm_small<V, true>) : launch(&k_gm_small<V, false>);
     };
     for (;;) {
         // residual in FP64, preconditioned, in the working precision
