@@ -1743,8 +1743,10 @@ static int run_cg1(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_info
 // The iteration counter and the done flag reach the host through a word in
 // pinned memory, which it polls a few iterations behind what it has queued.
 // What bounds it: small systems, the chain of four launches (each two or
-// three dependent memory round trips, 4-6 us); large ones, reading the basis
-// (6 TB/s with 32 vectors of 373k rows: 15-17 us a pass).  Whole time steps
+// three dependent memory round trips, 4-7 us); large ones, reading the basis
+// (17 to 30 vectors of 373k rows: 15-17 us a pass, 4.2 to 4.7 TB/s).  A column
+// is closed beside the next iteration's dot products, so a solve runs one
+// product (and one pair of sweeps) past the last column.  Whole time steps
 // on one MI355X, against ten launches and three waits for the host an
 // iteration: 64 x 64 P1 triangles, 18 iterations, 2.04 -> 0.65 ms; 71^3 x 6
 // P1 tetrahedra, 30 iterations, 5.80 -> 2.87 ms; 40^3 x 6 P2, 14.4 -> 9.7 ms.
