@@ -1746,10 +1746,11 @@ static int run_cg1(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_info
 // three dependent memory round trips, 4-7 us); large ones, reading the basis
 // (17 to 30 vectors of 373k rows: 15-17 us a pass, 4.2 to 4.7 TB/s).  A column
 // is closed beside the next iteration's dot products, so a solve runs one
-// product (and one pair of sweeps) past the last column.  Whole time steps
-// on one MI355X, against ten launches and three waits for the host an
-// iteration: 64 x 64 P1 triangles, 18 iterations, 2.04 -> 0.65 ms; 71^3 x 6
-// P1 tetrahedra, 30 iterations, 5.80 -> 2.87 ms; 40^3 x 6 P2, 14.4 -> 9.7 ms.
+// product (and one pair of sweeps) past the last column.  Whole time steps on
+// one MI355X, with ten launches and three waits for the host an iteration and
+// now (the sliced products' share included): 64 x 64 P1 triangles, 17
+// iterations, 2.08 -> 0.62 ms; 71^3 x 6 P1 tetrahedra, 29 iterations, 5.87 ->
+// 2.77 ms; 40^3 x 6 P2, 52 iterations, 14.4 -> 7.4 ms.
 
 constexpr int kGmGrid = 256;    // blocks of the basis kernels: one per CU, so that a consumer block can sum the
                                 // partial sums of every basis vector itself (256 x 31 doubles)
@@ -2304,7 +2305,7 @@ k_gm_precres(int n, const double* __restrict__ r64, const double* __restrict__ d
 // (the product gathers there); a thread keeps the same rows of every basis
 // vector, which stay in this CU's caches, and with at most one row a thread
 // it reads them once an iteration.  Bound by the latency of the block sums
-// (6 us an iteration) and by what one CU reads (gm_small_fits): 324 rows 7.8
+// (6 us an iteration) and by what one CU reads (gm_small_fits): 324 rows 7.3
 // us an iteration, 4225 rows 32 us, where the four launches take 21 us.
 // Time step on 17 x 17 P1 triangles: 0.56 -> 0.32 ms.
 constexpr int kGmSmallBlock = 512;
