@@ -107,3 +107,24 @@ def test_quadratic_products_numbered_at_random(require_gpu, scale):
         # mass-dominated: condition numbers below 1e3
         assert info.reason > 0 and np.linalg.norm(x - xr) <= 1e3 * 1e-10 * np.linalg.norm(xr), precision
     pr.close()
+
+
+@pytest.mark.parametrize("ksp,pc", [("cg", "jacobi"), ("cg", "sor"), ("fcg", "fsai"), ("pipecg", "jacobi"),
+                                    ("pipecg", "fsai")])
+def test_batches_of_iterations_change_nothing(require_gpu, ksp, pc):
+    """The iterations that are queued between two looks at the scalars, few or
+    more than the solve takes, and ended by convergence or by the limit."""
+    cfg = M.config("c2", seed=41, scale=12)
+    pr = cg.problem_from_config(cfg)
+    cg.assemble_advection_diffusion_cg(pr, cg.options_from_config(cfg), cfg.dt)
+    cg.apply_dirichlet_conditions(pr, cfg.mesh.boundary, 0.0, cfg.dt)
+    for limit in (1, 2, 5, 16, 17, 10000):
+        seen = []
+        for every in (1, 2, 5, 16, 300):
+            print(f"\n[case] {ksp} {pc} limit {limit} batches of {every}", flush=True)
+            so = cg.SolverOptions(ksp, pc, relative_error=1e-9, max_iterations=limit, check_every=every)
+            x, info = cg.petsc_solve(pr, so)
+            assert info.reason == (2 if limit == 10000 else -3) and (limit == 10000 or info.its == limit)
+            seen.append((info.its, x))
+        assert all(its == seen[0][0] and np.array_equal(x, seen[0][1]) for its, x in seen)
+    pr.close()
