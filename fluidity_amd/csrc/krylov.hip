@@ -59,8 +59,9 @@ struct KrylovWork {
     DevBuf<float> sval32;
     Scal* h_scal = nullptr;  // host copy of the current slot (pinned when h_scal_owned)
     bool h_scal_owned = false;
-    int64_t* word = nullptr;   // the CG loops' progress, 2 its + done, behind h_scal when that is pinned:
-    int64_t* d_word = nullptr; // written by the device (null: not published)
+    int64_t* word = nullptr;   // the CG loops' progress, 2 its + done, behind h_scal when that is pinned,
+    int64_t* d_word = nullptr; // its address for the device,
+    int64_t* pub = nullptr;    // and what a batch's iterations write to (null: not published)
     int nblk = 1;
     Scal* S() { return scal.p + cur; }
     double* part(int region) { return partials.p + (size_t)region * kPartStride; }
@@ -1420,10 +1421,10 @@ static int cg_iteration(flgpu_ctx* c, KrylovWork* k, const CgVecs<V>& v, PcMode 
     k->cur ^= 1;
     if (rows_aligned<R>(v.z, v.p))
         hipLaunchKernelGGL((k_cg_p<V, R>), dim3(k->nblk), dim3(kVecBlock), 0, c->stream, c->rows, v.z, v.p,
-                           k->part(PART_VEC), k->nblk, diag ? nullptr : k->part(PART_PC), npc, in, k->S(), k->d_word);
+                           k->part(PART_VEC), k->nblk, diag ? nullptr : k->part(PART_PC), npc, in, k->S(), k->pub);
     else
         hipLaunchKernelGGL((k_cg_p<V, 1>), dim3(k->nblk), dim3(kVecBlock), 0, c->stream, c->rows, v.z, v.p,
-                           k->part(PART_VEC), k->nblk, diag ? nullptr : k->part(PART_PC), npc, in, k->S(), k->d_word);
+                           k->part(PART_VEC), k->nblk, diag ? nullptr : k->part(PART_PC), npc, in, k->S(), k->pub);
     FLGPU_HIP(hipGetLastError());
     return FLGPU_OK;
 }
@@ -1455,17 +1456,20 @@ static int wait_word(flgpu_ctx* c, const int64_t* word, int64_t its) {
 // ahead of the device and queues none once that is done.  Before iteration q
 // of a batch that began at iteration `its`: true if it is still wanted.  (The
 // single-reduction CG counts an iteration when the next one begins.)  Solves
-// of 17 iterations, 1681 rows: Jacobi 574 -> 395 us, sor 1039 -> 714 us; of 64,
-// which leave nothing over: as before.
-constexpr int kCgAhead = 4;
+// of 17 iterations, 1681 rows: Jacobi 574 -> 395 us, sor 1039 -> 714 us.  Past
+// kCgPublish iterations what is left over is small beside the solve, and only
+// the sor sweeps' iterations, of many launches, are still published (0.3 us
+// each: 0.5% of a solve of 538 on 1.37M rows).
+constexpr int kCgAhead = 4, kCgPublish = 64;
 
-static int cg_ahead(flgpu_ctx* c, KrylovWork* k, int64_t its, int q, bool* wanted) {
+static int cg_ahead(flgpu_ctx* c, KrylovWork* k, PcMode mode, int64_t its, int q, bool* wanted) {
     *wanted = true;
-    if (!k->d_word) return FLGPU_OK;
     if (q == 0) {  // nothing is in flight
-        __atomic_store_n(k->word, 2 * its, __ATOMIC_RELEASE);
+        k->pub = its < kCgPublish || mode == PCM_SSOR ? k->d_word : nullptr;
+        if (k->pub) __atomic_store_n(k->word, 2 * its, __ATOMIC_RELEASE);
         return FLGPU_OK;
     }
+    if (!k->pub) return FLGPU_OK;
     FLGPU_TRY(wait_word(c, k->word, its + q - kCgAhead));
     *wanted = !(__atomic_load_n(k->word, __ATOMIC_ACQUIRE) & 1);
     return FLGPU_OK;
@@ -1530,7 +1534,7 @@ static int run_cg(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_info*
     while (!h.done) {
         for (int q = 0; q < check_every; q++) {
             bool wanted;
-            FLGPU_TRY(cg_ahead(c, k, h.its, q, &wanted));
+            FLGPU_TRY(cg_ahead(c, k, mode, h.its, q, &wanted));
             if (!wanted) break;
             FLGPU_TRY(cg_iteration<V>(c, k, v, mode));
         }
@@ -1637,7 +1641,7 @@ static int cg1_iteration(flgpu_ctx* c, KrylovWork* k, const CgVecs<V>& v, PcMode
         hipLaunchKernelGGL(kern, dim3(k->nblk), dim3(kVecBlock), 0, c->stream, c->rows, k->x.p, v.p, v.s, v.r, v.z,
                            (const V*)v.w, (const V*)v.dinv, diag ? 1 : 0, dsc, v.rt, (const double*)k->part(PART_SPMV),
                            spmv_grid(c), pg, ng, diag ? 0 : 1, (const double*)k->part(reg), k->nblk, first ? 1 : 0,
-                           k->part(reg_out), (const Scal*)in, k->S(), k->d_word);
+                           k->part(reg_out), (const Scal*)in, k->S(), k->pub);
     };
     if (rows_aligned<R>(k->x.p, v.p, v.s, v.r, v.z, v.w, v.dinv, dsc, v.rt))
         launch(&k_cg1_vec<V, R>);
@@ -1713,7 +1717,7 @@ static int run_cg1(flgpu_ctx* c, const flgpu_solver_params* sp, flgpu_solve_info
     while (!h.done) {
         for (int q = 0; q < check_every; q++) {
             bool wanted;
-            FLGPU_TRY(cg_ahead(c, k, h.its, q, &wanted));
+            FLGPU_TRY(cg_ahead(c, k, mode, h.its, q, &wanted));
             if (!wanted) break;
             FLGPU_TRY(cg1_iteration<V>(c, k, v, mode, first, reg));
             first = false;
